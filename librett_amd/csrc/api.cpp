@@ -492,15 +492,16 @@ int librett_c_host_replay(int rank, const int* dim, const int* permutation, size
     std::vector<Candidate> cands = make_candidates(full, dev);
     if (index < 0 || index >= (int)cands.size()) return LIBRETT_INVALID_PARAMETER;
     // Guard bands around both buffers: a stray store shows up as a changed
-    // output guard, a stray load as guard bytes in the output.
+    // output guard, a stray load as guard bytes in the output. As in
+    // run_plan, pointers off the candidate's alignment take its fallback.
+    const Candidate& c = cands[index];
     const size_t n = (size_t)full.vol * sizeofType;
-    const size_t g = 1 << 16;
-    std::vector<unsigned char> in(n + 2 * g, 0xA5), out(n + 2 * g, 0x5A);
-    std::memcpy(in.data() + g, idata, n);
-    if (!replay_candidate(cands[index], in.data() + g, out.data() + g)) return LIBRETT_INTERNAL_ERROR;
-    for (size_t i = 0; i < g; i++)
-      if (out[i] != 0x5A || out[g + n + i] != 0x5A) return LIBRETT_UNDEFINED_ERROR;
-    std::memcpy(odata, out.data() + g, n);
+    GuardedBuffer in(n, idata, (int)sizeofType, 0xA5), out(n, odata, (int)sizeofType, 0x5A);
+    std::memcpy(in.data(), idata, n);
+    const uintptr_t mis = ((uintptr_t)in.data() | (uintptr_t)out.data()) & (uintptr_t)(needed_alignment(c) - 1);
+    if (!replay_candidate(mis ? unaligned_fallback(c) : c, in.data(), out.data())) return LIBRETT_INTERNAL_ERROR;
+    if (!out.intact()) return LIBRETT_UNDEFINED_ERROR;
+    std::memcpy(odata, out.data(), n);
     return LIBRETT_SUCCESS;
   } catch (...) {
     return LIBRETT_INTERNAL_ERROR;

@@ -18,7 +18,7 @@ namespace {
 //   Tiled:     tile_x, tile_y, vec_x, vec_y; group flag 1 for planes over
 //              dim groups (their own family, so the one-dim kernels keep
 //              their registers)
-//   TiledCopy: word, copy_tx
+//   TiledCopy: none
 //   Packed:    nreg
 #define LRT_BATCH_TABLE(X)                                                  \
   X(0, kTiled, 4, 64, 64, 1, 1, 0) X(1, kTiled, 4, 64, 64, 4, 1, 0)         \
@@ -26,21 +26,19 @@ namespace {
   X(4, kTiled, 8, 32, 32, 1, 1, 0) X(5, kTiled, 8, 32, 32, 2, 1, 0)         \
   X(6, kTiled, 8, 32, 32, 1, 2, 0) X(7, kTiled, 8, 32, 32, 2, 2, 0)         \
   X(8, kTiled, 16, 32, 32, 1, 1, 0)                                         \
-  X(9, kTiledCopy, 4, 4, 16, 0, 0, 0) X(10, kTiledCopy, 4, 4, 64, 0, 0, 0)  \
-  X(11, kTiledCopy, 8, 8, 16, 0, 0, 0) X(12, kTiledCopy, 8, 8, 64, 0, 0, 0) \
-  X(13, kTiledCopy, 16, 16, 16, 0, 0, 0)                                    \
-  X(14, kTiledCopy, 16, 16, 64, 0, 0, 0)                                    \
-  X(15, kPacked, 4, 1, 0, 0, 0, 0) X(16, kPacked, 4, 2, 0, 0, 0, 0)         \
-  X(17, kPacked, 4, 4, 0, 0, 0, 0) X(18, kPacked, 4, 8, 0, 0, 0, 0)         \
-  X(19, kPacked, 8, 1, 0, 0, 0, 0) X(20, kPacked, 8, 2, 0, 0, 0, 0)         \
-  X(21, kPacked, 8, 4, 0, 0, 0, 0) X(22, kPacked, 8, 8, 0, 0, 0, 0)         \
-  X(23, kPacked, 16, 1, 0, 0, 0, 0) X(24, kPacked, 16, 2, 0, 0, 0, 0)       \
-  X(25, kPacked, 16, 4, 0, 0, 0, 0)                                         \
-  X(26, kTiled, 4, 64, 64, 1, 1, 1) X(27, kTiled, 4, 64, 64, 4, 1, 1)       \
-  X(28, kTiled, 4, 64, 64, 1, 4, 1) X(29, kTiled, 4, 64, 64, 4, 4, 1)       \
-  X(30, kTiled, 8, 32, 32, 1, 1, 1) X(31, kTiled, 8, 32, 32, 2, 1, 1)       \
-  X(32, kTiled, 8, 32, 32, 1, 2, 1) X(33, kTiled, 8, 32, 32, 2, 2, 1)       \
-  X(34, kTiled, 16, 32, 32, 1, 1, 1)
+  X(9, kTiledCopy, 4, 0, 0, 0, 0, 0) X(10, kTiledCopy, 8, 0, 0, 0, 0, 0)    \
+  X(11, kTiledCopy, 16, 0, 0, 0, 0, 0)                                      \
+  X(12, kPacked, 4, 1, 0, 0, 0, 0) X(13, kPacked, 4, 2, 0, 0, 0, 0)         \
+  X(14, kPacked, 4, 4, 0, 0, 0, 0) X(15, kPacked, 4, 8, 0, 0, 0, 0)         \
+  X(16, kPacked, 8, 1, 0, 0, 0, 0) X(17, kPacked, 8, 2, 0, 0, 0, 0)         \
+  X(18, kPacked, 8, 4, 0, 0, 0, 0) X(19, kPacked, 8, 8, 0, 0, 0, 0)         \
+  X(20, kPacked, 16, 1, 0, 0, 0, 0) X(21, kPacked, 16, 2, 0, 0, 0, 0)       \
+  X(22, kPacked, 16, 4, 0, 0, 0, 0)                                         \
+  X(23, kTiled, 4, 64, 64, 1, 1, 1) X(24, kTiled, 4, 64, 64, 4, 1, 1)       \
+  X(25, kTiled, 4, 64, 64, 1, 4, 1) X(26, kTiled, 4, 64, 64, 4, 4, 1)       \
+  X(27, kTiled, 8, 32, 32, 1, 1, 1) X(28, kTiled, 8, 32, 32, 2, 1, 1)       \
+  X(29, kTiled, 8, 32, 32, 1, 2, 1) X(30, kTiled, 8, 32, 32, 2, 2, 1)       \
+  X(31, kTiled, 16, 32, 32, 1, 1, 1)
 
 struct BatchShape {
   int id, method, b, p1, p2, p3, p4, g;
@@ -96,14 +94,12 @@ __device__ __forceinline__ void dev_tiled(const BatchDesc& D, int lu, unsigned c
   }
 }
 
-template <int W, int TX>
+template <int B>
 __device__ __forceinline__ void dev_copy(const BatchDesc& D, int lu) {
-  using Ops = CopyOps<W, TX, 4>;
-  using V = typename Ops::V;
-  for (int w = lu; w < D.items; w += D.groups) {
-    const TileCtx c = Ops::item(D.a.copy, (uint32_t)w);
-    Ops::run(D.a.copy, c, threadIdx.x, static_cast<const V*>(D.in), static_cast<V*>(D.out));
-  }
+  using Ops = CopyOps<B>;
+  using E = typename Ops::E;
+  for (int w = lu; w < D.items; w += D.groups)
+    Ops::run(D.a.copy, (uint32_t)w, threadIdx.x, static_cast<const E*>(D.in), static_cast<E*>(D.out));
 }
 
 template <int B, int NREG>
@@ -146,40 +142,37 @@ __device__ __forceinline__ void dev_unit(const BatchDesc& D, int lu, unsigned ch
     }
   } else if constexpr (FAM == kFamTiledG) {
     switch (D.variant) {
-      case 26: dev_tiled<4, 64, 64, 1, 1, true>(D, lu, lds); break;
-      case 27: dev_tiled<4, 64, 64, 4, 1, true>(D, lu, lds); break;
-      case 28: dev_tiled<4, 64, 64, 1, 4, true>(D, lu, lds); break;
-      case 29: dev_tiled<4, 64, 64, 4, 4, true>(D, lu, lds); break;
-      case 30: dev_tiled<8, 32, 32, 1, 1, true>(D, lu, lds); break;
-      case 31: dev_tiled<8, 32, 32, 2, 1, true>(D, lu, lds); break;
-      case 32: dev_tiled<8, 32, 32, 1, 2, true>(D, lu, lds); break;
-      case 33: dev_tiled<8, 32, 32, 2, 2, true>(D, lu, lds); break;
-      case 34: dev_tiled<16, 32, 32, 1, 1, true>(D, lu, lds); break;
+      case 23: dev_tiled<4, 64, 64, 1, 1, true>(D, lu, lds); break;
+      case 24: dev_tiled<4, 64, 64, 4, 1, true>(D, lu, lds); break;
+      case 25: dev_tiled<4, 64, 64, 1, 4, true>(D, lu, lds); break;
+      case 26: dev_tiled<4, 64, 64, 4, 4, true>(D, lu, lds); break;
+      case 27: dev_tiled<8, 32, 32, 1, 1, true>(D, lu, lds); break;
+      case 28: dev_tiled<8, 32, 32, 2, 1, true>(D, lu, lds); break;
+      case 29: dev_tiled<8, 32, 32, 1, 2, true>(D, lu, lds); break;
+      case 30: dev_tiled<8, 32, 32, 2, 2, true>(D, lu, lds); break;
+      case 31: dev_tiled<16, 32, 32, 1, 1, true>(D, lu, lds); break;
       default: break;
     }
   } else if constexpr (FAM == kFamCopy) {
     switch (D.variant) {
-      case 9: dev_copy<4, 16>(D, lu); break;
-      case 10: dev_copy<4, 64>(D, lu); break;
-      case 11: dev_copy<8, 16>(D, lu); break;
-      case 12: dev_copy<8, 64>(D, lu); break;
-      case 13: dev_copy<16, 16>(D, lu); break;
-      case 14: dev_copy<16, 64>(D, lu); break;
+      case 9: dev_copy<4>(D, lu); break;
+      case 10: dev_copy<8>(D, lu); break;
+      case 11: dev_copy<16>(D, lu); break;
       default: break;
     }
   } else {
     switch (D.variant) {
-      case 15: dev_packed<4, 1>(D, lu, lds); break;
-      case 16: dev_packed<4, 2>(D, lu, lds); break;
-      case 17: dev_packed<4, 4>(D, lu, lds); break;
-      case 18: dev_packed<4, 8>(D, lu, lds); break;
-      case 19: dev_packed<8, 1>(D, lu, lds); break;
-      case 20: dev_packed<8, 2>(D, lu, lds); break;
-      case 21: dev_packed<8, 4>(D, lu, lds); break;
-      case 22: dev_packed<8, 8>(D, lu, lds); break;
-      case 23: dev_packed<16, 1>(D, lu, lds); break;
-      case 24: dev_packed<16, 2>(D, lu, lds); break;
-      case 25: dev_packed<16, 4>(D, lu, lds); break;
+      case 12: dev_packed<4, 1>(D, lu, lds); break;
+      case 13: dev_packed<4, 2>(D, lu, lds); break;
+      case 14: dev_packed<4, 4>(D, lu, lds); break;
+      case 15: dev_packed<4, 8>(D, lu, lds); break;
+      case 16: dev_packed<8, 1>(D, lu, lds); break;
+      case 17: dev_packed<8, 2>(D, lu, lds); break;
+      case 18: dev_packed<8, 4>(D, lu, lds); break;
+      case 19: dev_packed<8, 8>(D, lu, lds); break;
+      case 20: dev_packed<16, 1>(D, lu, lds); break;
+      case 21: dev_packed<16, 2>(D, lu, lds); break;
+      case 22: dev_packed<16, 4>(D, lu, lds); break;
       default: break;
     }
   }
@@ -227,14 +220,13 @@ void host_tiled(const BatchDesc& D, int lu, unsigned char* lds_raw) {
   }
 }
 
-template <int W, int TX>
+template <int B>
 void host_copy(const BatchDesc& D, int lu) {
-  using Ops = CopyOps<W, TX, 4>;
-  using V = typename Ops::V;
-  for (int w = lu; w < D.items; w += D.groups) {
-    const TileCtx c = Ops::item(D.a.copy, (uint32_t)w);
-    for (int t = 0; t < 256; t++) Ops::run(D.a.copy, c, t, static_cast<const V*>(D.in), static_cast<V*>(D.out));
-  }
+  using Ops = CopyOps<B>;
+  using E = typename Ops::E;
+  for (int w = lu; w < D.items; w += D.groups)
+    for (int t = 0; t < Ops::NT; t++)
+      Ops::run(D.a.copy, (uint32_t)w, t, static_cast<const E*>(D.in), static_cast<E*>(D.out));
 }
 
 template <int B, int NREG>
@@ -266,32 +258,29 @@ void host_unit(const BatchDesc& D, int lu, unsigned char* lds) {
     case 6: host_tiled<8, 32, 32, 1, 2>(D, lu, lds); break;
     case 7: host_tiled<8, 32, 32, 2, 2>(D, lu, lds); break;
     case 8: host_tiled<16, 32, 32, 1, 1>(D, lu, lds); break;
-    case 9: host_copy<4, 16>(D, lu); break;
-    case 10: host_copy<4, 64>(D, lu); break;
-    case 11: host_copy<8, 16>(D, lu); break;
-    case 12: host_copy<8, 64>(D, lu); break;
-    case 13: host_copy<16, 16>(D, lu); break;
-    case 14: host_copy<16, 64>(D, lu); break;
-    case 15: host_packed<4, 1>(D, lu, lds); break;
-    case 16: host_packed<4, 2>(D, lu, lds); break;
-    case 17: host_packed<4, 4>(D, lu, lds); break;
-    case 18: host_packed<4, 8>(D, lu, lds); break;
-    case 19: host_packed<8, 1>(D, lu, lds); break;
-    case 20: host_packed<8, 2>(D, lu, lds); break;
-    case 21: host_packed<8, 4>(D, lu, lds); break;
-    case 22: host_packed<8, 8>(D, lu, lds); break;
-    case 23: host_packed<16, 1>(D, lu, lds); break;
-    case 24: host_packed<16, 2>(D, lu, lds); break;
-    case 25: host_packed<16, 4>(D, lu, lds); break;
-    case 26: host_tiled<4, 64, 64, 1, 1, true>(D, lu, lds); break;
-    case 27: host_tiled<4, 64, 64, 4, 1, true>(D, lu, lds); break;
-    case 28: host_tiled<4, 64, 64, 1, 4, true>(D, lu, lds); break;
-    case 29: host_tiled<4, 64, 64, 4, 4, true>(D, lu, lds); break;
-    case 30: host_tiled<8, 32, 32, 1, 1, true>(D, lu, lds); break;
-    case 31: host_tiled<8, 32, 32, 2, 1, true>(D, lu, lds); break;
-    case 32: host_tiled<8, 32, 32, 1, 2, true>(D, lu, lds); break;
-    case 33: host_tiled<8, 32, 32, 2, 2, true>(D, lu, lds); break;
-    case 34: host_tiled<16, 32, 32, 1, 1, true>(D, lu, lds); break;
+    case 9: host_copy<4>(D, lu); break;
+    case 10: host_copy<8>(D, lu); break;
+    case 11: host_copy<16>(D, lu); break;
+    case 12: host_packed<4, 1>(D, lu, lds); break;
+    case 13: host_packed<4, 2>(D, lu, lds); break;
+    case 14: host_packed<4, 4>(D, lu, lds); break;
+    case 15: host_packed<4, 8>(D, lu, lds); break;
+    case 16: host_packed<8, 1>(D, lu, lds); break;
+    case 17: host_packed<8, 2>(D, lu, lds); break;
+    case 18: host_packed<8, 4>(D, lu, lds); break;
+    case 19: host_packed<8, 8>(D, lu, lds); break;
+    case 20: host_packed<16, 1>(D, lu, lds); break;
+    case 21: host_packed<16, 2>(D, lu, lds); break;
+    case 22: host_packed<16, 4>(D, lu, lds); break;
+    case 23: host_tiled<4, 64, 64, 1, 1, true>(D, lu, lds); break;
+    case 24: host_tiled<4, 64, 64, 4, 1, true>(D, lu, lds); break;
+    case 25: host_tiled<4, 64, 64, 1, 4, true>(D, lu, lds); break;
+    case 26: host_tiled<4, 64, 64, 4, 4, true>(D, lu, lds); break;
+    case 27: host_tiled<8, 32, 32, 1, 1, true>(D, lu, lds); break;
+    case 28: host_tiled<8, 32, 32, 2, 1, true>(D, lu, lds); break;
+    case 29: host_tiled<8, 32, 32, 1, 2, true>(D, lu, lds); break;
+    case 30: host_tiled<8, 32, 32, 2, 2, true>(D, lu, lds); break;
+    case 31: host_tiled<16, 32, 32, 1, 1, true>(D, lu, lds); break;
     default: break;
   }
 }
@@ -303,12 +292,6 @@ bool batch_tiled_available(int elem, int tx, int ty, int vx, int vy, bool genera
     if (s.method == kTiled && s.b == elem && s.p1 == tx && s.p2 == ty && s.p3 == vx && s.p4 == vy &&
         (s.g != 0) == general)
       return true;
-  return false;
-}
-
-bool batch_copy_available(int word, int tx) {
-  for (const auto& s : kBatchShapes)
-    if (s.method == kTiledCopy && s.p1 == word && s.p2 == tx) return true;
   return false;
 }
 
@@ -340,7 +323,7 @@ int batch_variant(const Candidate& c) {
           return s.id;
         break;
       case kTiledCopy:
-        if (s.method == kTiledCopy && s.p1 == c.word && s.p2 == c.copy_tx) return s.id;
+        if (s.method == kTiledCopy && s.b == c.elem) return s.id;
         break;
       case kPacked:
       case kPackedSplit:
@@ -368,7 +351,7 @@ bool batch_describe(const Candidate& c, BatchDesc& d) {
     case kTiledCopy:
       d.a.copy = c.copy;
       d.items = c.copy.items;
-      d.item_bytes = 2 * 1024 * c.word;  // copy_tx words x 1024/copy_tx rows
+      d.item_bytes = 2 * c.copy.per * c.elem;
       break;
     default:
       d.a.packed = c.packed;
@@ -406,7 +389,7 @@ long long batch_unit_bytes(long long total_bytes, int grid) {
 }
 
 int batch_family(int variant) {
-  return variant <= 8 ? kFamTiled : variant <= 14 ? kFamCopy : variant <= 25 ? kFamPacked : kFamTiledG;
+  return variant <= 8 ? kFamTiled : variant <= 11 ? kFamCopy : variant <= 22 ? kFamPacked : kFamTiledG;
 }
 
 hipError_t launch_batch(int fam, const BatchDesc* d_descs, const int* d_start, int nprob, int total, int grid,

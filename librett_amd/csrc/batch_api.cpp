@@ -51,43 +51,26 @@ int check_problem(int rank, const int* dim, const int* perm, size_t elem) {
   return LIBRETT_C_SUCCESS;
 }
 
-// A flat copy of `bytes` bytes in words of W bytes as TiledCopy
-// descriptors: 64-word rows, plus a one-row descriptor for the tail. Used for
-// problems that reduce to a plain copy (the reference's Trivial method).
-void copy_descs(long long bytes, int W, std::vector<BatchDesc>& out, std::vector<long long>& byte_offsets) {
-  const long long n = bytes / W;
-  const long long rows = n / 64, tail = n % 64;
-  auto make = [&](int X, long long Y, long long off_words) {
-    Candidate c;
-    c.method = kTiledCopy;
-    c.word = W;
-    c.elem = W;
-    c.copy_tx = X <= 16 ? 16 : 64;
-    CopyArgs& a = c.copy;
-    a.X = X;
-    a.Y = (int)Y;
-    a.in_ys = X;
-    a.out_ys = X;
-    const int ty = (256 / c.copy_tx) * 4;
-    a.ntx = (X + c.copy_tx - 1) / c.copy_tx;
-    const int nty = (int)((Y + ty - 1) / ty);
-    a.ntiles = a.ntx * nty;
-    a.ntx_div = make_fastdiv((uint32_t)a.ntx);
-    a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
-    a.items = a.ntiles;
-    a.outer.n = 0;
-    for (int r = 0; r < kMaxRank; r++) {
-      a.outer.div[r] = make_fastdiv(1);
-      a.outer.ct_in[r] = a.outer.ct_out[r] = 0;
-    }
-    BatchDesc d;
-    if (batch_describe(c, d)) {
-      out.push_back(d);
-      byte_offsets.push_back(off_words * W);
-    }
-  };
-  if (rows > 0) make(64, rows, 0);
-  if (tail > 0) make((int)tail, 1, rows * 64);
+// A problem that reduces to a plain copy (the reference's Trivial method) as
+// a TiledCopy candidate of one row.
+Candidate flat_copy(const Problem& p) {
+  Candidate c;
+  c.method = kTiledCopy;
+  c.elem = p.elem;
+  c.word = 16;
+  CopyArgs& a = c.copy;
+  a.n = a.X = (int)p.vol;
+  a.row_div = make_fastdiv((uint32_t)p.vol);
+  a.per = 256 * (16 / p.elem);
+  a.items = (int)((p.vol + 128 / p.elem - 1 + a.per - 1) / a.per);
+  a.xcds = 1;
+  a.stream_in = 0;
+  a.rows.n = 0;
+  for (int r = 0; r < kMaxRank; r++) {
+    a.rows.div[r] = make_fastdiv(1);
+    a.rows.ct_in[r] = a.rows.ct_out[r] = 0;
+  }
+  return c;
 }
 
 struct BatchObj {
@@ -355,7 +338,7 @@ std::vector<Candidate> batch_candidates(const Problem& p, const DeviceInfo& dev)
   std::vector<Candidate> cands = make_candidates(p, bdev);
   std::vector<Candidate> ok;
   for (auto& c : cands)
-    if (c.method == kTrivial || batch_variant(c) >= 0) ok.push_back(c);
+    if (c.method == kTrivial || (batch_variant(c) >= 0 && !copy_beats(cands, c))) ok.push_back(c);
   std::stable_sort(ok.begin(), ok.end(), [](const Candidate& a, const Candidate& b) {
     return a.model.t_stream < b.model.t_stream;
   });
@@ -365,7 +348,6 @@ std::vector<Candidate> batch_candidates(const Problem& p, const DeviceInfo& dev)
 int batch_alignment(const Problem& p, const Candidate& c) {
   if (c.method == kTrivial) return p.elem;
   if (c.method == kTiled) return c.elem * std::max(c.vec_x, c.vec_y);
-  if (c.method == kTiledCopy) return c.word;
   return c.elem;
 }
 
@@ -374,37 +356,10 @@ bool describe_problem(const Problem& p, const Candidate& c, std::vector<BatchDes
   descs.clear();
   fallback.clear();
   offsets.clear();
-  if (c.method == kTrivial) {
-    // Element-sized words: always aligned, so the fallback is the same.
-    copy_descs((long long)p.vol * p.elem, p.elem, descs, offsets);
-    fallback = descs;
-    return !descs.empty();
-  }
   BatchDesc d, f;
-  if (!batch_describe(c, d)) return false;
-  Candidate fc = c;
+  if (!batch_describe(c.method == kTrivial ? flat_copy(p) : c, d)) return false;
+  Candidate fc = c.method == kTrivial ? flat_copy(p) : c;
   if (c.method == kTiled) fc.vec_x = fc.vec_y = 1;
-  if (c.method == kTiledCopy && c.word > c.elem) {
-    // Element-sized words for unaligned buffers.
-    const int k = c.word / c.elem;
-    CopyArgs& a = fc.copy;
-    a.X *= k;
-    a.in_ys *= k;
-    a.out_ys *= k;
-    for (int r = 0; r < a.outer.n; r++) {
-      a.outer.ct_in[r] *= k;
-      a.outer.ct_out[r] *= k;
-    }
-    fc.word = c.elem;
-    fc.copy_tx = 64;
-    const int ty = (256 / fc.copy_tx) * 4;
-    const long long vol_outer = c.copy.items / std::max(1, c.copy.ntiles);
-    a.ntx = (a.X + fc.copy_tx - 1) / fc.copy_tx;
-    a.ntiles = a.ntx * ((a.Y + ty - 1) / ty);
-    a.ntx_div = make_fastdiv((uint32_t)a.ntx);
-    a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
-    a.items = (int)(a.ntiles * vol_outer);
-  }
   if (!batch_describe(fc, f)) f = d;
   descs.push_back(d);
   fallback.push_back(f);
@@ -645,21 +600,20 @@ int librett_c_batch_host_candidate(int rank, const int* dim, const int* permutat
     if (fallback) ds = fs;
     const long long ub = unit_bytes > 0 ? unit_bytes : kBatchUnitBytes;
     const size_t n = (size_t)p.vol * p.elem;
-    const size_t g = 4096;
-    std::vector<unsigned char> gin(n + 2 * g, 0xA5), gout(n + 2 * g, 0x5A);
-    std::memcpy(gin.data() + g, idata, n);
+    const int align = fallback ? p.elem : batch_alignment(p, ranked[index]);
+    GuardedBuffer gin(n, idata, align, 0xA5), gout(n, odata, align, 0x5A);
+    std::memcpy(gin.data(), idata, n);
     std::vector<int> start(ds.size() + 1, 0);
     for (size_t k = 0; k < ds.size(); k++) {
       batch_regroup(ds[k], ub);
-      ds[k].in = gin.data() + g + offs[k];
-      ds[k].out = gout.data() + g + offs[k];
+      ds[k].in = gin.data() + offs[k];
+      ds[k].out = gout.data() + offs[k];
       start[k + 1] = start[k] + ds[k].units;
     }
     const int gr = grid > 0 ? grid : dev.cu_count * 4;
     if (!replay_batch(ds.data(), start.data(), (int)ds.size(), start.back(), gr)) return LIBRETT_C_UNDEFINED_ERROR;
-    for (size_t j = 0; j < g; j++)
-      if (gout[j] != 0x5A || gout[g + n + j] != 0x5A) return LIBRETT_C_UNDEFINED_ERROR;
-    std::memcpy(odata, gout.data() + g, n);
+    if (!gout.intact()) return LIBRETT_C_UNDEFINED_ERROR;
+    std::memcpy(odata, gout.data(), n);
     return LIBRETT_C_SUCCESS;
   } catch (...) {
     return LIBRETT_C_INTERNAL_ERROR;

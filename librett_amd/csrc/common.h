@@ -154,22 +154,32 @@ __host__ __device__ inline int tiled_in_y(const TiledArgs& a, uint32_t y) {
   return a.yg.n > 1 ? group_offset(a.yg, y) : (int)y * a.in_ys;
 }
 
-// TiledCopy: rows that stay contiguous in input and output (perm[0] == 0),
-// moved as W-byte words. Plane = (x = words of dim 0, y = the input dim that
-// becomes output dim 1). Reference counterpart: transposeTiledCopy,
-// src/kernel.cpp:453-545.
+// TiledCopy: rows that stay contiguous in input and output (perm[0] == 0).
+// The output is written front to back, so its element index is (row, c) with
+// row = e / X; the row's digits in output order give its input offset.
+// Reference counterpart: transposeTiledCopy, src/kernel.cpp:453-545.
 struct CopyArgs {
-  int X, Y;          // plane extents (x in words)
-  int in_ys;         // input stride of y in words
-  int out_ys;        // output stride of y in words
-  int ntx;
-  int ntiles;
-  FastDiv ntx_div;
-  FastDiv ntiles_div;
-  int items;
+  int n;             // elements
+  int X;             // elements per row
+  FastDiv row_div;   // X
+  int per;           // elements per item (CopyOps::PER)
+  int items;         // items; in the batched engine enough for an output at any address
   int xcds;          // work order across XCDs, as in TiledArgs
-  OuterMap outer;    // strides in words
+  int stream_in;     // non-temporal loads: the input cannot stay in the Infinity Cache
+  // Row index digits, fastest first: ct_in[r] elements of input each. The
+  // last digit needs no division.
+  OuterMap rows;
 };
+
+__host__ __device__ inline int copy_row_offset(const OuterMap& m, uint32_t row) {
+  int off = 0;
+  for (int r = 0; r + 1 < m.n; r++) {
+    const uint32_t q = fdiv(row, m.div[r]);
+    off += (int)(row - q * m.div[r].d) * m.ct_in[r];
+    row = q;
+  }
+  return m.n > 0 ? off + (int)row * m.ct_in[m.n - 1] : off;
+}
 
 // One on-chip ("Mmk") sub-tensor shape. The LDS holds it in input order, so
 // LDS position p is also its input-order linear index. Input-order digits of

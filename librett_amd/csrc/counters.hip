@@ -34,14 +34,18 @@ namespace {
 constexpr int kCountThreads = 256;
 constexpr int kCountMaxGrid = 2048;
 
+// Row pieces of a TiledCopy item: at most 1024 elements (of 4 bytes) in rows
+// of at least 2, the first of which may be cut.
+constexpr int kCopyPieces = 514;
+
 struct RunRef {
   int off, n;  // start and length in the run table (pairs of ints)
 };
 
 struct CountJob {
   int method;          // kTiled, kTiledCopy, kPacked or kPackedSplit
-  int B;               // element bytes (Tiled, Packed) or word bytes (TiledCopy)
-  int TX, TY, VX, VY;  // Tiled: tile and vector widths; TiledCopy: TX words, TY rows
+  int B;               // element bytes
+  int TX, TY, VX, VY;  // Tiled: tile and vector widths
   int nt, nreg;        // Packed: threads and registers (passes) per thread
   long long items;
   const int* runs;     // Packed: (start, length) element runs of each staged shape
@@ -56,12 +60,12 @@ struct CountJob {
 __host__ __device__ inline int imin(int a, int b) { return a < b ? a : b; }
 
 struct ItemCtx {
-  int x0, y0, tx, ty;  // Tiled / TiledCopy: tile origin and extent
+  int x0, y0, tx, ty;  // Tiled: tile origin and extent
   int plus;            // Packed: staged shape variant
-  long long in0, out0; // element (or word) offset of the item's base
+  long long in0, out0; // element offset of the item's base (TiledCopy: out0 only)
 };
 
-// Tile origin of work item w; same order as TiledOps::item / CopyOps::item.
+// Origin of work item w; same order as TiledOps::item.
 __host__ __device__ inline ItemCtx item_ctx(const CountJob& j, uint32_t w) {
   ItemCtx c{};
   if (j.method == kTiled) {
@@ -88,19 +92,7 @@ __host__ __device__ inline ItemCtx item_ctx(const CountJob& j, uint32_t w) {
     c.in0 = oi;
     c.out0 = oo;
   } else if (j.method == kTiledCopy) {
-    const CopyArgs& a = j.a.copy;
-    const uint32_t mb = fdiv(w, a.ntiles_div);
-    const uint32_t tile = w - mb * (uint32_t)a.ntiles;
-    const uint32_t ty = fdiv(tile, a.ntx_div);
-    const uint32_t tx = tile - ty * (uint32_t)a.ntx;
-    c.x0 = (int)tx * j.TX;
-    c.y0 = (int)ty * j.TY;
-    c.tx = imin(j.TX, a.X - c.x0);
-    c.ty = imin(j.TY, a.Y - c.y0);
-    int oi, oo;
-    outer_offsets(a.outer, mb, oi, oo);
-    c.in0 = oi;
-    c.out0 = oo;
+    c.out0 = (long long)w * j.a.copy.per;
   } else {
     // Round (split, o): chunk `split` of the split dim at outer index o, as
     // PackedOps::prepare and the outer loop of k_packed address it.
@@ -129,7 +121,10 @@ __host__ __device__ inline int job_passes(const CountJob& j, int store) {
     case kTiled:
       return store ? (j.TX * j.TY) / (j.VY * kCountThreads) : (j.TX * j.TY) / (j.VX * kCountThreads);
     case kTiledCopy:
-      return j.TY / (kCountThreads / j.TX);
+      // A lane's word, or the elements of a word that crosses a row's end
+      // (loads) or the tensor's end: its k-th access is counted with the other
+      // lanes' k-th.
+      return 16 / j.B;
     default:
       return j.nreg;
   }
@@ -141,10 +136,11 @@ __host__ __device__ inline int job_access_bytes(const CountJob& j, int store) {
 }
 
 // Byte offset of thread t's access in pass p of an item, false when the lane
-// is inactive. Mirrors the lane arithmetic of TiledOps::load / store,
+// is inactive; `bytes` changes where the access is not job_access_bytes long.
+// Mirrors the lane arithmetic of TiledOps::load / store,
 // CopyOps::run and PackedOps::prepare / load / store.
 __host__ __device__ inline bool lane_access(const CountJob& j, const ItemCtx& c, int store, int p, int t,
-                                            long long& off) {
+                                            long long& off, int& bytes) {
   if (j.method == kTiled) {
     const TiledArgs& a = j.a.tiled;
     if (!store) {
@@ -165,12 +161,19 @@ __host__ __device__ inline bool lane_access(const CountJob& j, const ItemCtx& c,
     return true;
   }
   if (j.method == kTiledCopy) {
+    // Addresses for an output that starts on a line.
     const CopyArgs& a = j.a.copy;
-    const int RP = kCountThreads / j.TX;
-    const int x = c.x0 + t % j.TX;
-    const int y = c.y0 + t / j.TX + p * RP;
-    if (x >= a.X || y >= a.Y) return false;
-    off = (long long)((store ? c.out0 : c.in0) + x + (long long)y * (store ? a.out_ys : a.in_ys)) * j.B;
+    const int pe = 16 / j.B;
+    const long long e = c.out0 + (long long)t * pe;
+    if (e >= a.n) return false;
+    const long long row = e / a.X, k = e - row * a.X;
+    const bool word = a.n - e >= pe && (store || a.X - k >= pe);
+    if (word && p > 0) return false;
+    if (word) bytes = 16;
+    const long long q = e + p;
+    if (q >= a.n) return false;
+    const long long qrow = q / a.X;
+    off = (store ? q : copy_row_offset(a.rows, (uint32_t)qrow) + (q - qrow * a.X)) * j.B;
     return true;
   }
   const StagedShape& s = j.a.packed.shape[c.plus];
@@ -237,8 +240,9 @@ __host__ __device__ inline void sort_small(long long* v, int n) {
 }
 
 // Lines one item reads and writes: Tiled reads tile rows (y ascending) and
-// writes tile columns (x ascending); TiledCopy reads and writes rows; Packed
-// walks the staged shape's runs, which the host sorted by start.
+// writes tile columns (x ascending); TiledCopy reads pieces of rows and
+// writes one run; Packed walks the staged shape's runs, which the host sorted
+// by start.
 __host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, unsigned long long* acc) {
   LineWalk rd, wr;
   const long long B = j.B;
@@ -254,11 +258,22 @@ __host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, 
     if (a.xg.n > 1) sort_small(st, c.tx);
     for (int x = 0; x < c.tx; x++) wr.add(st[x], c.ty * B);
   } else if (j.method == kTiledCopy) {
+    // Whole rows lie anywhere in the input, so their starts are sorted; the
+    // item's first and last row may be cut.
     const CopyArgs& a = j.a.copy;
-    for (int y = 0; y < c.ty; y++) {
-      rd.add((c.in0 + c.x0 + (long long)(c.y0 + y) * a.in_ys) * B, c.tx * B);
-      wr.add((c.out0 + c.x0 + (long long)(c.y0 + y) * a.out_ys) * B, c.tx * B);
+    const long long e1 = c.out0 + a.per < a.n ? c.out0 + a.per : a.n;
+    long long st[kCopyPieces];
+    int ns = 0;
+    for (long long e = c.out0; e < e1; ns++) {
+      const long long row = e / a.X, k = e - row * a.X;
+      const long long len = a.X - k < e1 - e ? a.X - k : e1 - e;
+      // Start and length in one sortable value.
+      st[ns] = ((copy_row_offset(a.rows, (uint32_t)row) + k) << 12) | len;
+      e += len;
     }
+    sort_small(st, ns);
+    for (int i = 0; i < ns; i++) rd.add((st[i] >> 12) * B, (st[i] & 4095) * B);
+    wr.add(c.out0 * B, (e1 - c.out0) * B);
   } else {
     const RunRef ri = j.run[c.plus][0], ro = j.run[c.plus][1];
     for (int r = 0; r < ri.n; r++) {
@@ -279,7 +294,8 @@ __host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, 
 }
 
 // One wave instruction: requests, distinct 128-byte segments and bytes of
-// its active lanes. An access of `bytes` may span two segments; both count.
+// its active lanes (each moves `bytes` bytes, which may differ between lanes).
+// An access may span two segments; both count.
 __device__ inline void wave_count(bool act, long long off, int bytes, int lane, unsigned long long& req,
                                   unsigned long long& tran, unsigned long long& nbytes) {
   const unsigned long long m = __ballot(act);
@@ -304,7 +320,13 @@ __device__ inline void wave_count(bool act, long long off, int bytes, int lane, 
   if (lane == 0) {
     req += 1;
     tran += (unsigned long long)n;
-    nbytes += (unsigned long long)__popcll(m) * (unsigned long long)bytes;
+  }
+  left = m;
+  while (left) {
+    const int b = __shfl(bytes, __ffsll((unsigned long long)left) - 1);
+    const unsigned long long same = __ballot(act && bytes == b);
+    if (lane == 0) nbytes += (unsigned long long)__popcll(same) * (unsigned long long)b;
+    left &= ~same;
   }
 }
 
@@ -320,12 +342,12 @@ __global__ __launch_bounds__(kCountThreads) void k_count(CountJob job, unsigned 
     const ItemCtx c = item_ctx(job, (uint32_t)w);
     for (int store = 0; store < 2; store++) {
       const int np = job_passes(job, store);
-      const int bytes = job_access_bytes(job, store);
       for (int p = 0; p < np; p++)
         for (int v = wv; v < waves; v += kCountThreads / 64) {
           const int t = v * 64 + lane;
           long long off = 0;
-          const bool act = t < nthreads && lane_access(job, c, store, p, t, off);
+          int bytes = job_access_bytes(job, store);
+          const bool act = t < nthreads && lane_access(job, c, store, p, t, off, bytes);
           wave_count(act, off, bytes, lane, acc[kLdReq + store], acc[kLdTran + store], acc[kLdBytes + store]);
         }
     }
@@ -344,7 +366,7 @@ __global__ __launch_bounds__(kCountThreads) void k_count(CountJob job, unsigned 
 }
 
 // Host version of wave_count over one wave's lanes.
-void host_wave_count(const bool* act, const long long* off, int bytes, unsigned long long& req,
+void host_wave_count(const bool* act, const long long* off, const int* bytes, unsigned long long& req,
                      unsigned long long& tran, unsigned long long& nbytes) {
   long long segs[128];
   int ns = 0, na = 0;
@@ -352,13 +374,13 @@ void host_wave_count(const bool* act, const long long* off, int bytes, unsigned 
     if (!act[l]) continue;
     na++;
     segs[ns++] = off[l] >> 7;
-    segs[ns++] = (off[l] + bytes - 1) >> 7;
+    segs[ns++] = (off[l] + bytes[l] - 1) >> 7;
+    nbytes += (unsigned long long)bytes[l];
   }
   if (na == 0) return;
   std::sort(segs, segs + ns);
   req += 1;
   tran += (unsigned long long)(std::unique(segs, segs + ns) - segs);
-  nbytes += (unsigned long long)na * (unsigned long long)bytes;
 }
 
 // Fills a job from a candidate; `runs` receives the Packed run table (host
@@ -379,10 +401,8 @@ bool make_job(const Candidate& c, CountJob& j, std::vector<int>& runs) {
       if (j.TX % j.VX || j.TY % j.VY || kCountThreads % (j.TX / j.VX) || kCountThreads % (j.TY / j.VY)) return false;
       return job_passes(j, 0) >= 1 && job_passes(j, 1) >= 1;
     case kTiledCopy:
-      j.B = c.word;
-      j.TX = c.copy_tx;
-      if (j.TX <= 0 || kCountThreads % j.TX) return false;
-      j.TY = (kCountThreads / j.TX) * 4;  // CopyOps<W, TX, 4>
+      j.B = c.elem;
+      if (c.copy.per != kCountThreads * (16 / j.B) || c.copy.X < 2) return false;
       j.a.copy = c.copy;
       j.items = c.copy.items;
       return true;
@@ -421,18 +441,19 @@ void host_walk(const CountJob& j, unsigned long long* acc, F&& f) {
   const int waves = (nthreads + 63) / 64;
   bool act[64];
   long long off[64];
+  int bytes[64];
   for (long long w = 0; w < j.items; w++) {
     const ItemCtx c = item_ctx(j, (uint32_t)w);
     for (int store = 0; store < 2; store++) {
       const int np = job_passes(j, store);
-      const int bytes = job_access_bytes(j, store);
       for (int p = 0; p < np; p++)
         for (int v = 0; v < waves; v++) {
           for (int l = 0; l < 64; l++) {
             const int t = v * 64 + l;
             off[l] = 0;
-            act[l] = t < nthreads && lane_access(j, c, store, p, t, off[l]);
-            if (act[l]) f(w, store, p, t, off[l], bytes);
+            bytes[l] = job_access_bytes(j, store);
+            act[l] = t < nthreads && lane_access(j, c, store, p, t, off[l], bytes[l]);
+            if (act[l]) f(w, store, p, t, off[l], bytes[l]);
           }
           host_wave_count(act, off, bytes, acc[kLdReq + store], acc[kLdTran + store], acc[kLdBytes + store]);
         }
@@ -531,10 +552,11 @@ bool trace_kernel(const Candidate& c, std::vector<AccessRecord>& recs) {
   recs.clear();
   if (c.method == kTrivial) return false;
   const size_t n = (size_t)(c.bytes / 2);
-  std::vector<unsigned char> in(n + 16, 0), out(n + 16, 0);
-  // 16-byte aligned bases, as device allocations are (vector accesses).
-  unsigned char* pi = in.data() + ((16 - ((uintptr_t)in.data() & 15)) & 15);
-  unsigned char* po = out.data() + ((16 - ((uintptr_t)out.data() & 15)) & 15);
+  std::vector<unsigned char> in(n + 128, 0), out(n + 128, 0);
+  // Line-aligned bases, as device allocations are: where a word of the output
+  // begins depends on the base's place in its line.
+  unsigned char* pi = in.data() + ((128 - ((uintptr_t)in.data() & 127)) & 127);
+  unsigned char* po = out.data() + ((128 - ((uintptr_t)out.data() & 127)) & 127);
   if ((size_t)(pi - in.data()) + n > in.size() || (size_t)(po - out.data()) + n > out.size()) return false;
   TraceObserver obs;
   obs.in = pi;

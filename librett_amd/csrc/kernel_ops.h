@@ -34,16 +34,14 @@ __host__ __device__ inline void vset(V& v, int k, const E& e) {
 }
 
 // Global stores and loads of the transpose kernels. Every output byte is
-// written once and never read back by the kernel, and every input byte is
-// read once, so streaming (non-temporal) accesses keep the caches from
-// holding lines nobody will reuse. On MI355X, non-temporal stores lift a
-// plain 256 MiB copy from about 5.5 to about 7.1 TB/s. LRT_NT_STORES and
-// LRT_NT_LOADS select them at build time.
+// written once and never read back by the kernel, so stores are streaming
+// (non-temporal): on MI355X they lift a plain 256 MiB copy from about 5.5 to
+// about 7.1 TB/s. LRT_NT_STORES selects them at build time. Loads are
+// streaming only where a kernel says so (STREAM): they help where whole lines
+// are read once and the input is too large for the 256 MiB Infinity Cache,
+// and cost where neighbouring work items share lines.
 #ifndef LRT_NT_STORES
 #define LRT_NT_STORES 1
-#endif
-#ifndef LRT_NT_LOADS
-#define LRT_NT_LOADS 0
 #endif
 // Host replay only: an observer that is told which work item and thread the
 // replay is running and sees every global load and store it makes. The
@@ -68,18 +66,42 @@ __host__ __device__ inline void st(V* p, const V& v) {
   *p = v;
 #endif
 }
-template <typename V>
+template <bool STREAM = false, typename V>
 __host__ __device__ inline V ld(const V* p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-#if LRT_NT_LOADS
-  return __builtin_nontemporal_load(p);
-#else
-  return *p;
-#endif
+  if constexpr (STREAM)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
 #else
   if (g_replay_observer) g_replay_observer->access(p, (int)sizeof(V), 0);
   return *p;
 #endif
+}
+
+// A V read from an address that is a multiple of AL bytes only (gfx950 loads
+// 16 bytes from any 4-byte boundary in one instruction).
+template <typename V, int AL, bool STREAM = false>
+__host__ __device__ inline V ld_unaligned(const void* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef V U __attribute__((aligned(AL)));
+  if constexpr (STREAM)
+    return __builtin_nontemporal_load(static_cast<const U*>(p));
+  else
+    return *static_cast<const U*>(p);
+#else
+  if (g_replay_observer) g_replay_observer->access(p, (int)sizeof(V), 0);
+  V v;
+  __builtin_memcpy(&v, p, sizeof(V));
+  return v;
+#endif
+}
+
+// Elements between the last 128-byte line boundary and p (p a multiple of
+// the element size).
+template <typename E>
+__host__ __device__ inline int line_phase(const E* p) {
+  return (int)(((uintptr_t)p & 127) / sizeof(E));
 }
 
 struct TileCtx {
@@ -237,59 +259,73 @@ struct TiledOps {
 };
 
 // ---------------------------------------------------------------------------
-// TiledCopy: rows that are contiguous in both tensors, moved as W-byte words
-// straight through registers. TX words per tile row, 256 / TX rows per pass,
-// NP passes. Reference counterpart: transposeTiledCopy, src/kernel.cpp:453-545.
+// TiledCopy: rows that are contiguous in both tensors (perm[0] == 0). The
+// output is written front to back in 16-byte words that start on its 16-byte
+// boundaries, so a wave stores 1024 consecutive bytes in whole lines whatever
+// the row length; each thread finds its word's row and input offset by
+// itself and loads the word from wherever the row starts (any element
+// boundary). A word that crosses a row's end is loaded element by element.
+// Bound by HBM. On MI355X a copy of [2307, 115, 126] f64 rows (18456 B, no
+// row on a line boundary) takes 86 us against 129 us for row tiles of 8-byte
+// words, whose lines are written in two parts by different workgroups, and
+// [1024, 256, 256] f32 takes 86 us against 94 us; a plain copy of the bytes
+// takes 85 us. One word per thread runs faster than two or four (85.8, 87.8,
+// 90.3 us; in the batched engine 3.34 ms against 3.46 ms for four): more,
+// shorter workgroups keep the open DRAM pages close together.
+// Reference counterpart: transposeTiledCopy, src/kernel.cpp:453-545.
 // ---------------------------------------------------------------------------
-template <int W, int TX, int NP>
+template <int B>
 struct CopyOps {
-  using V = typename Word<W>::type;
+  using E = typename Word<B>::type;
+  using V = typename Word<16>::type;
   static constexpr int NT = 256;
-  static constexpr int RP = NT / TX;
-  static constexpr int TY = RP * NP;
-  static_assert(NT % TX == 0, "copy shape");
+  static constexpr int PE = 16 / B;    // elements per word
+  static constexpr int PER = NT * PE;  // elements per item
 
-  __host__ __device__ static TileCtx item(const CopyArgs& a, uint32_t w) {
-    TileCtx c;
-    uint32_t mb = fdiv(w, a.ntiles_div);
-    uint32_t tile = w - mb * (uint32_t)a.ntiles;
-    uint32_t ty = fdiv(tile, a.ntx_div);
-    uint32_t tx = tile - ty * (uint32_t)a.ntx;
-    c.x0 = (int)tx * TX;
-    c.y0 = (int)ty * TY;
-    outer_offsets(a.outer, mb, c.off_in, c.off_out);
-    c.full = (c.x0 + TX <= a.X) && (c.y0 + TY <= a.Y);
-    return c;
+  // Words of item w start at element w * PER - phase: word boundaries are
+  // 16-byte boundaries of the output's addresses, and items start on lines.
+  __host__ __device__ static void run(const CopyArgs& a, uint32_t w, int t, const E* __restrict__ in,
+                                      E* __restrict__ out) {
+    if (a.stream_in)
+      move<true>(a, w, t, in, out);
+    else
+      move<false>(a, w, t, in, out);
   }
 
-  __host__ __device__ static void run(const CopyArgs& a, const TileCtx& c, int t,
-                                      const V* __restrict__ in, V* __restrict__ out) {
-    const int lx = t % TX;
-    const int ly = t / TX;
-    const int x = c.x0 + lx;
-    V r[NP];
-    if (c.full) {
-      const V* p = in + (c.off_in + x + (c.y0 + ly) * a.in_ys);
-      const int step = RP * a.in_ys;
+  template <bool STREAM>
+  __host__ __device__ static void move(const CopyArgs& a, uint32_t w, int t, const E* __restrict__ in,
+                                       E* __restrict__ out) {
+    const uint32_t e = first(w, t, line_phase(out));
+    if (whole(a, e)) {
+      V r;
+      const uint32_t row = fdiv(e, a.row_div);
+      const int c = (int)(e - row * (uint32_t)a.X);
+      if (a.X - c >= PE) {
+        r = ld_unaligned<V, B, STREAM>(in + (copy_row_offset(a.rows, row) + c));
+      } else {
 #pragma unroll
-      for (int j = 0; j < NP; j++) r[j] = ld(p + j * step);
-      V* q = out + (c.off_out + x + (c.y0 + ly) * a.out_ys);
-      const int ostep = RP * a.out_ys;
-#pragma unroll
-      for (int j = 0; j < NP; j++) st(q + j * ostep, r[j]);
+        for (int k = 0; k < PE; k++) vset<E>(r, k, ld(in + source(a, e + k)));
+      }
+      st(reinterpret_cast<V*>(out + e), r);
     } else {
-      const bool xin = x < a.X;
 #pragma unroll
-      for (int j = 0; j < NP; j++) {
-        const int y = c.y0 + ly + j * RP;
-        if (xin && y < a.Y) r[j] = ld(in + (c.off_in + x + y * a.in_ys));
-      }
-#pragma unroll
-      for (int j = 0; j < NP; j++) {
-        const int y = c.y0 + ly + j * RP;
-        if (xin && y < a.Y) st(out + (c.off_out + x + y * a.out_ys), r[j]);
-      }
+      for (int k = 0; k < PE; k++)
+        if (e + k < (uint32_t)a.n) st(out + (e + k), ld(in + source(a, e + k)));
     }
+  }
+
+  // First element of thread t in item w. Unsigned: elements before the
+  // tensor wrap to values above any volume, as do words past 2^31.
+  __host__ __device__ static uint32_t first(uint32_t w, int t, int phase) {
+    return w * (uint32_t)PER + (uint32_t)(t * PE) - (uint32_t)phase;
+  }
+  __host__ __device__ static bool whole(const CopyArgs& a, uint32_t e) {
+    return e < (uint32_t)a.n && (uint32_t)a.n - e >= (uint32_t)PE;
+  }
+  // Input offset of output element e.
+  __host__ __device__ static int source(const CopyArgs& a, uint32_t e) {
+    const uint32_t row = fdiv(e, a.row_div);
+    return copy_row_offset(a.rows, row) + (int)(e - row * (uint32_t)a.X);
   }
 };
 

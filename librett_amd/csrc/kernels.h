@@ -34,9 +34,7 @@ void kernels_warm_up();
 bool tiled_shape_available(int elem, int tx, int ty, int vx, int vy, bool general = false);
 // Shapes the batched engine's persistent kernel is instantiated for (batch.hip).
 bool batch_tiled_available(int elem, int tx, int ty, int vx, int vy, bool general = false);
-bool batch_copy_available(int word, int tx);
 bool batch_packed_available(int elem, int nreg);
-bool copy_shape_available(int word, int tx);
 int packed_max_nreg(int elem);
 bool packed_nreg_available(int elem, int nreg);
 

@@ -66,18 +66,14 @@ __global__ __launch_bounds__(256) void k_tiled(TiledArgs a, const void* __restri
   }
 }
 
-template <int W, int TX, int NP>
+// One item per workgroup.
+template <int B>
 __global__ __launch_bounds__(256) void k_copy(CopyArgs a, const void* __restrict__ in,
                                               void* __restrict__ out) {
-  using Ops = CopyOps<W, TX, NP>;
-  using V = typename Ops::V;
-  const V* src = static_cast<const V*>(in);
-  V* dst = static_cast<V*>(out);
-  const uint32_t w0 = a.xcds > 1 ? (uint32_t)xcd_logical((int)blockIdx.x, (int)gridDim.x, a.xcds) : blockIdx.x;
-  for (uint32_t w = w0; w < (uint32_t)a.items; w += gridDim.x) {
-    const TileCtx c = Ops::item(a, w);
-    Ops::run(a, c, threadIdx.x, src, dst);
-  }
+  using Ops = CopyOps<B>;
+  using E = typename Ops::E;
+  const uint32_t w = a.xcds > 1 ? (uint32_t)xcd_logical((int)blockIdx.x, (int)gridDim.x, a.xcds) : blockIdx.x;
+  Ops::run(a, w, threadIdx.x, static_cast<const E*>(in), static_cast<E*>(out));
 }
 
 template <int B, int NREG>
@@ -195,6 +191,13 @@ void kernels_warm_up() {
 
 thread_local ReplayObserver* g_replay_observer = nullptr;
 
+// Items of a TiledCopy launch: an output that does not start on a line
+// shifts the words back to the line before it.
+static int copy_items(const Candidate& c, const void* out) {
+  const long long phase = (long long)((uintptr_t)out & 127) / c.elem;
+  return (int)((c.copy.n + phase + c.copy.per - 1) / c.copy.per);
+}
+
 static inline void replay_at(long long item, int t) {
   if (g_replay_observer) g_replay_observer->at(item, t);
 }
@@ -221,18 +224,16 @@ static void replay_tiled(const Candidate& c, const void* in, void* out) {
   }
 }
 
-template <int W, int TX, int NP>
+template <int B>
 static void replay_copy(const Candidate& c, const void* in, void* out) {
-  using Ops = CopyOps<W, TX, NP>;
-  using V = typename Ops::V;
-  const CopyArgs& a = c.copy;
-  for (uint32_t w = 0; w < (uint32_t)a.items; w++) {
-    const TileCtx ctx = Ops::item(a, w);
+  using Ops = CopyOps<B>;
+  using E = typename Ops::E;
+  const int items = copy_items(c, out);
+  for (int w = 0; w < items; w++)
     for (int t = 0; t < Ops::NT; t++) {
       replay_at(w, t);
-      Ops::run(a, ctx, t, static_cast<const V*>(in), static_cast<V*>(out));
+      Ops::run(c.copy, (uint32_t)w, t, static_cast<const E*>(in), static_cast<E*>(out));
     }
-  }
 }
 
 template <int B, int NREG>
@@ -321,7 +322,7 @@ struct TiledEntry {
   void (*replay)(const Candidate&, const void*, void*);
 };
 struct CopyEntry {
-  int w, tx, np;
+  int b;
   const void* kernel;
   void (*replay)(const Candidate&, const void*, void*);
 };
@@ -364,11 +365,9 @@ static const TiledEntry kTiledTable[] = {
     LRT_TILED_G(16, 16, 16, 1, 1, true) LRT_TILED_G(16, 32, 32, 1, 1, true)
 };
 
-#define LRT_COPY(W, TX) \
-  {W, TX, 4, reinterpret_cast<const void*>(&k_copy<W, TX, 4>), &replay_copy<W, TX, 4>},
-#define LRT_COPY_W(W) LRT_COPY(W, 4) LRT_COPY(W, 8) LRT_COPY(W, 16) LRT_COPY(W, 32) LRT_COPY(W, 64)
+#define LRT_COPY(B) {B, reinterpret_cast<const void*>(&k_copy<B>), &replay_copy<B>},
 
-static const CopyEntry kCopyTable[] = {LRT_COPY_W(4) LRT_COPY_W(8) LRT_COPY_W(16)};
+static const CopyEntry kCopyTable[] = {LRT_COPY(4) LRT_COPY(8) LRT_COPY(16)};
 
 #define LRT_PACKED(B, N) {B, N, reinterpret_cast<const void*>(&k_packed<B, N>), &replay_packed<B, N>},
 #define LRT_PACKED_8(B) \
@@ -391,7 +390,7 @@ static const TiledEntry* find_tiled(const Candidate& c) {
 }
 static const CopyEntry* find_copy(const Candidate& c) {
   for (const auto& e : kCopyTable)
-    if (e.w == c.word && e.tx == c.copy_tx) return &e;
+    if (e.b == c.elem) return &e;
   return nullptr;
 }
 static const PackedEntry* find_packed(const Candidate& c) {
@@ -403,11 +402,6 @@ static const PackedEntry* find_packed(const Candidate& c) {
 bool tiled_shape_available(int elem, int tx, int ty, int vx, int vy, bool general) {
   for (const auto& e : kTiledTable)
     if (e.b == elem && e.tx == tx && e.ty == ty && e.vx == vx && e.vy == vy && e.general == general) return true;
-  return false;
-}
-bool copy_shape_available(int word, int tx) {
-  for (const auto& e : kCopyTable)
-    if (e.w == word && e.tx == tx) return true;
   return false;
 }
 int packed_max_nreg(int elem) {
@@ -448,7 +442,7 @@ hipError_t launch_candidate(const Candidate& c, const void* in, void* out, hipSt
   }
   const void* k = kernel_of(c);
   if (!k) return hipErrorInvalidDeviceFunction;
-  dim3 grid(c.grid_x, c.grid_y, 1);
+  dim3 grid(c.method == kTiledCopy ? copy_items(c, out) : c.grid_x, c.grid_y, 1);
   dim3 block(c.block, 1, 1);
   void* args[3];
   switch (c.method) {

@@ -67,11 +67,13 @@ void output_strides(const Problem& p, long long* s) {
   }
 }
 
-int pow2ceil(int x) {
-  int p = 1;
-  while (p < x) p <<= 1;
-  return p;
-}
+// Rows of at least this many bytes that stay rows (perm[0] == 0) are copied by
+// TiledCopy, not by a Packed plan (which librettPlanMeasure still times). On
+// MI355X, best TiledCopy against best Packed plan of ~200 MiB f32 / f64 / c128 problems: rows of 16 B
+// 148 / 146 / - against 142 / 142 / - us; of 32 B 103 / 103 / 89 against
+// 109 / 107 / 98; of 64 B 79 / 79 / 78 against 88 / 90 / 86; of 1040 B
+// 73 / 74 / 72 against 105 / 100 / 89.
+constexpr int kCopyOnlyRow = 32;
 
 // Outer map over the input dims for which `skip[d]` is false, in input order.
 void build_outer(const Problem& p, const bool* skip, const long long* cin, const long long* cout,
@@ -340,7 +342,7 @@ std::string Candidate::describe() const {
                  tile_order(*this) ? " xcd" : "");
       break;
     case kTiledCopy:
-      snprintf(buf, sizeof(buf), "%s word %dB tx %d grid %d%s", n, word, copy_tx, grid_x,
+      snprintf(buf, sizeof(buf), "%s word %dB rows %d grid %d%s", n, word, copy.X, grid_x,
                tile_order(*this) ? " xcd" : "");
       break;
     case kPacked:
@@ -525,62 +527,59 @@ void add_tiled(const Problem& r, const DeviceInfo& dev, std::vector<Candidate>& 
   }
 }
 
+// Non-temporal loads for an input of `bytes` bytes that a kernel reads in
+// whole lines, once, or nearly so: copies between rotating buffers on MI355X gain from
+// 96 MiB on (33.8 -> 32.2 us at 96 MiB, 85.5 -> 83.1 us at 256 MiB), where
+// input and output no longer fit the 256 MiB Infinity Cache together; below,
+// the input may still be there from whoever wrote it, and streaming it costs
+// (19.9 -> 22.0 us at 64 MiB).
+int stream_input(long long bytes) { return bytes >= (96LL << 20) ? 1 : 0; }
+
+// Words of 16 bytes over the output in order; one plan (and its twin in the
+// other work order).
 void add_tiled_copy(const Problem& r, const DeviceInfo& dev, std::vector<Candidate>& out) {
   long long cin[kMaxRank], cout[kMaxRank];
   input_strides(r, cin);
   output_strides(r, cout);
   const int B = r.elem;
-  const long long rowbytes = (long long)r.dim[0] * B;
-  int W = 4;
-  if (rowbytes % 16 == 0) W = 16;
-  else if (rowbytes % 8 == 0) W = 8;
-  const int X = (int)(rowbytes / W);
-  const int ydim = r.perm[1];
-  bool skip[kMaxRank] = {false};
-  skip[0] = true;
-  skip[ydim] = true;
-  OuterMap outer;
-  int vol_outer;
-  build_outer(r, skip, cin, cout, B, W, outer, vol_outer);
-  int txs[2] = {std::min(64, std::max(4, pow2ceil(X))), 64};
-  if (dev.batch_mode) {
-    txs[0] = X <= 16 ? 16 : 64;
-    txs[1] = 64;
+  Candidate c;
+  c.method = kTiledCopy;
+  c.elem = B;
+  c.source = "reduced";
+  c.word = 16;
+  c.copy_tx = 64;  // words a wave moves at a time
+  CopyArgs& a = c.copy;
+  a.n = (int)r.vol;
+  a.X = r.dim[0];
+  a.row_div = make_fastdiv((uint32_t)r.dim[0]);
+  a.rows.n = r.rank - 1;
+  for (int k = 0; k < kMaxRank; k++) {
+    const int d = k + 1 < r.rank ? r.perm[k + 1] : -1;
+    a.rows.div[k] = make_fastdiv(d >= 0 ? (uint32_t)r.dim[d] : 1u);
+    a.rows.ct_in[k] = d >= 0 ? (int)cin[d] : 0;
+    a.rows.ct_out[k] = d >= 0 ? (int)cout[d] : 0;
   }
-  for (int k = 0; k < 2; k++) {
-    if (k == 1 && txs[1] == txs[0]) continue;
-    Candidate c;
-    c.method = kTiledCopy;
-    c.elem = B;
-    c.source = "reduced";
-    c.word = W;
-    c.copy_tx = txs[k];
-    if (dev.batch_mode ? !batch_copy_available(W, c.copy_tx) : !copy_shape_available(W, c.copy_tx)) continue;
-    CopyArgs& a = c.copy;
-    a.X = X;
-    a.Y = r.dim[ydim];
-    a.in_ys = (int)(cin[ydim] * B / W);
-    a.out_ys = (int)(cout[ydim] * B / W);
-    const int ty = (256 / c.copy_tx) * 4;
-    a.ntx = (X + c.copy_tx - 1) / c.copy_tx;
-    const int nty = (a.Y + ty - 1) / ty;
-    a.ntiles = a.ntx * nty;
-    a.ntx_div = make_fastdiv((uint32_t)a.ntx);
-    a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
-    a.items = (int)std::min<long long>((long long)a.ntiles * vol_outer, 0x7fffffffLL);
-    a.xcds = 1;
-    a.outer = outer;
-    c.block = 256;
-    c.lds_bytes = 0;
-    c.grid_x = std::max(1, std::min(a.items, dev.cu_count * grid_per_cu()));
-    c.bytes = 2 * r.vol * B;
-    c.split.sizeMm = 1;
-    c.split.sizeMk = 2;
-    c.split.volMm = r.dim[0];
-    c.split.volMkBar = a.Y;
-    c.split.volMbar = vol_outer;
-    out.push_back(c);
-  }
+  a.per = 256 * (16 / B);
+  // The batched engine learns its buffers after planning: its items cover
+  // the most that an output off its line can need.
+  const long long span = r.vol + (dev.batch_mode ? 128 / B - 1 : 0);
+  a.items = (int)((span + a.per - 1) / a.per);
+  a.xcds = 1;
+  // Rows that end inside lines are read partly by two items; streaming pays
+  // from rows of 2 KiB on (f64, 200 MiB: 72.8 -> 69.9 us with 4104-byte rows,
+  // 73.1 -> 72.8 with 2056, but 73.5 -> 78.7 with 1032 and 79 -> 82 with 520).
+  const long long row = (long long)r.dim[0] * B;
+  a.stream_in = !dev.batch_mode && (row % 128 == 0 || row >= 2048) ? stream_input(r.vol * B) : 0;
+  c.block = 256;
+  c.lds_bytes = 0;
+  c.grid_x = a.items;
+  c.bytes = 2 * r.vol * B;
+  c.split.sizeMm = 1;
+  c.split.sizeMk = 2;
+  c.split.volMm = r.dim[0];
+  c.split.volMkBar = r.dim[r.perm[1]];
+  c.split.volMbar = (int)(r.vol / r.dim[0] / r.dim[r.perm[1]]);
+  out.push_back(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -971,26 +970,29 @@ void model_tiled(Candidate& c) {
 
 void model_copy(Candidate& c) {
   const CopyArgs& a = c.copy;
-  const int Wb = c.word;
-  const int ty_tile = (256 / c.copy_tx) * 4;
-  double R = 0, W = 0, P = 0, TR = 0, TW = 0;
+  const int B = c.elem;
+  const long long word = 16 / B;
+  double R = 0, W = 0, TR = 0, TW = 0, P = 0;
   std::vector<long long> ws = sample_indices(a.items, 24);
   std::vector<Run> rin, rout;
   for (long long w : ws) {
-    uint32_t mb = (uint32_t)(w / a.ntiles);
-    int tile = (int)(w % a.ntiles);
-    int x0 = (tile % a.ntx) * c.copy_tx, y0 = (tile / a.ntx) * ty_tile;
-    int oi, oo;
-    outer_offsets(a.outer, mb, oi, oo);
-    int tx = std::min(c.copy_tx, a.X - x0), ty = std::min(ty_tile, a.Y - y0);
+    const long long e0 = w * a.per, e1 = std::min<long long>(a.n, e0 + a.per);
     rin.clear();
     rout.clear();
-    for (int y = 0; y < ty; y++) {
-      rin.push_back({(oi + x0 + (long long)(y0 + y) * a.in_ys) * Wb, (long long)tx * Wb});
-      rout.push_back({(oo + x0 + (long long)(y0 + y) * a.out_ys) * Wb, (long long)tx * Wb});
+    // Row pieces of the item, and for the transactions the pieces of each
+    // wave's words.
+    for (long long v0 = e0; v0 < e1; v0 += 64 * word) {
+      const long long v1 = std::min(e1, v0 + 64 * word);
+      for (long long e = v0; e < v1;) {
+        const long long row = e / a.X, k = e - row * a.X, m = std::min<long long>(a.X - k, v1 - e);
+        const long long src = copy_row_offset(a.rows, (uint32_t)row) + k;
+        rin.push_back({src * B, m * B});
+        TR += tran(src * B, m * B);
+        e += m;
+      }
+      TW += tran(v0 * B, (v1 - v0) * B);
     }
-    for (const Run& r : rin) TR += tran(r.s, r.n);
-    for (const Run& r : rout) TW += tran(r.s, r.n);
+    rout.push_back({e0 * B, (e1 - e0) * B});
     double l, p;
     line_stats(rin, l, p);
     R += l;
@@ -1404,10 +1406,16 @@ std::vector<Candidate> make_candidates(const Problem& full, const DeviceInfo& de
   return ok;
 }
 
+bool copy_beats(const std::vector<Candidate>& cands, const Candidate& c) {
+  return c.method != kTiledCopy && cands[0].method == kTiledCopy &&
+         (long long)cands[0].copy.X * cands[0].elem >= kCopyOnlyRow;
+}
+
 int choose_by_model(const std::vector<Candidate>& cands) {
   int best = -1;
   for (int i = 0; i < (int)cands.size(); i++) {
     if (cands[i].method == kTrivial) return i;
+    if (copy_beats(cands, cands[i])) continue;
     if (best < 0 || cands[i].model.predicted_s < cands[best].model.predicted_s) best = i;
   }
   return best;
@@ -1426,45 +1434,11 @@ int needed_alignment(const Candidate& c) {
   switch (c.method) {
     case kTiled:
       return c.elem * std::max(c.vec_x, c.vec_y);
-    case kTiledCopy:
-      return c.word;
     default:
       return c.elem;
   }
 }
 
-Candidate copy_fallback(const Candidate& c) {
-  // TiledCopy moves W-byte words; for pointers aligned only to the element,
-  // rebuild the arguments with W = element size.
-  Candidate f = c;
-  if (c.method != kTiledCopy || c.word == c.elem) return f;
-  const int k = c.word / c.elem;
-  CopyArgs& a = f.copy;
-  a.X *= k;
-  a.in_ys *= k;
-  a.out_ys *= k;
-  for (int r = 0; r < a.outer.n; r++) {
-    a.outer.ct_in[r] *= k;
-    a.outer.ct_out[r] *= k;
-  }
-  f.word = c.elem;
-  f.copy_tx = 64;
-  const int ty = (256 / f.copy_tx) * 4;
-  a.ntx = (a.X + f.copy_tx - 1) / f.copy_tx;
-  const int nty = (a.Y + ty - 1) / ty;
-  const long long vol_outer = c.copy.items / std::max(1, c.copy.ntiles);
-  a.ntiles = a.ntx * nty;
-  a.ntx_div = make_fastdiv((uint32_t)a.ntx);
-  a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
-  a.items = (int)(a.ntiles * vol_outer);
-  f.grid_x = std::max(1, std::min(a.items, 16384));
-  return f;
-}
-
-Candidate unaligned_fallback(const Candidate& c) {
-  if (c.method == kTiled) return scalar_fallback(c);
-  if (c.method == kTiledCopy) return copy_fallback(c);
-  return c;
-}
+Candidate unaligned_fallback(const Candidate& c) { return c.method == kTiled ? scalar_fallback(c) : c; }
 
 }  // namespace lrt

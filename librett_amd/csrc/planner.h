@@ -134,6 +134,11 @@ void model_times(Candidate& c, const DeviceInfo& dev);
 // inflight_half, round_latency, launch); entries <= 0 keep their value.
 void set_model_constants(const double* v, int n);
 
+// Whether candidate c need not be looked at because TiledCopy, which is among
+// `cands`, is faster: c is a Packed plan of a problem whose rows stay rows
+// (perm[0] == 0) and are long enough.
+bool copy_beats(const std::vector<Candidate>& cands, const Candidate& c);
+
 // Index of the candidate with the smallest modelled time (Trivial wins, as
 // in operator> of src/plan.cpp:721-768).
 int choose_by_model(const std::vector<Candidate>& cands);
@@ -149,13 +154,39 @@ Candidate scalar_fallback(const Candidate& c);
 // Pointer alignment a candidate's vector accesses need.
 int needed_alignment(const Candidate& c);
 
-// Variant of a TiledCopy candidate that moves element-sized words.
-Candidate copy_fallback(const Candidate& c);
-
 // The candidate to launch when the pointers are not aligned to
-// needed_alignment(c): scalar Tiled lanes, element-sized TiledCopy words,
-// or c itself (Packed and Trivial need only element alignment).
+// needed_alignment(c): scalar Tiled lanes, or c itself (the other methods
+// need only element alignment).
 Candidate unaligned_fallback(const Candidate& c);
+
+// A host buffer of n bytes between guard bands, for replays: the data starts
+// at the same place within a 128-byte line as `like` does (the kernels'
+// stores depend on it), rounded down to a multiple of `align`.
+class GuardedBuffer {
+ public:
+  GuardedBuffer(size_t n, const void* like, int align, unsigned char fill)
+      : n_(n), fill_(fill), bytes_(n + 2 * kGuard + 256, fill) {
+    const size_t phase = ((uintptr_t)like & 127) / (size_t)align * (size_t)align;
+    unsigned char* p = bytes_.data() + kGuard;
+    data_ = p + ((128 - ((uintptr_t)p & 127)) & 127) + phase;
+  }
+  unsigned char* data() { return data_; }
+  // Whether the bytes around the data still hold the fill value.
+  bool intact() const {
+    for (const unsigned char* p = bytes_.data(); p < data_; p++)
+      if (*p != fill_) return false;
+    for (const unsigned char* p = data_ + n_; p < bytes_.data() + bytes_.size(); p++)
+      if (*p != fill_) return false;
+    return true;
+  }
+
+ private:
+  static constexpr size_t kGuard = 1 << 16;
+  size_t n_;
+  unsigned char fill_;
+  std::vector<unsigned char> bytes_;
+  unsigned char* data_;
+};
 
 // Contiguous runs (start offset, length in elements) of one staged shape
 // walked in LDS order (input side) or output order (output side).

@@ -294,6 +294,7 @@ int selector_choose(const std::vector<Candidate>& cands, const Problem& full, in
   int best = -1;
   for (int i = 0; i < n; i++) {
     if (!std::isfinite(score[i])) return -1;
+    if (copy_beats(cands, cands[i])) continue;
     if (best < 0 || score[i] < score[best]) best = i;
   }
   // The analytic model's choice stands unless the selector predicts its own

@@ -1,0 +1,58 @@
+"""Kernels at the sizes where they can go wrong, on the GPU: rows and tiles
+cut by the tensor's end, outputs that start anywhere in a cache line, the
+smallest and a large volume. Every candidate plan, bit for bit against the
+oracle, with guard bytes around the output."""
+import numpy as np
+import pytest
+
+import librett_amd as L
+import oracle
+from librett_amd import data, hip
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 256
+
+
+def check(stream, dim, perm, elem, offsets, methods=None, only=None):
+    """Every candidate of `methods` on buffers `offset` elements into an allocation."""
+    n = int(np.prod(dim))
+    x = data.uniform(n, elem, 41)
+    ref = oracle.transpose(dim, perm, elem, x).view(np.uint8)
+    room = (max(offsets) + n) * elem + 2 * GUARD
+    a, b = hip.DeviceBuffer(room), hip.DeviceBuffer(room)
+    ran = 0
+    try:
+        for i, c in enumerate(L.candidates(dim, perm, elem)):
+            if methods and c["method"] not in methods or only and only not in c["desc"]:
+                continue
+            r, h = L.plan_candidate(len(dim), dim, perm, elem, stream, i)
+            assert r == L.LIBRETT_SUCCESS, c["desc"]
+            for off in offsets:
+                print("case:", dim, perm, elem, "offset", off, c["desc"], flush=True)
+                at = GUARD + off * elem
+                hip.htod(a.ptr + at, x)
+                hip.memset(b.ptr, 0xEE, room)
+                assert L.librettExecute(h, a.ptr + at, b.ptr + at) == L.LIBRETT_SUCCESS
+                hip.stream_sync(stream)
+                got = np.empty(room, dtype=np.uint8)
+                hip.dtoh(got, b.ptr)
+                assert np.array_equal(got[at:at + n * elem], ref), (dim, perm, elem, off, c["desc"])
+                assert np.all(got[:at] == 0xEE) and np.all(got[at + n * elem:] == 0xEE), (off, c["desc"])
+                ran += 1
+            L.librettDestroy(h)
+    finally:
+        a.free()
+        b.free()
+    return ran
+
+
+# Rows shorter than a word, of one word, odd, longer than a workgroup's
+# block; volumes that end inside a word; ranks that need several digits.
+@pytest.mark.parametrize("elem", [4, 8, 16])
+@pytest.mark.parametrize("dim,perm", [
+    ([2, 3, 5], [0, 2, 1]), ([3, 7, 11, 2], [0, 3, 2, 1]), ([4, 9, 8], [0, 2, 1]), ([33, 5, 7, 4, 3], [0, 4, 2, 3, 1]),
+    ([1031, 3, 5], [0, 2, 1]), ([4097, 2, 3], [0, 2, 1]), ([2, 2, 2, 3, 2, 5, 2, 3], [0, 7, 2, 5, 4, 3, 6, 1]),
+])
+def test_copy_rows(gpu_stream, dim, perm, elem):
+    assert check(gpu_stream, dim, perm, elem, [0, 1, 5, 128 // elem - 1], methods=(L.TILED_COPY,)) >= 4
