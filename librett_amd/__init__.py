@@ -395,7 +395,7 @@ def _ptrs(v):
 
 
 class Batch:
-    """Many transposes in one persistent launch (extension of the API).
+    """Many transposes in one launch (extension of the API).
 
     ``problems`` is a list of (dims, perm, elem). ``tune`` = 0 uses the cost
     model, k > 0 times the model's k best batch plans of each problem."""

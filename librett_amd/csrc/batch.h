@@ -1,13 +1,12 @@
-// Batched engine: many independent transposes in one persistent launch.
+// Batched engine: many independent transposes in one launch.
 //
 // Every problem gets a plan from the batch-mode planner (256-thread
 // workgroups, small LDS, a fixed set of kernel shapes) and a descriptor in
 // one device arena. The work of all problems is a single index space of
 // units (tiles, row tiles, or a few staged rounds), laid out problem after
-// problem; workgroup g of the persistent kernel takes units g, g + G,
-// g + 2G, ... so neighbouring units of one problem run at the same time on
-// different CUs, and no counters or atomics are needed (the launch can be
-// replayed from a HIP graph as is).
+// problem, one workgroup per unit: neighbouring units of one problem run at
+// the same time on different CUs, and no counters or atomics are needed (the
+// launch can be replayed from a HIP graph as is).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -19,7 +18,7 @@
 namespace lrt {
 
 struct BatchDesc {
-  int variant;       // index into the persistent kernel's shape table
+  int variant;       // index into the kernel's shape table
   int units;         // work units of this problem
   int rounds;        // items per unit (at most)
   int items;         // tiles (Tiled, TiledCopy) or outer indices (Packed) of the problem
@@ -48,13 +47,13 @@ bool batch_describe(const Candidate& c, BatchDesc& d);
 // (at least one item per unit).
 void batch_regroup(BatchDesc& d, long long unit_bytes);
 
-// Unit size for a batch of `total_bytes` algorithmic bytes run by `grid`
-// workgroups: about 32 units per workgroup, between 16 KiB and
+// Unit size for a batch of `total_bytes` algorithmic bytes on a device that
+// runs `grid` workgroups at a time: about 32 units per workgroup, between 16 KiB and
 // kBatchUnitBytes (environment overrides: LIBRETT_BATCH_UNIT_KB,
 // LIBRETT_BATCH_UNITS_PER_WG).
 long long batch_unit_bytes(long long total_bytes, int grid);
 
-// The persistent kernel comes in one instantiation per family of shapes, so
+// The kernel comes in one instantiation per family of shapes, so
 // that each holds only the registers its own shapes need.
 enum BatchFamily : int { kFamTiled = 0, kFamCopy = 1, kFamPacked = 2, kFamTiledG = 3 };
 constexpr int kBatchFamilies = 4;
@@ -77,15 +76,13 @@ struct BatchLayout {
 // original index of the k-th ordered descriptor.
 void batch_layout(std::vector<BatchDesc>& descs, BatchLayout& layout, std::vector<int>* order);
 
-// Launches family `fam`'s persistent kernel over `total` units of `nprob`
-// descriptors (`start`: first unit of each, then `total`), with at most
-// `grid` workgroups.
-hipError_t launch_batch(int fam, const BatchDesc* d_descs, const int* d_start, int nprob, int total, int grid,
+// Launches family `fam`'s kernel over `total` units of `nprob`
+// descriptors (`start`: first unit of each, then `total`).
+hipError_t launch_batch(int fam, const BatchDesc* d_descs, const int* d_start, int nprob, int total,
                         hipStream_t stream);
 
-// One launch per non-empty family, in family order on one stream; grid[f]
-// caps family f's workgroups.
-hipError_t launch_batch_all(const BatchDesc* d_descs, const int* d_start, const BatchLayout& layout, const int* grid,
+// One launch per non-empty family, in family order on one stream.
+hipError_t launch_batch_all(const BatchDesc* d_descs, const int* d_start, const BatchLayout& layout,
                             hipStream_t stream);
 
 // Resident workgroups per CU of family `fam`'s kernel (runtime query).
@@ -104,7 +101,7 @@ int batch_alignment(const Problem& p, const Candidate& c);
 // Batch-mode candidates of a problem, best modelled streaming cost first.
 std::vector<Candidate> batch_candidates(const Problem& p, const DeviceInfo& dev);
 
-// Host replay of the persistent kernel (descriptors hold host pointers).
+// Host replay of the kernel (descriptors hold host pointers).
 // Returns false if a unit wrote past the kernel's LDS.
 bool replay_batch(const BatchDesc* descs, const int* start, int nprob, int total, int grid);
 

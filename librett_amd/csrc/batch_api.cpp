@@ -85,8 +85,7 @@ struct BatchObj {
   std::vector<long long> byte_offset;   // offset of the descriptor's data in its problem
   BatchLayout layout;                   // descriptors grouped by kernel family
   long long total = 0;                  // units of all families
-  int grid[kBatchFamilies] = {}; // workgroups of each family's launch
-  int grid_max = 0;
+  int grid_max = 0;  // workgroups resident at a time, of the family that holds most
   long long unit_bytes = kBatchUnitBytes;
   BatchDesc* d_descs = nullptr;
   int* d_start = nullptr;
@@ -123,15 +122,14 @@ std::string problem_key(const Problem& p) {
 }
 
 
-// Times candidate c of problem p inside the persistent kernel, on enough
+// Times candidate c of problem p inside its family's kernel, on enough
 // clones of the problem to fill the device (scratch buffers `a`, `b`).
 double time_in_batch(const Candidate& c, const Problem& p, void* a, void* b, size_t scratch, hipStream_t stream,
-                     BatchDesc* d_desc, int* d_start, int max_clones, const int* grids, long long unit_bytes) {
+                     BatchDesc* d_desc, int* d_start, int max_clones, long long unit_bytes) {
   BatchDesc d;
   if (!batch_describe(c, d)) return -1;
   batch_regroup(d, unit_bytes);
   const int fam = batch_family(d.variant);
-  const int grid = grids[fam];
   const size_t bytes = (size_t)p.vol * p.elem;
   const size_t span = (bytes + 255) / 256 * 256;
   if (span > scratch) return -1;  // every clone must lie inside the scratch buffers
@@ -155,11 +153,11 @@ double time_in_batch(const Candidate& c, const Problem& p, void* a, void* b, siz
     (void)hipEventDestroy(e0);
     return -1;
   }
-  bool ok = launch_batch(fam, d_desc, d_start, clones, st[clones], grid, stream) == hipSuccess;
+  bool ok = launch_batch(fam, d_desc, d_start, clones, st[clones], stream) == hipSuccess;
   float best = 1e30f;
   for (int r = 0; ok && r < 2; r++) {
     ok = hipEventRecord(e0, stream) == hipSuccess &&
-         launch_batch(fam, d_desc, d_start, clones, st[clones], grid, stream) == hipSuccess &&
+         launch_batch(fam, d_desc, d_start, clones, st[clones], stream) == hipSuccess &&
          hipEventRecord(e1, stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
     float ms = 0;
     if (ok && hipEventElapsedTime(&ms, e0, e1) == hipSuccess) best = std::min(best, ms);
@@ -189,16 +187,15 @@ int build_batch(BatchObj& B, const DeviceInfo& dev, int tune) {
   B.grid_max = 0;
   for (int f = 0; f < kBatchFamilies; f++) {
     const int occ = std::max(1, dev.has_gpu ? batch_occupancy(f) : 4);
-    B.grid[f] = dev.cu_count * occ;
-    B.grid_max = std::max(B.grid_max, B.grid[f]);
+    B.grid_max = std::max(B.grid_max, dev.cu_count * occ);
   }
   long long total_bytes = 0;
   for (const Problem& p : B.probs) total_bytes += 2LL * p.vol * p.elem;
   B.unit_bytes = batch_unit_bytes(total_bytes, B.grid_max);
 
   if (tune && dev.has_gpu) {
-    // Autotuner: time the top candidates of each distinct problem inside the
-    // persistent kernel on clones of the problem, keep the fastest, and
+    // Autotuner: time the top candidates of each distinct problem inside their
+    // family's kernel on clones of the problem, keep the fastest, and
     // remember it across batches.
     const double t1 = now_s();
     // Scratch for the clones: at least 256 MiB, and room for the largest
@@ -227,7 +224,7 @@ int build_batch(BatchObj& B, const DeviceInfo& dev, int tune) {
       int bi = 0;
       for (int k = 0; k < (int)ranked[i].size() && k < topk; k++) {
         const double t = time_in_batch(ranked[i][k], B.probs[i], a, b, scratch, B.stream, d_desc, d_start,
-                                       max_clones, B.grid, B.unit_bytes);
+                                       max_clones, B.unit_bytes);
         if (t > 0 && t < best) {
           best = t;
           bi = k;
@@ -468,7 +465,7 @@ int librett_c_batch_execute(unsigned int handle, int use_graph) {
   if (!B) return LIBRETT_C_INVALID_PLAN;
   if (!B->buffers_set) return LIBRETT_C_INVALID_PARAMETER;
   if (!use_graph) {
-    return launch_batch_all(B->d_descs, B->d_start, B->layout, B->grid, B->stream) == hipSuccess
+    return launch_batch_all(B->d_descs, B->d_start, B->layout, B->stream) == hipSuccess
                ? LIBRETT_C_SUCCESS
                : LIBRETT_C_INTERNAL_ERROR;
   }
@@ -477,7 +474,7 @@ int librett_c_batch_execute(unsigned int handle, int use_graph) {
       (void)hipGetLastError();
       return LIBRETT_C_INTERNAL_ERROR;
     }
-    const hipError_t le = launch_batch_all(B->d_descs, B->d_start, B->layout, B->grid, B->stream);
+    const hipError_t le = launch_batch_all(B->d_descs, B->d_start, B->layout, B->stream);
     hipGraph_t g = nullptr;
     const hipError_t ce = hipStreamEndCapture(B->stream, &g);
     if (le != hipSuccess || ce != hipSuccess || !g) {

@@ -32,7 +32,7 @@ void kernels_warm_up();
 
 // general: a kernel for planes whose x or y is a group of several dims.
 bool tiled_shape_available(int elem, int tx, int ty, int vx, int vy, bool general = false);
-// Shapes the batched engine's persistent kernel is instantiated for (batch.hip).
+// Shapes the batched engine's kernel is instantiated for (batch.hip).
 bool batch_tiled_available(int elem, int tx, int ty, int vx, int vy, bool general = false);
 bool batch_packed_available(int elem, int nreg);
 int packed_max_nreg(int elem);

@@ -29,12 +29,12 @@ struct DeviceInfo {
   double hbm_bytes_per_s = 8.0e12;   // published MI355X HBM3E peak
   double l2_bytes = 32.0 * 1024 * 1024;  // L2 of all XCDs (8 x 4 MiB on MI355X)
   int has_gpu = 0;                   // occupancy may be queried from the runtime
-  // Batched engine: candidates must run in its persistent kernel (256-thread
+  // Batched engine: candidates must run in its kernel (256-thread
   // workgroups, at most kBatchLds bytes of LDS, its instantiated shapes).
   int batch_mode = 0;
 };
 
-// LDS of the batched engine's persistent kernel.
+// LDS of the batched engine's kernel.
 constexpr int kBatchLds = 17 * 1024;
 
 // A transpose problem: column-major input dims, output dims dim[perm[i]].

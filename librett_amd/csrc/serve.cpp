@@ -4,7 +4,7 @@
 // thread. One dispatcher thread owns a few launch slots, each a stream with
 // its own pinned staging and device descriptor area. Whenever a slot is
 // free, every queued request (up to a cap) becomes one micro-batch: its
-// descriptors are copied to the device and the batched engine's persistent
+// descriptors are copied to the device and the batched engine's
 // kernel runs them; micro-batches on different slots overlap on the device,
 // so requests that arrive while others run are admitted as soon as a slot
 // frees up. Completion is observed with one event per micro-batch.
@@ -130,8 +130,7 @@ class Server {
     dev_.has_gpu = 1;
     grid_max_ = 0;
     for (int f = 0; f < kBatchFamilies; f++) {
-      grid_[f] = dev_.cu_count * std::max(1, batch_occupancy(f));
-      grid_max_ = std::max(grid_max_, grid_[f]);
+      grid_max_ = std::max(grid_max_, dev_.cu_count * std::max(1, batch_occupancy(f)));
     }
     max_batch_ = std::max(1, max_batch);
     if (!arena_.init(arena_bytes)) return LIBRETT_C_INTERNAL_ERROR;
@@ -369,7 +368,7 @@ class Server {
                hipSuccess &&
            hipMemcpyAsync(s.d_start, s.h_start, L.start.size() * sizeof(int), hipMemcpyHostToDevice, s.stream) ==
                hipSuccess &&
-           launch_batch_all(s.d_desc, s.d_start, L, grid_, s.stream) == hipSuccess &&
+           launch_batch_all(s.d_desc, s.d_start, L, s.stream) == hipSuccess &&
            hipEventRecord(s.done, s.stream) == hipSuccess;
       if (!ok) (void)hipGetLastError();
     }
@@ -462,7 +461,6 @@ class Server {
 
   int device_ = 0;
   DeviceInfo dev_;
-  int grid_[kBatchFamilies] = {};
   int grid_max_ = 0;
   int max_batch_ = 64;
   Arena arena_;
