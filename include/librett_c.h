@@ -319,6 +319,15 @@ void librett_c_mlp_sizes(int* nfeat, int* hidden, int* nparams);
 int librett_c_measure_candidates(int rank, const int* dim, const int* permutation, size_t sizeofType, void* stream,
                                  const void* idata, void* odata, double* times, int max, int* count);
 
+/* Times every candidate in a stream of launches, as a program that runs a plan
+ * again and again sees it: `sets` buffer pairs lie `stride` bytes apart from
+ * idata and odata (a multiple of 128; `sets` of them must fit) and are used
+ * in turn. Seconds per launch; candidates well behind the fastest before them
+ * are timed briefly. */
+int librett_c_measure_steady(int rank, const int* dim, const int* permutation, size_t sizeofType, void* stream,
+                             const void* idata, void* odata, size_t stride, int sets, double* times, int max,
+                             int* count);
+
 /* Raw features (count x LIBRETT_C_SELECTOR_FEATURES floats, candidate order
  * as above) and the analytic model's choice. `device` NULL: the current GPU;
  * otherwise host-only planning for the described device. */

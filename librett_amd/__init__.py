@@ -76,7 +76,7 @@ EXPORTED = [
     "librett_c_server_create", "librett_c_server_alloc", "librett_c_server_free", "librett_c_server_submit",
     "librett_c_server_wait", "librett_c_server_drain", "librett_c_server_stats_get", "librett_c_server_reset_stats",
     "librett_c_server_destroy", "librett_c_server_run_poisson",
-    "librett_c_mlp_sizes", "librett_c_measure_candidates", "librett_c_selector_features", "librett_c_selector_choose",
+    "librett_c_mlp_sizes", "librett_c_measure_candidates", "librett_c_measure_steady", "librett_c_selector_features", "librett_c_selector_choose",
     "librett_c_selector_set", "librett_c_selector_load", "librett_c_selector_generation", "librett_c_mlp_forward",
     "librett_c_mlp_grad", "librett_c_mlp_adam", "librett_c_mlp_train", "librett_c_mlp_host_forward",
     "librett_c_mlp_host_grad", "librett_c_mlp_host_adam",
@@ -218,6 +218,8 @@ def lib():
         L.librett_c_mlp_sizes.argtypes = [ip, ip, ip]
         L.librett_c_measure_candidates.argtypes = [ctypes.c_int, ip, ip, ctypes.c_size_t, vp, vp, vp, dp, ctypes.c_int,
                                                    ip]
+        L.librett_c_measure_steady.argtypes = [ctypes.c_int, ip, ip, ctypes.c_size_t, vp, vp, vp, ctypes.c_size_t,
+                                               ctypes.c_int, dp, ctypes.c_int, ip]
         L.librett_c_selector_features.argtypes = [ctypes.c_int, ip, ip, ctypes.c_size_t, ctypes.POINTER(DeviceDesc),
                                                   fp, ctypes.c_int, ip, ip]
         L.librett_c_selector_choose.argtypes = [ctypes.c_int, ip, ip, ctypes.c_size_t, ip]
@@ -561,6 +563,21 @@ def measure_candidates(dim, permutation, sizeofType, stream, idata, odata, max_c
                                            ctypes.byref(n))
     if r != LIBRETT_SUCCESS:
         raise ValueError("measure_candidates failed: %d" % r)
+    return t[:min(n.value, max_count)].copy()
+
+
+def measure_steady(dim, permutation, sizeofType, stream, idata, odata, stride, sets, max_count=1024):
+    """Seconds per launch of every candidate in a stream of launches over
+    `sets` buffer pairs, `stride` bytes apart."""
+    import numpy as np
+    t = np.full(max_count, -1.0)
+    n = ctypes.c_int(0)
+    r = lib().librett_c_measure_steady(len(dim), _iarr(dim), _iarr(permutation), int(sizeofType),
+                                       ctypes.c_void_p(stream), ctypes.c_void_p(idata), ctypes.c_void_p(odata),
+                                       int(stride), int(sets), t.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                                       max_count, ctypes.byref(n))
+    if r != LIBRETT_SUCCESS:
+        raise ValueError("measure_steady failed: %d" % r)
     return t[:min(n.value, max_count)].copy()
 
 

@@ -216,6 +216,32 @@ double time_candidate(const Candidate& c, hipStream_t stream, const void* in, vo
   return ts[ts.size() / 2] * 1e-3;
 }
 
+// Time of candidate c in a stream of launches over `sets` buffer pairs that
+// lie `stride` bytes apart, in turn: seconds per launch, or negative on
+// failure. One launch that takes more than three times `best` (positive: the
+// fastest so far) is enough to place it.
+double time_steady(const Candidate& c, hipStream_t stream, const char* in, char* out, size_t stride, int sets,
+                   hipEvent_t e0, hipEvent_t e1, double best) {
+  if (prepare_kernel(c) != 0) return -1;
+  int at = 0;
+  auto timed = [&](int n) -> double {
+    bool ok = hipEventRecord(e0, stream) == hipSuccess;
+    for (int i = 0; ok && i < n; i++, at = (at + 1) % sets)
+      ok = launch_candidate(c, in + at * stride, out + at * stride, stream) == hipSuccess;
+    ok = ok && hipEventRecord(e1, stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
+    float ms = 0;
+    if (!ok || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) return -1;
+    return ms * 1e-3 / n;
+  };
+  double t = timed(1);
+  if (t < 0 || (best > 0 && t > 3 * best + 30e-6)) return t;
+  const int n = std::max(6, std::min(24, (int)(150e-6 / t) + 1));
+  t = timed(n);
+  if (t < 0 || (best > 0 && t > 1.3 * best)) return t;
+  const double u = timed(n);
+  return u < 0 ? u : std::min(t, u);
+}
+
 void fill_info(const Candidate& c, double measured, librett_c_plan_info* info) {
   std::memset(info, 0, sizeof(*info));
   info->method = c.method;
@@ -521,6 +547,42 @@ int librett_c_measure_candidates(int rank, const int* dim, const int* permutatio
     const std::vector<double> ts = measure_all(full, cands, dev, (hipStream_t)stream, idata, odata);
     if (count) *count = (int)cands.size();
     for (int i = 0; i < (int)ts.size() && i < max && times; i++) times[i] = ts[i];
+    return LIBRETT_SUCCESS;
+  } catch (...) {
+    return LIBRETT_INTERNAL_ERROR;
+  }
+}
+
+int librett_c_measure_steady(int rank, const int* dim, const int* permutation, size_t sizeofType, void* stream,
+                             const void* idata, void* odata, size_t stride, int sets, double* times, int max,
+                             int* count) {
+  librettResult r = check_input(rank, dim, permutation, sizeofType);
+  if (r != LIBRETT_SUCCESS) return r;
+  if (!idata || !odata || idata == odata || sets < 1 || stride % 128 != 0) return LIBRETT_INVALID_PARAMETER;
+  try {
+    DeviceInfo dev;
+    if (!device_info(dev)) return LIBRETT_INTERNAL_ERROR;
+    const Problem full = canonicalize(rank, dim, permutation, (int)sizeofType);
+    if (sets > 1 && stride < (size_t)full.vol * sizeofType) return LIBRETT_INVALID_PARAMETER;
+    const std::vector<Candidate> cands = make_candidates(full, dev);
+    if (count) *count = (int)cands.size();
+    hipEvent_t e0, e1;
+    if (hipEventCreate(&e0) != hipSuccess) return LIBRETT_INTERNAL_ERROR;
+    if (hipEventCreate(&e1) != hipSuccess) {
+      (void)hipEventDestroy(e0);
+      return LIBRETT_INTERNAL_ERROR;
+    }
+    double best = -1;
+    for (int i = 0; i < (int)cands.size() && i < max && times; i++) {
+      const Candidate& c = cands[i];
+      const uintptr_t mis = ((uintptr_t)idata | (uintptr_t)odata) & (uintptr_t)(needed_alignment(c) - 1);
+      times[i] = time_steady(mis ? unaligned_fallback(c) : c, (hipStream_t)stream, (const char*)idata, (char*)odata,
+                             stride, sets, e0, e1, best);
+      if (times[i] > 0 && (best < 0 || times[i] < best)) best = times[i];
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    (void)hipGetLastError();
     return LIBRETT_SUCCESS;
   } catch (...) {
     return LIBRETT_INTERNAL_ERROR;

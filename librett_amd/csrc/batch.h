@@ -55,7 +55,9 @@ long long batch_unit_bytes(long long total_bytes, int grid);
 
 // The kernel comes in one instantiation per family of shapes, so
 // that each holds only the registers its own shapes need.
-enum BatchFamily : int { kFamTiled = 0, kFamCopy = 1, kFamPacked = 2, kFamTiledG = 3 };
+// kFamLines holds the kernels that write whole lines wherever the output
+// starts: TiledCopy and the skewed, narrow and short forms of Tiled.
+enum BatchFamily : int { kFamTiled = 0, kFamLines = 1, kFamPacked = 2, kFamTiledG = 3 };
 constexpr int kBatchFamilies = 4;
 
 // Family of a shape-table index.

@@ -14,36 +14,44 @@ namespace lrt {
 
 namespace {
 
-// Shape table: id, method, element bytes, four method parameters, group flag
+// Shape table: id, method, element bytes, four method parameters, group flag,
+// tile form
 //   Tiled:     tile_x, tile_y, vec_x, vec_y; group flag 1 for planes over
-//              dim groups (their own family, so the one-dim kernels keep
-//              their registers)
+//              dim groups (rectangular tiles: their own family, so the one-dim
+//              kernels keep their registers); narrow and short tiles size
+//              themselves
 //   TiledCopy: none
 //   Packed:    nreg
 #define LRT_BATCH_TABLE(X)                                                  \
-  X(0, kTiled, 4, 64, 64, 1, 1, 0) X(1, kTiled, 4, 64, 64, 4, 1, 0)         \
-  X(2, kTiled, 4, 64, 64, 1, 4, 0) X(3, kTiled, 4, 64, 64, 4, 4, 0)         \
-  X(4, kTiled, 8, 32, 32, 1, 1, 0) X(5, kTiled, 8, 32, 32, 2, 1, 0)         \
-  X(6, kTiled, 8, 32, 32, 1, 2, 0) X(7, kTiled, 8, 32, 32, 2, 2, 0)         \
-  X(8, kTiled, 16, 32, 32, 1, 1, 0)                                         \
-  X(9, kTiledCopy, 4, 0, 0, 0, 0, 0) X(10, kTiledCopy, 8, 0, 0, 0, 0, 0)    \
-  X(11, kTiledCopy, 16, 0, 0, 0, 0, 0)                                      \
-  X(12, kPacked, 4, 1, 0, 0, 0, 0) X(13, kPacked, 4, 2, 0, 0, 0, 0)         \
-  X(14, kPacked, 4, 4, 0, 0, 0, 0) X(15, kPacked, 4, 8, 0, 0, 0, 0)         \
-  X(16, kPacked, 8, 1, 0, 0, 0, 0) X(17, kPacked, 8, 2, 0, 0, 0, 0)         \
-  X(18, kPacked, 8, 4, 0, 0, 0, 0) X(19, kPacked, 8, 8, 0, 0, 0, 0)         \
-  X(20, kPacked, 16, 1, 0, 0, 0, 0) X(21, kPacked, 16, 2, 0, 0, 0, 0)       \
-  X(22, kPacked, 16, 4, 0, 0, 0, 0)                                         \
-  X(23, kTiled, 4, 64, 64, 1, 1, 1) X(24, kTiled, 4, 64, 64, 4, 1, 1)       \
-  X(25, kTiled, 4, 64, 64, 1, 4, 1) X(26, kTiled, 4, 64, 64, 4, 4, 1)       \
-  X(27, kTiled, 8, 32, 32, 1, 1, 1) X(28, kTiled, 8, 32, 32, 2, 1, 1)       \
-  X(29, kTiled, 8, 32, 32, 1, 2, 1) X(30, kTiled, 8, 32, 32, 2, 2, 1)       \
-  X(31, kTiled, 16, 32, 32, 1, 1, 1)
+  X(0, kTiled, 4, 64, 64, 1, 1, 0, kTileRect) X(1, kTiled, 4, 64, 64, 4, 1, 0, kTileRect)         \
+  X(2, kTiled, 4, 64, 64, 1, 4, 0, kTileRect) X(3, kTiled, 4, 64, 64, 4, 4, 0, kTileRect)         \
+  X(4, kTiled, 8, 32, 32, 1, 1, 0, kTileRect) X(5, kTiled, 8, 32, 32, 2, 1, 0, kTileRect)         \
+  X(6, kTiled, 8, 32, 32, 1, 2, 0, kTileRect) X(7, kTiled, 8, 32, 32, 2, 2, 0, kTileRect)         \
+  X(8, kTiled, 16, 32, 32, 1, 1, 0, kTileRect)                                         \
+  X(9, kTiledCopy, 4, 0, 0, 0, 0, 0, kTileRect) X(10, kTiledCopy, 8, 0, 0, 0, 0, 0, kTileRect)    \
+  X(11, kTiledCopy, 16, 0, 0, 0, 0, 0, kTileRect)                                      \
+  X(12, kPacked, 4, 1, 0, 0, 0, 0, kTileRect) X(13, kPacked, 4, 2, 0, 0, 0, 0, kTileRect)         \
+  X(14, kPacked, 4, 4, 0, 0, 0, 0, kTileRect) X(15, kPacked, 4, 8, 0, 0, 0, 0, kTileRect)         \
+  X(16, kPacked, 8, 1, 0, 0, 0, 0, kTileRect) X(17, kPacked, 8, 2, 0, 0, 0, 0, kTileRect)         \
+  X(18, kPacked, 8, 4, 0, 0, 0, 0, kTileRect) X(19, kPacked, 8, 8, 0, 0, 0, 0, kTileRect)         \
+  X(20, kPacked, 16, 1, 0, 0, 0, 0, kTileRect) X(21, kPacked, 16, 2, 0, 0, 0, 0, kTileRect)       \
+  X(22, kPacked, 16, 4, 0, 0, 0, 0, kTileRect)                                         \
+  X(23, kTiled, 4, 64, 64, 1, 1, 1, kTileRect) X(24, kTiled, 4, 64, 64, 4, 1, 1, kTileRect)       \
+  X(25, kTiled, 4, 64, 64, 1, 4, 1, kTileRect) X(26, kTiled, 4, 64, 64, 4, 4, 1, kTileRect)       \
+  X(27, kTiled, 8, 32, 32, 1, 1, 1, kTileRect) X(28, kTiled, 8, 32, 32, 2, 1, 1, kTileRect)       \
+  X(29, kTiled, 8, 32, 32, 1, 2, 1, kTileRect) X(30, kTiled, 8, 32, 32, 2, 2, 1, kTileRect)       \
+  X(31, kTiled, 16, 32, 32, 1, 1, 1, kTileRect) \
+  X(32, kTiled, 4, 32, 64, 1, 4, 0, kTileSkew) X(33, kTiled, 4, 32, 64, 1, 4, 1, kTileSkew)   \
+  X(34, kTiled, 8, 32, 32, 1, 2, 0, kTileSkew) X(35, kTiled, 8, 32, 32, 1, 2, 1, kTileSkew)   \
+  X(36, kTiled, 16, 16, 32, 1, 1, 0, kTileSkew) X(37, kTiled, 16, 16, 32, 1, 1, 1, kTileSkew) \
+  X(38, kTiled, 4, 0, 0, 1, 4, 0, kTileNarrow) X(39, kTiled, 8, 0, 0, 1, 2, 0, kTileNarrow)   \
+  X(40, kTiled, 16, 0, 0, 1, 1, 0, kTileNarrow) X(41, kTiled, 4, 0, 0, 1, 4, 0, kTileShort)   \
+  X(42, kTiled, 8, 0, 0, 1, 2, 0, kTileShort) X(43, kTiled, 16, 0, 0, 1, 1, 0, kTileShort)
 
 struct BatchShape {
-  int id, method, b, p1, p2, p3, p4, g;
+  int id, method, b, p1, p2, p3, p4, g, form;
 };
-#define LRT_BATCH_ROW(ID, M, B, P1, P2, P3, P4, G) {ID, M, B, P1, P2, P3, P4, G},
+#define LRT_BATCH_ROW(ID, M, B, P1, P2, P3, P4, G, FORM) {ID, M, B, P1, P2, P3, P4, G, FORM},
 const BatchShape kBatchShapes[] = {LRT_BATCH_TABLE(LRT_BATCH_ROW)};
 #undef LRT_BATCH_ROW
 
@@ -79,6 +87,27 @@ __device__ __forceinline__ void dev_tiled(const BatchDesc& D, int lu, unsigned c
     Ops::load(D.a.tiled, c, threadIdx.x, static_cast<const E*>(D.in), lds);
     __syncthreads();
     Ops::store(D.a.tiled, c, threadIdx.x, static_cast<E*>(D.out), lds);
+    __syncthreads();
+  }
+}
+
+// Skewed, narrow and short tiles.
+template <class Ops>
+__device__ __forceinline__ void dev_lines(const BatchDesc& D, int lu, unsigned char* lds_raw) {
+  using E = typename Ops::E;
+  E* lds = reinterpret_cast<E*>(lds_raw);
+  const TiledArgs& a = D.a.tiled;
+  E* out = static_cast<E*>(D.out);
+  const int phase = line_phase(out);
+  for (int w = lu; w < D.items; w += D.groups) {
+    const TileCtx c = Ops::item(a, (uint32_t)w);
+    if (Ops::early(a)) {
+      Ops::prepare(a, c, threadIdx.x, lds);
+      __syncthreads();
+    }
+    Ops::load(a, c, threadIdx.x, static_cast<const E*>(D.in), lds, phase);
+    __syncthreads();
+    Ops::store(a, c, threadIdx.x, out, lds, phase);
     __syncthreads();
   }
 }
@@ -142,11 +171,23 @@ __device__ __forceinline__ void dev_unit(const BatchDesc& D, int lu, unsigned ch
       case 31: dev_tiled<16, 32, 32, 1, 1, true>(D, lu, lds); break;
       default: break;
     }
-  } else if constexpr (FAM == kFamCopy) {
+  } else if constexpr (FAM == kFamLines) {
     switch (D.variant) {
       case 9: dev_copy<4>(D, lu); break;
       case 10: dev_copy<8>(D, lu); break;
       case 11: dev_copy<16>(D, lu); break;
+      case 32: dev_lines<SkewOps<4, 32, 64, 256, false>>(D, lu, lds); break;
+      case 33: dev_lines<SkewOps<4, 32, 64, 256, true>>(D, lu, lds); break;
+      case 34: dev_lines<SkewOps<8, 32, 32, 256, false>>(D, lu, lds); break;
+      case 35: dev_lines<SkewOps<8, 32, 32, 256, true>>(D, lu, lds); break;
+      case 36: dev_lines<SkewOps<16, 16, 32, 256, false>>(D, lu, lds); break;
+      case 37: dev_lines<SkewOps<16, 16, 32, 256, true>>(D, lu, lds); break;
+      case 38: dev_lines<NarrowOps<4, 256, 8>>(D, lu, lds); break;
+      case 39: dev_lines<NarrowOps<8, 256, 6>>(D, lu, lds); break;
+      case 40: dev_lines<NarrowOps<16, 256, 4>>(D, lu, lds); break;
+      case 41: dev_lines<ShortOps<4, 256, 8>>(D, lu, lds); break;
+      case 42: dev_lines<ShortOps<8, 256, 6>>(D, lu, lds); break;
+      case 43: dev_lines<ShortOps<16, 256, 4>>(D, lu, lds); break;
       default: break;
     }
   } else {
@@ -173,8 +214,12 @@ __device__ __forceinline__ void dev_unit(const BatchDesc& D, int lu, unsigned ch
 // fixed share of them each finished far apart. It also needs fewer registers
 // than a loop over units (48 to 68 VGPRs, no scratch; 58 to 85 with the loop),
 // so 7 or 8 workgroups fit a CU where 5 or 6 did. On MI355X, 4096 problems of
-// 13.8 GB 3335 -> 2981 us, a burst of 128 served requests 775 -> 746 us. Bound by
-// HBM; a copy of the bytes takes 2180 us.
+// 13.8 GB 3335 -> 2981 us (2710 us with their kernels ranked by batch_cost), a
+// burst of 128 served requests 775 -> 746 us (700 us). Bound by HBM; a copy of
+// the bytes takes 2180 us. One kernel for all families (71 VGPRs, one launch
+// instead of four) ran no faster: 2737 us and 688 us. Neither did units sorted
+// by shape (3428 us against 3349 with the loop): problems of unlike kernels
+// fill each other's waits.
 template <int FAM>
 __global__ __launch_bounds__(256) void k_batch(
     const BatchDesc* __restrict__ descs, const int* __restrict__ start, int nprob, int total) {
@@ -189,7 +234,7 @@ const void* batch_kernel(int fam) {
   switch (fam) {
     case kFamTiled: return reinterpret_cast<const void*>(&k_batch<kFamTiled>);
     case kFamTiledG: return reinterpret_cast<const void*>(&k_batch<kFamTiledG>);
-    case kFamCopy: return reinterpret_cast<const void*>(&k_batch<kFamCopy>);
+    case kFamLines: return reinterpret_cast<const void*>(&k_batch<kFamLines>);
     default: return reinterpret_cast<const void*>(&k_batch<kFamPacked>);
   }
 }
@@ -208,6 +253,22 @@ void host_tiled(const BatchDesc& D, int lu, unsigned char* lds_raw) {
     for (int t = 0; t < 256; t++) Ops::prepare(D.a.tiled, c, t, lds);
     for (int t = 0; t < 256; t++) Ops::load(D.a.tiled, c, t, static_cast<const E*>(D.in), lds);
     for (int t = 0; t < 256; t++) Ops::store(D.a.tiled, c, t, static_cast<E*>(D.out), lds);
+  }
+}
+
+template <class Ops>
+void host_lines(const BatchDesc& D, int lu, unsigned char* lds_raw) {
+  using E = typename Ops::E;
+  E* lds = reinterpret_cast<E*>(lds_raw);
+  const TiledArgs& a = D.a.tiled;
+  E* out = static_cast<E*>(D.out);
+  const int phase = line_phase(out);
+  for (int w = lu; w < D.items; w += D.groups) {
+    const TileCtx c = Ops::item(a, (uint32_t)w);
+    if (Ops::early(a))
+      for (int t = 0; t < Ops::NT; t++) Ops::prepare(a, c, t, lds);
+    for (int t = 0; t < Ops::NT; t++) Ops::load(a, c, t, static_cast<const E*>(D.in), lds, phase);
+    for (int t = 0; t < Ops::NT; t++) Ops::store(a, c, t, out, lds, phase);
   }
 }
 
@@ -272,6 +333,18 @@ void host_unit(const BatchDesc& D, int lu, unsigned char* lds) {
     case 29: host_tiled<8, 32, 32, 1, 2, true>(D, lu, lds); break;
     case 30: host_tiled<8, 32, 32, 2, 2, true>(D, lu, lds); break;
     case 31: host_tiled<16, 32, 32, 1, 1, true>(D, lu, lds); break;
+    case 32: host_lines<SkewOps<4, 32, 64, 256, false>>(D, lu, lds); break;
+    case 33: host_lines<SkewOps<4, 32, 64, 256, true>>(D, lu, lds); break;
+    case 34: host_lines<SkewOps<8, 32, 32, 256, false>>(D, lu, lds); break;
+    case 35: host_lines<SkewOps<8, 32, 32, 256, true>>(D, lu, lds); break;
+    case 36: host_lines<SkewOps<16, 16, 32, 256, false>>(D, lu, lds); break;
+    case 37: host_lines<SkewOps<16, 16, 32, 256, true>>(D, lu, lds); break;
+    case 38: host_lines<NarrowOps<4, 256, 8>>(D, lu, lds); break;
+    case 39: host_lines<NarrowOps<8, 256, 6>>(D, lu, lds); break;
+    case 40: host_lines<NarrowOps<16, 256, 4>>(D, lu, lds); break;
+    case 41: host_lines<ShortOps<4, 256, 8>>(D, lu, lds); break;
+    case 42: host_lines<ShortOps<8, 256, 6>>(D, lu, lds); break;
+    case 43: host_lines<ShortOps<16, 256, 4>>(D, lu, lds); break;
     default: break;
   }
 }
@@ -280,9 +353,15 @@ void host_unit(const BatchDesc& D, int lu, unsigned char* lds) {
 
 bool batch_tiled_available(int elem, int tx, int ty, int vx, int vy, bool general) {
   for (const auto& s : kBatchShapes)
-    if (s.method == kTiled && s.b == elem && s.p1 == tx && s.p2 == ty && s.p3 == vx && s.p4 == vy &&
-        (s.g != 0) == general)
+    if (s.method == kTiled && s.form == kTileRect && s.b == elem && s.p1 == tx && s.p2 == ty && s.p3 == vx &&
+        s.p4 == vy && (s.g != 0) == general)
       return true;
+  return false;
+}
+
+bool batch_skew_available(int elem, int tx, int ty) {
+  for (const auto& s : kBatchShapes)
+    if (s.form == kTileSkew && s.b == elem && s.p1 == tx && s.p2 == ty) return true;
   return false;
 }
 
@@ -309,8 +388,9 @@ int batch_variant(const Candidate& c) {
   for (const auto& s : kBatchShapes) {
     switch (c.method) {
       case kTiled:
-        if (s.method == kTiled && s.b == c.elem && s.p1 == c.tile_x && s.p2 == c.tile_y && s.p3 == c.vec_x &&
-            s.p4 == c.vec_y && (s.g != 0) == (c.xgroup > 1 || c.ygroup > 1))
+        if (s.method == kTiled && s.b == c.elem && s.form == c.tiled.form &&
+            (s.form >= kTileNarrow || (s.p1 == c.tile_x && s.p2 == c.tile_y && s.p3 == c.vec_x && s.p4 == c.vec_y &&
+                                       (s.g != 0) == (c.xgroup > 1 || c.ygroup > 1))))
           return s.id;
         break;
       case kTiledCopy:
@@ -337,7 +417,7 @@ bool batch_describe(const Candidate& c, BatchDesc& d) {
     case kTiled:
       d.a.tiled = c.tiled;
       d.items = c.tiled.items;
-      d.item_bytes = 2 * c.tile_x * c.tile_y * c.elem;
+      d.item_bytes = 2 * c.elem * (c.tiled.form == kTileShort ? c.tile_x : c.tile_x * c.tile_y);
       break;
     case kTiledCopy:
       d.a.copy = c.copy;
@@ -380,7 +460,7 @@ long long batch_unit_bytes(long long total_bytes, int grid) {
 }
 
 int batch_family(int variant) {
-  return variant <= 8 ? kFamTiled : variant <= 11 ? kFamCopy : variant <= 22 ? kFamPacked : kFamTiledG;
+  return variant <= 8 ? kFamTiled : variant <= 11 ? kFamLines : variant <= 22 ? kFamPacked : variant <= 31 ? kFamTiledG : kFamLines;
 }
 
 hipError_t launch_batch(int fam, const BatchDesc* d_descs, const int* d_start, int nprob, int total,

@@ -344,7 +344,7 @@ std::vector<Candidate> batch_candidates(const Problem& p, const DeviceInfo& dev)
 
 int batch_alignment(const Problem& p, const Candidate& c) {
   if (c.method == kTrivial) return p.elem;
-  if (c.method == kTiled) return c.elem * std::max(c.vec_x, c.vec_y);
+  if (c.method == kTiled && c.tiled.form == kTileRect) return c.elem * std::max(c.vec_x, c.vec_y);
   return c.elem;
 }
 
@@ -356,7 +356,7 @@ bool describe_problem(const Problem& p, const Candidate& c, std::vector<BatchDes
   BatchDesc d, f;
   if (!batch_describe(c.method == kTrivial ? flat_copy(p) : c, d)) return false;
   Candidate fc = c.method == kTrivial ? flat_copy(p) : c;
-  if (c.method == kTiled) fc.vec_x = fc.vec_y = 1;
+  if (c.method == kTiled && c.tiled.form == kTileRect) fc.vec_x = fc.vec_y = 1;
   if (!batch_describe(fc, f)) f = d;
   descs.push_back(d);
   fallback.push_back(f);

@@ -111,6 +111,8 @@ __host__ __device__ inline int group_offset(const GroupMap& g, uint32_t v) {
   return off + (int)v * g.stride[kMaxGroup - 1];
 }
 
+enum TileForm : int { kTileRect = 0, kTileSkew = 1, kTileNarrow = 2, kTileShort = 3 };
+
 // Tiled: 2-D tile plane of (x = input dim 0, y = the input dim that becomes
 // output dim 0). Reference counterpart: transposeTiled, src/kernel.cpp:48-170.
 // x may also be a group of leading input dims (contiguous in the input, in
@@ -139,6 +141,16 @@ struct TiledArgs {
   FastDiv group_row_div;  // group * ntx
   FastDiv last_div;       // rows in the last (possibly partial) group
   int last_group_start;   // first tile index of the last group
+  // Form of the tiles. kTileSkew (SkewOps) and kTileNarrow (NarrowOps): a
+  // tile's columns start on 128-byte lines of the output, each up to a line
+  // before row y0, so the last tile row may start past Y for some columns.
+  // kTileNarrow tiles hold all X columns. kTileShort (ShortOps): tiles are
+  // stretches of the output, each column of which is all Y elements.
+  int form;
+  FastDiv x_div;  // kTileNarrow: X; kTileShort: Y
+  FastDiv nx_div; // kTileShort: columns that a tile's loads are laid out for
+  int word_shift; // kTileNarrow: log2 of the 16-byte words of a tile's column
+  int stream_in;  // non-temporal loads: whole lines, and more than the Infinity Cache keeps
   // > 1: workgroup b starts at tile xcd_logical(b, grid, xcds), so each XCD
   // walks one contiguous range of tiles (tiles that share 128-byte lines
   // then meet in one XCD's L2); 1: workgroup b starts at tile b.
@@ -152,6 +164,63 @@ __host__ __device__ inline int tiled_out_x(const TiledArgs& a, uint32_t x) {
 }
 __host__ __device__ inline int tiled_in_y(const TiledArgs& a, uint32_t y) {
   return a.yg.n > 1 ? group_offset(a.yg, y) : (int)y * a.in_ys;
+}
+
+// Skews of the columns of a skewed (or narrow) tile at (x0, y0) of width tx,
+// for an output that starts on a line of `le` elements.
+constexpr int kMaxSkewTile = 64;
+struct SkewTile {
+  int tx, lo, hi;  // columns; smallest and largest skew
+  unsigned char s[kMaxSkewTile];
+};
+
+__host__ __device__ inline SkewTile skew_tile(const TiledArgs& a, int off_out, int x0, int tx, int le) {
+  SkewTile k;
+  k.tx = tx;
+  k.lo = le;
+  k.hi = 0;
+  for (int i = 0; i < tx; i++) {
+    const int s = (off_out + tiled_out_x(a, (uint32_t)(x0 + i))) & (le - 1);
+    k.s[i] = (unsigned char)s;
+    if (s < k.lo) k.lo = s;
+    if (s > k.hi) k.hi = s;
+  }
+  return k;
+}
+
+// f(first column, columns) for each run of neighbouring columns that cover
+// plane row y of a tile at y0 with ty rows.
+template <class F>
+__host__ __device__ inline void skew_row_runs(const SkewTile& k, int y, int y0, int ty, F&& f) {
+  if (y >= y0 - k.lo && y < y0 - k.hi + ty) {
+    f(0, k.tx);
+    return;
+  }
+  int i = 0;
+  while (i < k.tx) {
+    const int d = y - y0 + k.s[i];
+    if (d < 0 || d >= ty) {
+      i++;
+      continue;
+    }
+    const int i0 = i;
+    while (i < k.tx && y - y0 + k.s[i] >= 0 && y - y0 + k.s[i] < ty) i++;
+    f(i0, i - i0);
+  }
+}
+
+// Output elements [e0, e1) of tile `tile` of a plane of short columns, tiles of
+// ch elements, for an output that starts on a line; and the columns [xa, xb) of
+// plane row y among them.
+__host__ __device__ inline void short_tile(const TiledArgs& a, int off_out, int tile, int ch, int le, int& e0,
+                                           int& e1) {
+  const int s = tile * ch - (off_out & (le - 1)), n = a.X * a.Y;
+  e0 = s < 0 ? 0 : s;
+  e1 = n - s < ch ? n : s + ch;
+}
+__host__ __device__ inline void short_row(const TiledArgs& a, int y, int e0, int e1, int& xa, int& xb) {
+  xa = (e0 - y + a.Y - 1) / a.Y;
+  xb = (e1 - y + a.Y - 1) / a.Y;
 }
 
 // TiledCopy: rows that stay contiguous in input and output (perm[0] == 0).

@@ -37,6 +37,8 @@ constexpr int kCountMaxGrid = 2048;
 // Row pieces of a TiledCopy item: at most 1024 elements (of 4 bytes) in rows
 // of at least 2, the first of which may be cut.
 constexpr int kCopyPieces = 514;
+// Rows of a skewed tile: at most 128 and a line of 4-byte elements.
+constexpr int kSkewRows = 160;
 
 struct RunRef {
   int off, n;  // start and length in the run table (pairs of ints)
@@ -46,7 +48,8 @@ struct CountJob {
   int method;          // kTiled, kTiledCopy, kPacked or kPackedSplit
   int B;               // element bytes
   int TX, TY, VX, VY;  // Tiled: tile and vector widths
-  int nt, nreg;        // Packed: threads and registers (passes) per thread
+  int nt;              // threads of a workgroup
+  int nreg;            // Packed: registers (passes) per thread
   long long items;
   const int* runs;     // Packed: (start, length) element runs of each staged shape
   RunRef run[2][2];    // [variant][0 input side, 1 output side]
@@ -60,8 +63,9 @@ struct CountJob {
 __host__ __device__ inline int imin(int a, int b) { return a < b ? a : b; }
 
 struct ItemCtx {
-  int x0, y0, tx, ty;  // Tiled: tile origin and extent
+  int x0, y0, tx, ty;  // Tiled: tile origin and extent (short columns: elements [tx, ty))
   int plus;            // Packed: staged shape variant
+  SkewTile skew;       // skewed tiles
   long long in0, out0; // element offset of the item's base (TiledCopy: out0 only)
 };
 
@@ -91,6 +95,8 @@ __host__ __device__ inline ItemCtx item_ctx(const CountJob& j, uint32_t w) {
     outer_offsets(a.outer, mb, oi, oo);
     c.in0 = oi;
     c.out0 = oo;
+    if (a.form == kTileShort) short_tile(a, oo, (int)tile, j.TX, 128 / j.B, c.tx, c.ty);
+    else if (a.form != kTileRect) c.skew = skew_tile(a, oo, c.x0, c.tx, 128 / j.B);
   } else if (j.method == kTiledCopy) {
     c.out0 = (long long)w * j.a.copy.per;
   } else {
@@ -111,15 +117,20 @@ __host__ __device__ inline ItemCtx item_ctx(const CountJob& j, uint32_t w) {
   return c;
 }
 
-__host__ __device__ inline int job_threads(const CountJob& j) {
-  return (j.method == kPacked || j.method == kPackedSplit) ? j.nt : kCountThreads;
-}
-
 // Instructions (passes) per thread of one kind.
 __host__ __device__ inline int job_passes(const CountJob& j, int store) {
   switch (j.method) {
     case kTiled:
-      return store ? (j.TX * j.TY) / (j.VY * kCountThreads) : (j.TX * j.TY) / (j.VX * kCountThreads);
+      if (j.a.tiled.form == kTileShort)
+        return store ? j.TX / j.nt : (int)(j.a.tiled.nx_div.d * j.TY + j.nt - 1) / j.nt;
+      if (j.a.tiled.form == kTileNarrow)
+        return store ? (j.TX * j.TY + j.nt - 1) / j.nt + j.VY : (j.TX * (j.TY + 128 / j.B) + j.nt - 1) / j.nt;
+      if (j.a.tiled.form == kTileSkew) {
+        // At most: every row of a lane's column, and the elements of every word.
+        const int rp = j.nt / j.TX;
+        return store ? (j.TX * j.TY) / j.nt : (j.TY + 128 / j.B + rp - 1) / rp;
+      }
+      return store ? (j.TX * j.TY) / (j.VY * j.nt) : (j.TX * j.TY) / (j.VX * j.nt);
     case kTiledCopy:
       // A lane's word, or the elements of a word that crosses a row's end
       // (loads) or the tensor's end: its k-th access is counted with the other
@@ -131,7 +142,7 @@ __host__ __device__ inline int job_passes(const CountJob& j, int store) {
 }
 
 __host__ __device__ inline int job_access_bytes(const CountJob& j, int store) {
-  if (j.method == kTiled) return j.B * (store ? j.VY : j.VX);
+  if (j.method == kTiled && j.a.tiled.form == kTileRect) return j.B * (store ? j.VY : j.VX);
   return j.B;
 }
 
@@ -141,18 +152,101 @@ __host__ __device__ inline int job_access_bytes(const CountJob& j, int store) {
 // CopyOps::run and PackedOps::prepare / load / store.
 __host__ __device__ inline bool lane_access(const CountJob& j, const ItemCtx& c, int store, int p, int t,
                                             long long& off, int& bytes) {
+  if (j.method == kTiled && j.a.tiled.form == kTileShort) {
+    // The p-th element that a lane loads (every nt-th of the rows laid out nx
+    // columns each) or the p-th access of its words.
+    const TiledArgs& a = j.a.tiled;
+    int q = p;
+    if (!store) {
+      const int nx = (int)a.nx_div.d, xa = c.tx / a.Y;
+      for (int i = t; i < nx * a.Y; i += j.nt) {
+        const int y = i / nx, x = xa + i - y * nx, e = x * a.Y + y;
+        if (e < c.tx || e >= c.ty || q-- > 0) continue;
+        off = (c.in0 + x + (long long)tiled_in_y(a, (uint32_t)y)) * j.B;
+        return true;
+      }
+      return false;
+    }
+    const int e0 = c.tx == 0 ? -(int)(c.out0 & (128 / j.B - 1)) : c.tx;  // the tile's own start
+    for (int w = t; w < j.TX / j.VY; w += j.nt) {
+      const int e = e0 + w * j.VY;
+      const int ea = e > 0 ? e : 0, eb = imin(a.X * a.Y, e + j.VY);
+      const bool word = e >= 0 && e + j.VY <= a.X * a.Y;
+      const int n = word ? 1 : (eb > ea ? eb - ea : 0);
+      if (q < n) {
+        if (word) bytes = j.VY * j.B;
+        off = (c.out0 + (word ? e : ea + q)) * j.B;
+        return true;
+      }
+      q -= n;
+    }
+    return false;
+  }
+  if (j.method == kTiled && j.a.tiled.form != kTileRect) {
+    const TiledArgs& a = j.a.tiled;
+    const bool narrow = a.form == kTileNarrow;
+    if (!store && narrow) {
+      // Every nt-th element of the tile's rows, of which the lane skips those
+      // that their column does not cover: this is the p-th it takes.
+      const int LE = 128 / j.B, n = (j.TY + LE) * a.X;
+      int q = p;
+      for (int i = t; i < n; i += j.nt) {
+        const int row = i / a.X, x = i - row * a.X;
+        const int y = c.y0 - LE + row, d = y - c.y0 + c.skew.s[x];
+        if (d < 0 || d >= j.TY || y < 0 || y >= a.Y) continue;
+        if (q-- > 0) continue;
+        off = (c.in0 + (long long)y * a.X + x) * j.B;
+        return true;
+      }
+      return false;
+    }
+    if (!store) {
+      // Rows y0 - s .. y0 - s + TY of the lane's column, those of the plane;
+      // the lane takes every RP-th, and this is the p-th it takes.
+      const int RP = j.nt / j.TX, LE = 128 / j.B;
+      const int i = t % j.TX;
+      if (i >= c.tx) return false;
+      const int ya = c.y0 - c.skew.s[i] > 0 ? c.y0 - c.skew.s[i] : 0;
+      const int yb = imin(a.Y, c.y0 - c.skew.s[i] + j.TY);
+      int y = c.y0 - LE + t / j.TX;
+      if (y < ya) y += (ya - y + RP - 1) / RP * RP;
+      y += p * RP;
+      if (y >= yb) return false;
+      off = (long long)(c.in0 + c.x0 + i + (long long)tiled_in_y(a, (uint32_t)y)) * j.B;
+      return true;
+    }
+    // The lane's words: narrow tiles deal them column after column, skewed
+    // tiles give a lane one place in every WP-th column.
+    const int LW = j.TY / j.VY, step = narrow ? j.nt : j.nt / LW * LW;
+    int q = p;
+    for (int wd = t; wd < c.tx * LW; wd += step) {
+      const int i = wd / LW;
+      // The lane's word in column i: whole, or the elements inside the plane.
+      const int y = c.y0 - c.skew.s[i] + (wd - i * LW) * j.VY;
+      const int ya = y > 0 ? y : 0, yb = imin(a.Y, y + j.VY);
+      const bool word = y >= 0 && y + j.VY <= a.Y;
+      const int n = word ? 1 : (yb > ya ? yb - ya : 0);
+      if (q < n) {
+        if (word) bytes = j.VY * j.B;
+        off = (long long)(c.out0 + (word ? y : ya + q) + (long long)tiled_out_x(a, (uint32_t)(c.x0 + i))) * j.B;
+        return true;
+      }
+      q -= n;
+    }
+    return false;
+  }
   if (j.method == kTiled) {
     const TiledArgs& a = j.a.tiled;
     if (!store) {
       const int LR = j.TX / j.VX;
-      const int RP = kCountThreads / LR;
+      const int RP = j.nt / LR;
       const int x = c.x0 + (t % LR) * j.VX;
       const int y = c.y0 + t / LR + p * RP;
       if (x >= a.X || y >= a.Y) return false;
       off = (long long)(c.in0 + x + (long long)tiled_in_y(a, (uint32_t)y)) * j.B;
     } else {
       const int LW = j.TY / j.VY;
-      const int WP = kCountThreads / LW;
+      const int WP = j.nt / LW;
       const int y = c.y0 + (t % LW) * j.VY;
       const int x = c.x0 + t / LW + p * WP;
       if (x >= a.X || y >= a.Y) return false;
@@ -246,7 +340,46 @@ __host__ __device__ inline void sort_small(long long* v, int n) {
 __host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, unsigned long long* acc) {
   LineWalk rd, wr;
   const long long B = j.B;
-  if (j.method == kTiled) {
+  if (j.method == kTiled && j.a.tiled.form == kTileShort) {
+    const TiledArgs& a = j.a.tiled;
+    long long st[kSkewRows];
+    for (int y = 0; y < a.Y; y++) st[y] = ((long long)tiled_in_y(a, (uint32_t)y) << 8) | y;
+    if (a.yg.n > 1) sort_small(st, a.Y);
+    for (int k = 0; k < a.Y; k++) {
+      int xa, xb;
+      short_row(a, (int)(st[k] & 255), c.tx, c.ty, xa, xb);
+      rd.add((c.in0 + (st[k] >> 8) + xa) * B, (long long)(xb - xa) * B);
+    }
+    wr.add((c.out0 + c.tx) * B, (long long)(c.ty - c.tx) * B);
+  } else if (j.method == kTiled && j.a.tiled.form != kTileRect) {
+    // Rows and columns in address order; where the y or x group's order differs,
+    // each with its index as (start, index) in one sortable value (at most
+    // TY + a line's elements of them).
+    const TiledArgs& a = j.a.tiled;
+    long long st[kSkewRows];
+    int n = 0;
+    const int ya = c.y0 - c.skew.hi > 0 ? c.y0 - c.skew.hi : 0;
+    const int yb = imin(a.Y, c.y0 + j.TY);
+    if (a.yg.n > 1) {
+      for (int y = ya; y < yb; y++) st[n++] = ((c.in0 + c.x0 + (long long)tiled_in_y(a, (uint32_t)y)) << 8) | (y - ya);
+      sort_small(st, n);
+      for (int k = 0; k < n; k++)
+        skew_row_runs(c.skew, ya + (int)(st[k] & 255), c.y0, j.TY,
+                      [&](int i, int len) { rd.add(((st[k] >> 8) + i) * B, len * B); });
+    } else {
+      for (int y = ya; y < yb; y++)
+        skew_row_runs(c.skew, y, c.y0, j.TY, [&](int i, int len) {
+          rd.add((c.in0 + c.x0 + (long long)tiled_in_y(a, (uint32_t)y) + i) * B, len * B);
+        });
+    }
+    for (int i = 0; i < c.tx; i++) st[i] = ((c.out0 + (long long)tiled_out_x(a, (uint32_t)(c.x0 + i))) << 8) | i;
+    if (a.xg.n > 1) sort_small(st, c.tx);
+    for (int k = 0; k < c.tx; k++) {
+      const int s = c.skew.s[st[k] & 255];
+      const int y0 = c.y0 - s > 0 ? c.y0 - s : 0, y1 = imin(a.Y, c.y0 - s + j.TY);
+      if (y0 < y1) wr.add(((st[k] >> 8) + y0) * B, (long long)(y1 - y0) * B);
+    }
+  } else if (j.method == kTiled) {
     const TiledArgs& a = j.a.tiled;
     // Rows (columns) of a one-dim group are in address order; those of a
     // group of several dims are sorted first (a tile has at most 128).
@@ -336,7 +469,7 @@ __global__ __launch_bounds__(kCountThreads) void k_count(CountJob job, unsigned 
   for (int i = 0; i < kNumCounts; i++) acc[i] = 0;
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
-  const int nthreads = job_threads(job);
+  const int nthreads = job.nt;
   const int waves = (nthreads + 63) / 64;
   for (long long w = blockIdx.x; w < job.items; w += gridDim.x) {
     const ItemCtx c = item_ctx(job, (uint32_t)w);
@@ -398,10 +531,16 @@ bool make_job(const Candidate& c, CountJob& j, std::vector<int>& runs) {
       j.VY = c.vec_y;
       j.a.tiled = c.tiled;
       j.items = c.tiled.items;
-      if (j.TX % j.VX || j.TY % j.VY || kCountThreads % (j.TX / j.VX) || kCountThreads % (j.TY / j.VY)) return false;
+      j.nt = c.block;
+      if (c.tiled.form == kTileShort) return j.TY <= kSkewRows;
+      if (c.tiled.form != kTileRect && j.TX > kMaxSkewTile) return false;
+      if (c.tiled.form == kTileSkew && j.TY + 128 / j.B > kSkewRows) return false;
+      if (c.tiled.form == kTileNarrow) return c.tiled.yg.n == 1;
+      if (j.TX % j.VX || j.TY % j.VY || j.nt % (j.TX / j.VX) || j.nt % (j.TY / j.VY)) return false;
       return job_passes(j, 0) >= 1 && job_passes(j, 1) >= 1;
     case kTiledCopy:
       j.B = c.elem;
+      j.nt = c.block;
       if (c.copy.per != kCountThreads * (16 / j.B) || c.copy.X < 2) return false;
       j.a.copy = c.copy;
       j.items = c.copy.items;
@@ -437,7 +576,7 @@ bool make_job(const Candidate& c, CountJob& j, std::vector<int>& runs) {
 // enumeration, and returns the per-instruction counts through `acc`.
 template <class F>
 void host_walk(const CountJob& j, unsigned long long* acc, F&& f) {
-  const int nthreads = job_threads(j);
+  const int nthreads = j.nt;
   const int waves = (nthreads + 63) / 64;
   bool act[64];
   long long off[64];

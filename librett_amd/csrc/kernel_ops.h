@@ -97,6 +97,15 @@ __host__ __device__ inline V ld_unaligned(const void* p) {
 #endif
 }
 
+// At both ends of a branch that loads non-temporally what the other branch loads
+// temporally: without it the compiler merges the two into one temporal load
+// (8192 x 8192 f32 93 us instead of 85).
+__host__ __device__ inline void keep_branch() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" ::: "memory");
+#endif
+}
+
 // Elements between the last 128-byte line boundary and p (p a multiple of
 // the element size).
 template <typename E>
@@ -110,6 +119,29 @@ struct TileCtx {
   bool full;
 };
 
+// Tile w of a Tiled plan with tiles of tx_size x ty_size elements.
+__host__ __device__ inline TileCtx tile_item(const TiledArgs& a, uint32_t w, int tx_size, int ty_size) {
+  TileCtx c;
+  const uint32_t mb = fdiv(w, a.ntiles_div);
+  const uint32_t tile = w - mb * (uint32_t)a.ntiles;
+  uint32_t tx, ty;
+  if (a.group <= 1) {
+    ty = fdiv(tile, a.ntx_div);
+    tx = tile - ty * (uint32_t)a.ntx;
+  } else {
+    const uint32_t g = fdiv(tile, a.group_row_div);  // group index
+    const uint32_t within = tile - g * a.group_row_div.d;
+    const FastDiv& rows = (tile >= (uint32_t)a.last_group_start) ? a.last_div : a.group_div;
+    tx = fdiv(within, rows);
+    ty = g * (uint32_t)a.group + (within - tx * rows.d);
+  }
+  c.x0 = (int)tx * tx_size;
+  c.y0 = (int)ty * ty_size;
+  outer_offsets(a.outer, mb, c.off_in, c.off_out);
+  c.full = (c.x0 + tx_size <= a.X) && (c.y0 + ty_size <= a.Y);
+  return c;
+}
+
 // ---------------------------------------------------------------------------
 // Tiled: a TX x TY tile of the (x, y) plane goes through LDS. Reads walk x
 // (contiguous in the input) with VX elements per lane; writes walk y
@@ -118,6 +150,11 @@ struct TileCtx {
 // When x or y is a group of dims, each row (column) finds its offset on the
 // other side from the group's digits; a full tile of one-dim groups steps
 // through memory by a fixed stride instead.
+// Bound by HBM. One workgroup moves one tile and ends: a loop over tiles kept
+// 106 SGPRs and up to 20 more VGPRs alive (34 SGPRs without it), and the
+// dispatcher's order keeps neighbouring tiles closer in time than a stride
+// over the grid does ([2, 8, 16, 32, 64, 128] f32 95 -> 85 us with the loads
+// non-temporal too; a copy of the bytes takes 85 us).
 // Reference counterpart: transposeTiled, src/kernel.cpp:48-170.
 // ---------------------------------------------------------------------------
 // G = false compiles only the one-dim-group path (the kernel then needs no
@@ -127,7 +164,10 @@ struct TiledOps {
   using E = typename Word<B>::type;
   using VI = typename Word<B * VX>::type;
   using VO = typename Word<B * VY>::type;
-  static constexpr int NT = 256;
+  // 128 x 128 tiles take 512 threads: with 256, two workgroups of 66 KiB of LDS
+  // leave a CU 8 waves (8192 x 8192 f32 on MI355X: 104 us; with 512, 95 us, and
+  // 85 us with one tile per workgroup and non-temporal loads as well).
+  static constexpr int NT = TX * TY >= 128 * 128 ? 512 : 256;
   static constexpr int LR = TX / VX;   // lanes per input row
   static constexpr int RP = NT / LR;   // input rows per pass
   static constexpr int NPR = TY / RP;  // read passes
@@ -166,68 +206,55 @@ struct TiledOps {
     }
   }
 
-  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) {
-    TileCtx c;
-    uint32_t mb = fdiv(w, a.ntiles_div);
-    uint32_t tile = w - mb * (uint32_t)a.ntiles;
-    uint32_t tx, ty;
-    if (a.group <= 1) {
-      ty = fdiv(tile, a.ntx_div);
-      tx = tile - ty * (uint32_t)a.ntx;
-    } else {
-      const uint32_t g = fdiv(tile, a.group_row_div);  // group index
-      const uint32_t within = tile - g * a.group_row_div.d;
-      const FastDiv& rows = (tile >= (uint32_t)a.last_group_start) ? a.last_div : a.group_div;
-      tx = fdiv(within, rows);
-      ty = g * (uint32_t)a.group + (within - tx * rows.d);
-    }
-    c.x0 = (int)tx * TX;
-    c.y0 = (int)ty * TY;
-    outer_offsets(a.outer, mb, c.off_in, c.off_out);
-    c.full = (c.x0 + TX <= a.X) && (c.y0 + TY <= a.Y);
-    return c;
-  }
+  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) { return tile_item(a, w, TX, TY); }
 
+  // LARGE: whole tiles are loaded non-temporally where the plan asks for it.
+  template <bool LARGE = false>
   __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t,
                                        const E* __restrict__ in, E* lds) {
     VI r[NPR];
-    fetch(a, c, t, in, r, lds);
-    stash(a, c, t, r, lds);
-  }
-
-  // The two halves of load(): the tile's input rows into registers, then
-  // registers into LDS (the pipelined kernel fetches the next tile between
-  // them and the current tile's store phase).
-  __host__ __device__ static void fetch(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in,
-                                        VI* r, const E* lds) {
     const int lx = (t % LR) * VX;
     const int ly = t / LR;
     const int x = c.x0 + lx;
     if (c.full && (!G || a.yg.n == 1)) {
       const E* p = in + (c.off_in + x + (c.y0 + ly) * a.in_ys);
       const int step = RP * a.in_ys;
+      if (LARGE && a.stream_in) {
+        keep_branch();
 #pragma unroll
-      for (int j = 0; j < NPR; j++) r[j] = ld(reinterpret_cast<const VI*>(p + j * step));
+        for (int j = 0; j < NPR; j++) r[j] = ld<true>(reinterpret_cast<const VI*>(p + j * step));
+        keep_branch();
+      } else {
+#pragma unroll
+        for (int j = 0; j < NPR; j++) r[j] = ld(reinterpret_cast<const VI*>(p + j * step));
+      }
+    } else if (G && LARGE && c.full && a.stream_in) {
+      keep_branch();
+      const E* p = in + (c.off_in + x);
+#pragma unroll
+      for (int j = 0; j < NPR; j++) r[j] = ld<true>(reinterpret_cast<const VI*>(p + offsets(lds)[ly + j * RP]));
+      keep_branch();
     } else {
       const bool xin = x < a.X;
 #pragma unroll
       for (int j = 0; j < NPR; j++) {
         const int y = c.y0 + ly + j * RP;
         const int yoff = G ? offsets(lds)[ly + j * RP] : y * a.in_ys;
+        r[j] = VI{};
         if (xin && y < a.Y) r[j] = ld(reinterpret_cast<const VI*>(in + (c.off_in + x + yoff)));
       }
     }
+    stash(t, r, lds);
   }
-  __host__ __device__ static void stash(const TiledArgs& a, const TileCtx& c, int t, const VI* r, E* lds) {
+
+  // Rows and columns past the plane are stored too, and not read: no masks.
+  __host__ __device__ static void stash(int t, const VI* r, E* lds) {
     const int lx = (t % LR) * VX;
     const int ly = t / LR;
-    const bool xin = c.x0 + lx < a.X;
 #pragma unroll
     for (int j = 0; j < NPR; j++) {
-      if (c.full || (xin && c.y0 + ly + j * RP < a.Y)) {
 #pragma unroll
-        for (int e = 0; e < VX; e++) lds[(ly + j * RP) * PITCH + lx + e] = vget<E>(r[j], e);
-      }
+      for (int e = 0; e < VX; e++) lds[(ly + j * RP) * PITCH + lx + e] = vget<E>(r[j], e);
     }
   }
 
@@ -253,6 +280,350 @@ struct TiledOps {
         const int x = c.x0 + lx + j * WP;
         const int xoff = G ? offsets(lds)[TY + lx + j * WP] : x * a.out_xs;
         if (yin && x < a.X) st(reinterpret_cast<VO*>(out + (c.off_out + y + xoff)), r[j]);
+      }
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
+// Skewed tiles, for planes whose output columns do not all start on 128-byte
+// lines. Column x of a tile covers the TY rows that start at y0 - s(x), where
+// s(x) is how far output row y0 of that column lies past a line boundary, so
+// every store is an aligned 16-byte word and a tile writes whole lines; only
+// a column's own first and last line are written in part. The tile's LDS holds
+// LE (a line's elements) more rows than TY, of which each column uses its TY;
+// each lane loads just the rows of its column, so no element is loaded twice.
+// Bound by HBM. What it removes: lines written in two halves by two
+// workgroups (1.06 x the bytes in DRAM writes, but each partial line costs a
+// read-modify-write there). On MI355X, against unskewed tiles with their best
+// lanes: (8191, 8193) f32 130 -> 94 us, (4097, 8191) f64 122 -> 94 us,
+// (5, 97, 211, 331) f64 131 -> 105 us; a copy of the bytes takes 85 us.
+// One-element loads are as fast as 16-byte ones here (93-95 against 93 us,
+// f32), and non-temporal loads slower (106 us), as neighbouring tiles share
+// the lines of the rows they split. Tiles aligned to 64 bytes instead of 128
+// cost 5-10%.
+// ---------------------------------------------------------------------------
+template <int B, int TX, int TY, int NTH, bool G>
+struct SkewOps {
+  using E = typename Word<B>::type;
+  using V = typename Word<16>::type;
+  static constexpr int NT = NTH;
+  static constexpr int LE = 128 / B;               // elements per line
+  static constexpr int PE = 16 / B;                // elements per output word
+  static constexpr int R = TY + LE;                // tile rows held in LDS: row i is y0 - LE + i
+  static constexpr int RP = NT / TX;               // rows per load pass
+  static constexpr int NPR = (R + RP - 1) / RP;    // load passes
+  static constexpr int LW = TY / PE;               // lanes per output column
+  static constexpr int WP = NT / LW;               // columns per store pass
+  static constexpr int NPW = TX / WP;              // store passes
+  static constexpr int PITCH = TX + 1;
+  // After the tile, ints: R input offsets of the rows (G), TX output offsets
+  // of the columns (G).
+  static constexpr int OFF_ELEMS = G ? ((R + TX) * 4 + B - 1) / B : 0;
+  static constexpr int LDS_ELEMS = R * PITCH + OFF_ELEMS;
+  static_assert(R + TX <= NT && NT % TX == 0 && TY % PE == 0 && NT % LW == 0 && TX % WP == 0 && NPW >= 1, "skew shape");
+
+  __host__ __device__ static int* offsets(E* lds) { return reinterpret_cast<int*>(lds + R * PITCH); }
+  __host__ __device__ static const int* offsets(const E* lds) {
+    return reinterpret_cast<const int*>(lds + R * PITCH);
+  }
+
+  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) { return tile_item(a, w, TX, TY); }
+
+  // G only, as in TiledOps: prepare() with a barrier before load() where the y
+  // group has several dims; else only the columns' output offsets are needed,
+  // by store().
+  __host__ __device__ static bool early(const TiledArgs& a) { return G && a.yg.n > 1; }
+  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx& c, int t, E* lds) {
+    int* o = offsets(lds);
+    if (t < R) {
+      const int y = c.y0 - LE + t;
+      o[t] = y >= 0 && y < a.Y ? tiled_in_y(a, (uint32_t)y) : 0;
+    } else if (t < R + TX) {
+      const int x = c.x0 + (t - R);
+      o[t] = x < a.X ? tiled_out_x(a, (uint32_t)x) : 0;
+    }
+  }
+
+  // Output offset of tile column i, and its skew.
+  __host__ __device__ static int column(const TiledArgs& a, const TileCtx& c, int i, const E* lds) {
+    return c.off_out + (G ? offsets(lds)[R + i] : (c.x0 + i) * a.out_xs);
+  }
+  __host__ __device__ static int skew(int base, int phase) { return (base + phase) & (LE - 1); }
+
+  // Tile rows [lo, hi) that a column with skew s covers.
+  __host__ __device__ static void rows(const TiledArgs& a, const TileCtx& c, int s, int& lo, int& hi) {
+    const int first = LE - c.y0, end = a.Y - c.y0 + LE;  // rows of y = 0 and y = Y
+    lo = LE - s > first ? LE - s : first;
+    hi = LE - s + TY < end ? LE - s + TY : end;
+  }
+
+  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
+                                       int phase) {
+    const int lx = t % TX;
+    const int ly = t / TX;
+    int lo = 0, hi = 0;
+    const int x = c.x0 + lx;
+    if (x < a.X) rows(a, c, skew(c.off_out + (G ? tiled_out_x(a, (uint32_t)x) : x * a.out_xs), phase), lo, hi);
+    const E* p = in + (c.off_in + c.x0 + lx);
+    const int y = c.y0 - LE + ly;
+    E r[NPR];
+#pragma unroll
+    for (int j = 0; j < NPR; j++) {
+      const int i = ly + j * RP;
+      r[j] = E{};
+      if (i >= lo && i < hi) r[j] = ld(p + (early(a) ? offsets(lds)[i] : (y + j * RP) * a.in_ys));
+    }
+    if (G && !early(a) && t < TX && c.x0 + t < a.X) offsets(lds)[R + t] = tiled_out_x(a, (uint32_t)(c.x0 + t));
+    // Rows of the tile that the column does not cover are stored too (and not
+    // read): the lanes' masks then need no registers until here.
+#pragma unroll
+    for (int j = 0; j < NPR; j++) {
+      const int i = ly + j * RP;
+      if (RP * NPR == R || i < R) lds[i * PITCH + lx] = r[j];
+    }
+  }
+
+  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t, E* __restrict__ out,
+                                        const E* lds, int phase) {
+    const int ly = (t % LW) * PE;
+    const int lx = t / LW;
+#pragma unroll
+    for (int j = 0; j < NPW; j++) {
+      const int i = lx + j * WP;
+      if (c.x0 + i >= a.X) continue;
+      const int base = column(a, c, i, lds);
+      const int s = skew(base, phase);
+      const int y = c.y0 - s + ly;
+      const E* q = lds + ((LE - s + ly) * PITCH + i);
+      if (y >= 0 && y + PE <= a.Y) {
+        V v;
+#pragma unroll
+        for (int k = 0; k < PE; k++) vset<E>(v, k, q[k * PITCH]);
+        st(reinterpret_cast<V*>(out + (base + y)), v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < PE; k++)
+          if (y + k >= 0 && y + k < a.Y) st(out + (base + y + k), q[k * PITCH]);
+      }
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
+// Narrow planes: X is at most kNarrowX columns and the rows lie back to back in
+// the input (in_ys == X, y the input dim after x), as in an array of
+// structures that becomes a structure of arrays. A tile is all X columns of TY
+// rows: one contiguous stretch of the input, dealt to the threads element by
+// element whatever X is, and X long runs of the output, skewed as in SkewOps.
+// Bound by HBM. On MI355X, [7, 9587595] f32 takes 134 us as a Packed plan of
+// 10381 elements, which writes its lines in parts, 92 us here; [5, 6710040]
+// f64 118 -> 92 us, [2, 13107201] f64 288 -> 70 us; copies of the bytes take
+// 85, 85 and 66 us. Tiles are small (8 to 16 KiB) for 7 workgroups on a CU: of
+// 28 KiB with 512 threads, whose registers leave two, 113 us for the first.
+// ---------------------------------------------------------------------------
+template <int B, int NTH, int NL>
+struct NarrowOps {
+  using E = typename Word<B>::type;
+  using V = typename Word<16>::type;
+  static constexpr int NT = NTH;
+  static constexpr int LE = 128 / B;
+  static constexpr int PE = 16 / B;
+  static constexpr int MAX = NT * NL;  // elements of a tile, with its line more of rows
+  static constexpr int NW = (NL + PE - 1) / PE;  // store passes
+
+  // LDS: rows of odd pitch, then X output offsets of the columns.
+  __host__ __device__ static int pitch(const TiledArgs& a) { return a.X | 1; }
+  __host__ __device__ static int rows(const TiledArgs& a) { return (PE << a.word_shift) + LE; }
+  __host__ __device__ static int* offsets(const TiledArgs& a, E* lds) {
+    return reinterpret_cast<int*>(lds + rows(a) * pitch(a));
+  }
+  __host__ __device__ static const int* offsets(const TiledArgs& a, const E* lds) {
+    return reinterpret_cast<const int*>(lds + rows(a) * pitch(a));
+  }
+
+  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) {
+    return tile_item(a, w, a.X, PE << a.word_shift);
+  }
+
+  // Before load(), with a barrier between.
+  __host__ __device__ static constexpr bool early(const TiledArgs&) { return true; }
+  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx& c, int t, E* lds) {
+    if (t < a.X) offsets(a, lds)[t] = c.off_out + tiled_out_x(a, (uint32_t)t);
+  }
+
+  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
+                                       int phase) {
+    const int ty = PE << a.word_shift;
+    const int n = (ty + LE) * a.X;
+    // Element i of the tile lies i elements past row y0 - LE of the plane;
+    // elements [lo, hi) are in the plane.
+    const E* p = in + c.off_in;
+    const int p0 = (c.y0 - LE) * a.X;
+    const int lo = p0 < 0 ? -p0 : 0;
+    const long long left = (long long)a.Y * a.X - p0;
+    const int hi = n < left ? n : (int)left;
+    E r[NL];
+#pragma unroll
+    for (int j = 0; j < NL; j++) {
+      const int i = t + j * NT;
+      r[j] = E{};
+      bool use = i >= lo && i < hi;
+      // Only the first and last line's elements of rows depend on the column's
+      // skew.
+      if (use && (i < LE * a.X || i >= ty * a.X)) {
+        const int row = (int)fdiv((uint32_t)i, a.x_div);
+        const int d = row - LE + ((offsets(a, lds)[i - row * a.X] + phase) & (LE - 1));
+        use = d >= 0 && d < ty;
+      }
+      if (use) r[j] = ld(p + (p0 + i));
+    }
+    // An odd pitch X is the input's own layout.
+    if (a.X & 1) {
+#pragma unroll
+      for (int j = 0; j < NL; j++)
+        if (t + j * NT < n) lds[t + j * NT] = r[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < NL; j++) {
+        const int i = t + j * NT;
+        if (i < n) lds[i + (int)fdiv((uint32_t)i, a.x_div)] = r[j];
+      }
+    }
+  }
+
+  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t, E* __restrict__ out,
+                                        const E* lds, int phase) {
+    const int* off = offsets(a, lds);
+    const int P = pitch(a);
+    const int nw = a.X << a.word_shift;
+#pragma unroll
+    for (int j = 0; j < NW; j++) {
+      const int i = t + j * NT;
+      if (i >= nw) break;
+      const int x = i >> a.word_shift;
+      const int ly = (i - (x << a.word_shift)) * PE;
+      const int base = off[x];
+      const int s = (base + phase) & (LE - 1);
+      const int y = c.y0 - s + ly;
+      const E* q = lds + ((LE - s + ly) * P + x);
+      if (y >= 0 && y + PE <= a.Y) {
+        V v;
+#pragma unroll
+        for (int k = 0; k < PE; k++) vset<E>(v, k, q[k * P]);
+        st(reinterpret_cast<V*>(out + (base + y)), v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < PE; k++)
+          if (y + k >= 0 && y + k < a.Y) st(out + (base + y + k), q[k * P]);
+      }
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
+// Short columns: Y is at most kNarrowX elements and the columns lie back to back
+// in the output (out_xs == Y, x the output dim after y), as in a structure of
+// arrays that becomes an array of structures: NarrowOps the other way round. A
+// tile is a stretch of CH output elements that starts on a line; it reads a run
+// of each of the Y input rows and writes whole 16-byte words. Bound by HBM. On
+// MI355X, against the best other plan: [26000000, 2] f32 455 -> 72 us,
+// [13000000, 2] f64 315 -> 70 us; copies of the bytes take 66 us.
+// ---------------------------------------------------------------------------
+template <int B, int NTH, int NL>
+struct ShortOps {
+  using E = typename Word<B>::type;
+  using V = typename Word<16>::type;
+  static constexpr int NT = NTH;
+  static constexpr int LE = 128 / B;
+  static constexpr int PE = 16 / B;
+  static constexpr int NW = NL / PE;        // 16-byte words per thread
+  static constexpr int CH = NT * NW * PE;   // elements of a tile
+  static_assert(NL % PE == 0 && CH % LE == 0, "short shape");
+  // Columns of a tile whose first and last may be cut; loads per thread.
+  __host__ __device__ static int columns(int Y) { return (CH + Y - 2) / Y + 1; }
+  static constexpr int NLD = NL + 1;  // columns(Y) * Y <= CH + 2 * Y <= (NL + 1) * NT
+
+  __host__ __device__ static int pitch(const TiledArgs& a) { return (int)a.nx_div.d | 1; }
+  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) {
+    TileCtx c;
+    const uint32_t mb = fdiv(w, a.ntiles_div);
+    c.x0 = (int)(w - mb * (uint32_t)a.ntiles);  // tile of the plane
+    c.y0 = 0;
+    outer_offsets(a.outer, mb, c.off_in, c.off_out);
+    c.full = false;
+    return c;
+  }
+  // First element of the tile, counted from the plane's first output element.
+  __host__ __device__ static int first(const TileCtx& c, int phase) {
+    return c.x0 * CH - ((c.off_out + phase) & (LE - 1));
+  }
+  // Before load(), with a barrier between.
+  __host__ __device__ static constexpr bool early(const TiledArgs&) { return true; }
+  // After the tile's Y rows, their input offsets (ints).
+  __host__ __device__ static const int* offsets(const TiledArgs& a, const E* lds) {
+    return reinterpret_cast<const int*>(lds + a.Y * pitch(a));
+  }
+  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx&, int t, E* lds) {
+    if (t < a.Y) const_cast<int*>(offsets(a, lds))[t] = tiled_in_y(a, (uint32_t)t);
+  }
+
+  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
+                                       int phase) {
+    const int e0 = first(c, phase), n = a.X * a.Y;
+    const uint32_t lo = e0 < 0 ? 0 : (uint32_t)e0;
+    const uint32_t hi = (long long)n - e0 < CH ? (uint32_t)n : (uint32_t)(e0 + CH);
+    const int xa = (int)fdiv(lo, a.x_div);
+    const E* p = in + (c.off_in + xa);
+    const int* off = offsets(a, lds);
+    E r[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; j++) {
+      const uint32_t i = (uint32_t)(t + j * NT);
+      const int y = (int)fdiv(i, a.nx_div);
+      const int xi = (int)(i - (uint32_t)y * a.nx_div.d);
+      const uint32_t e = (uint32_t)(xa + xi) * (uint32_t)a.Y + (uint32_t)y;
+      r[j] = E{};
+      if (y < a.Y && e >= lo && e < hi) r[j] = ld(p + (xi + off[y]));
+    }
+#pragma unroll
+    for (int j = 0; j < NLD; j++) {
+      const uint32_t i = (uint32_t)(t + j * NT);
+      const int y = (int)fdiv(i, a.nx_div);
+      if (y < a.Y) lds[y * pitch(a) + (int)(i - (uint32_t)y * a.nx_div.d)] = r[j];
+    }
+  }
+
+  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t, E* __restrict__ out,
+                                        const E* lds, int phase) {
+    const int e0 = first(c, phase);
+    const uint32_t n = (uint32_t)(a.X * a.Y);
+    const int xa = (int)fdiv((uint32_t)(e0 < 0 ? 0 : e0), a.x_div);
+    const int P = pitch(a);
+#pragma unroll
+    for (int j = 0; j < NW; j++) {
+      // Elements before the plane wrap to values above any volume.
+      const uint32_t e = (uint32_t)e0 + (uint32_t)((t + j * NT) * PE);
+      if (e < n && n - e >= (uint32_t)PE) {
+        int x = (int)fdiv(e, a.x_div);
+        int y = (int)e - x * a.Y;
+        V v;
+#pragma unroll
+        for (int k = 0; k < PE; k++) {
+          vset<E>(v, k, lds[y * P + (x - xa)]);
+          if (++y == a.Y) {
+            y = 0;
+            x++;
+          }
+        }
+        st(reinterpret_cast<V*>(out + (c.off_out + (int)e)), v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < PE; k++)
+          if (e + k < n) {
+            const int x = (int)fdiv(e + k, a.x_div);
+            st(out + (c.off_out + (int)(e + k)), lds[((int)(e + k) - x * a.Y) * P + (x - xa)]);
+          }
       }
     }
   }
@@ -286,10 +657,13 @@ struct CopyOps {
   // 16-byte boundaries of the output's addresses, and items start on lines.
   __host__ __device__ static void run(const CopyArgs& a, uint32_t w, int t, const E* __restrict__ in,
                                       E* __restrict__ out) {
-    if (a.stream_in)
+    if (a.stream_in) {
+      keep_branch();
       move<true>(a, w, t, in, out);
-    else
+      keep_branch();
+    } else {
       move<false>(a, w, t, in, out);
+    }
   }
 
   template <bool STREAM>
@@ -300,7 +674,7 @@ struct CopyOps {
       V r;
       const uint32_t row = fdiv(e, a.row_div);
       const int c = (int)(e - row * (uint32_t)a.X);
-      if (a.X - c >= PE) {
+      if (PE == 1 || a.X - c >= PE) {
         r = ld_unaligned<V, B, STREAM>(in + (copy_row_offset(a.rows, row) + c));
       } else {
 #pragma unroll

@@ -35,7 +35,12 @@ bool tiled_shape_available(int elem, int tx, int ty, int vx, int vy, bool genera
 // Shapes the batched engine's kernel is instantiated for (batch.hip).
 bool batch_tiled_available(int elem, int tx, int ty, int vx, int vy, bool general = false);
 bool batch_packed_available(int elem, int nreg);
+bool batch_skew_available(int elem, int tx, int ty);
 int packed_max_nreg(int elem);
 bool packed_nreg_available(int elem, int nreg);
+// Threads of the narrow (short) Tiled kernel and the most elements its tiles hold.
+void narrow_shape(int elem, int form, int& threads, int& elements);
+// Threads of the Tiled kernel for a tile of tx x ty elements.
+int tiled_threads(int tx, int ty);
 
 }  // namespace lrt

@@ -39,31 +39,79 @@ namespace lrt {
 // Device kernels
 // ---------------------------------------------------------------------------
 
-// k_tiled walks its tiles with a stride of the grid, one LDS round per
-// tile. (Fetching the next tile into registers during the current tile's
-// store phase, as k_packed does for its large rounds, measured slower on
-// MI355X: 2-3% on the 8192 x 8192 planes and far slower on tiles whose
-// registers then cut occupancy, so Tiled rounds are not pipelined.)
+// The Tiled kernels run one tile per workgroup and leave it to the dispatcher
+// to keep the CUs filled: a loop over tiles holds both group maps in registers
+// between tiles (106 SGPRs and spills in the group kernels). (Fetching
+// the next tile into registers during the current tile's store phase, as
+// k_packed does for its large rounds, measured slower on MI355X: 2-3% on the
+// 8192 x 8192 planes and far slower on tiles whose registers then cut
+// occupancy.)
+// The tile of this workgroup, -1 past the last one. The grid has two dims only
+// because one dim holds at most 2^32 threads.
+__device__ __forceinline__ int tile_of(const TiledArgs& a) {
+  const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+  if (b >= (uint32_t)a.items) return -1;
+  return a.xcds > 1 ? xcd_logical((int)b, a.items, a.xcds) : (int)b;
+}
+
 template <int B, int TX, int TY, int VX, int VY, bool G>
-__global__ __launch_bounds__(256) void k_tiled(TiledArgs a, const void* __restrict__ in,
-                                               void* __restrict__ out) {
+__global__ __launch_bounds__((TiledOps<B, TX, TY, VX, VY, G>::NT)) void k_tiled(TiledArgs a,
+                                                                                 const void* __restrict__ in,
+                                                                                 void* __restrict__ out) {
   using Ops = TiledOps<B, TX, TY, VX, VY, G>;
   using E = typename Ops::E;
   __shared__ E lds[Ops::LDS_ELEMS];
   const E* src = static_cast<const E*>(in);
   E* dst = static_cast<E*>(out);
-  const uint32_t w0 = a.xcds > 1 ? (uint32_t)xcd_logical((int)blockIdx.x, (int)gridDim.x, a.xcds) : blockIdx.x;
-  for (uint32_t w = w0; w < (uint32_t)a.items; w += gridDim.x) {
-    const TileCtx c = Ops::item(a, w);
-    if constexpr (G) {
-      Ops::prepare(a, c, threadIdx.x, lds);
-      __syncthreads();
-    }
-    Ops::load(a, c, threadIdx.x, src, lds);
-    __syncthreads();
-    Ops::store(a, c, threadIdx.x, dst, lds);
+  const int w = tile_of(a);
+  if (w < 0) return;
+  const TileCtx c = Ops::item(a, (uint32_t)w);
+  if constexpr (G) {
+    Ops::prepare(a, c, threadIdx.x, lds);
     __syncthreads();
   }
+  Ops::template load<true>(a, c, threadIdx.x, src, lds);
+  __syncthreads();
+  Ops::store(a, c, threadIdx.x, dst, lds);
+}
+
+template <int B, int TX, int TY, int NT, bool G>
+__global__ __launch_bounds__(NT) void k_skew(TiledArgs a, const void* __restrict__ in, void* __restrict__ out) {
+  using Ops = SkewOps<B, TX, TY, NT, G>;
+  using E = typename Ops::E;
+  __shared__ E lds[Ops::LDS_ELEMS];
+  const E* src = static_cast<const E*>(in);
+  E* dst = static_cast<E*>(out);
+  const int phase = line_phase(dst);
+  const int w = tile_of(a);
+  if (w < 0) return;
+  const TileCtx c = Ops::item(a, (uint32_t)w);
+  if (Ops::early(a)) {
+    Ops::prepare(a, c, threadIdx.x, lds);
+    __syncthreads();
+  }
+  Ops::load(a, c, threadIdx.x, src, lds, phase);
+  __syncthreads();
+  Ops::store(a, c, threadIdx.x, dst, lds, phase);
+}
+
+// Ops: NarrowOps or ShortOps.
+template <class Ops>
+__global__ __launch_bounds__(Ops::NT) void k_narrow(TiledArgs a, const void* __restrict__ in, void* __restrict__ out) {
+  using E = typename Ops::E;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  E* lds = reinterpret_cast<E*>(smem);
+  const E* src = static_cast<const E*>(in);
+  E* dst = static_cast<E*>(out);
+  const int phase = line_phase(dst);
+  const int w = tile_of(a);
+  if (w < 0) return;
+  const TileCtx c = Ops::item(a, (uint32_t)w);
+  Ops::prepare(a, c, threadIdx.x, lds);
+  __syncthreads();
+  Ops::load(a, c, threadIdx.x, src, lds, phase);
+  __syncthreads();
+  Ops::store(a, c, threadIdx.x, dst, lds, phase);
 }
 
 // One item per workgroup.
@@ -224,6 +272,29 @@ static void replay_tiled(const Candidate& c, const void* in, void* out) {
   }
 }
 
+template <class Ops>
+static void replay_skew(const Candidate& c, const void* in, void* out) {
+  using E = typename Ops::E;
+  std::vector<E> lds((size_t)c.lds_bytes / sizeof(E) + 1);
+  const TiledArgs& a = c.tiled;
+  const E* src = static_cast<const E*>(in);
+  E* dst = static_cast<E*>(out);
+  const int phase = line_phase(dst);
+  for (uint32_t w = 0; w < (uint32_t)a.items; w++) {
+    const TileCtx ctx = Ops::item(a, w);
+    if (Ops::early(a))
+      for (int t = 0; t < Ops::NT; t++) Ops::prepare(a, ctx, t, lds.data());
+    for (int t = 0; t < Ops::NT; t++) {
+      replay_at(w, t);
+      Ops::load(a, ctx, t, src, lds.data(), phase);
+    }
+    for (int t = 0; t < Ops::NT; t++) {
+      replay_at(w, t);
+      Ops::store(a, ctx, t, dst, lds.data(), phase);
+    }
+  }
+}
+
 template <int B>
 static void replay_copy(const Candidate& c, const void* in, void* out) {
   using Ops = CopyOps<B>;
@@ -365,6 +436,40 @@ static const TiledEntry kTiledTable[] = {
     LRT_TILED_G(16, 16, 16, 1, 1, true) LRT_TILED_G(16, 32, 32, 1, 1, true)
 };
 
+struct SkewEntry {
+  int b, tx, ty, nt;
+  bool general;
+  const void* kernel;
+  void (*replay)(const Candidate&, const void*, void*);
+};
+
+#define LRT_SKEW_G(B, TX, TY, NT, G) \
+  {B, TX, TY, NT, G, reinterpret_cast<const void*>(&k_skew<B, TX, TY, NT, G>), &replay_skew<SkewOps<B, TX, TY, NT, G>>},
+#define LRT_SKEW(B, TX, TY, NT) LRT_SKEW_G(B, TX, TY, NT, false) LRT_SKEW_G(B, TX, TY, NT, true)
+
+static const SkewEntry kSkewTable[] = {
+    LRT_SKEW(4, 64, 128, 512) LRT_SKEW(4, 64, 64, 256) LRT_SKEW(4, 32, 128, 256) LRT_SKEW(4, 32, 64, 256)
+    LRT_SKEW(8, 64, 64, 512) LRT_SKEW(8, 32, 64, 256) LRT_SKEW(8, 32, 128, 512) LRT_SKEW(8, 32, 32, 256)
+    LRT_SKEW(16, 32, 32, 256) LRT_SKEW(16, 32, 64, 512) LRT_SKEW(16, 16, 32, 256) LRT_SKEW(16, 32, 16, 256)
+};
+
+// Narrow planes and short columns: threads, and the most elements of a tile.
+struct NarrowEntry {
+  int b;
+  TileForm form;
+  int nt, elements;
+  const void* kernel;
+  void (*replay)(const Candidate&, const void*, void*);
+};
+#define LRT_NARROW(B, NT, NL)                                                                                \
+  {B, kTileNarrow, NT, NarrowOps<B, NT, NL>::MAX, reinterpret_cast<const void*>(&k_narrow<NarrowOps<B, NT, NL>>), \
+   &replay_skew<NarrowOps<B, NT, NL>>},
+#define LRT_SHORT(B, NT, NL)                                                                             \
+  {B, kTileShort, NT, ShortOps<B, NT, NL>::CH, reinterpret_cast<const void*>(&k_narrow<ShortOps<B, NT, NL>>), \
+   &replay_skew<ShortOps<B, NT, NL>>},
+static const NarrowEntry kNarrowTable[] = {LRT_NARROW(4, 256, 8) LRT_NARROW(8, 256, 6) LRT_NARROW(16, 256, 4)
+                                           LRT_SHORT(4, 256, 8) LRT_SHORT(8, 256, 6) LRT_SHORT(16, 256, 4)};
+
 #define LRT_COPY(B) {B, reinterpret_cast<const void*>(&k_copy<B>), &replay_copy<B>},
 
 static const CopyEntry kCopyTable[] = {LRT_COPY(4) LRT_COPY(8) LRT_COPY(16)};
@@ -388,6 +493,17 @@ static const TiledEntry* find_tiled(const Candidate& c) {
       return &e;
   return nullptr;
 }
+static const SkewEntry* find_skew(const Candidate& c) {
+  const bool general = c.xgroup > 1 || c.ygroup > 1;
+  for (const auto& e : kSkewTable)
+    if (e.b == c.elem && e.tx == c.tile_x && e.ty == c.tile_y && e.nt == c.block && e.general == general) return &e;
+  return nullptr;
+}
+static const NarrowEntry* find_narrow(int elem, int form) {
+  for (const auto& e : kNarrowTable)
+    if (e.b == elem && e.form == form) return &e;
+  return nullptr;
+}
 static const CopyEntry* find_copy(const Candidate& c) {
   for (const auto& e : kCopyTable)
     if (e.b == c.elem) return &e;
@@ -404,6 +520,12 @@ bool tiled_shape_available(int elem, int tx, int ty, int vx, int vy, bool genera
     if (e.b == elem && e.tx == tx && e.ty == ty && e.vx == vx && e.vy == vy && e.general == general) return true;
   return false;
 }
+void narrow_shape(int elem, int form, int& threads, int& elements) {
+  const NarrowEntry* e = find_narrow(elem, form);
+  threads = e->nt;
+  elements = e->elements;
+}
+int tiled_threads(int tx, int ty) { return tx * ty >= 128 * 128 ? 512 : 256; }
 int packed_max_nreg(int elem) {
   int m = 0;
   for (const auto& e : kPackedTable)
@@ -419,6 +541,11 @@ bool packed_nreg_available(int elem, int nreg) {
 static const void* kernel_of(const Candidate& c) {
   switch (c.method) {
     case kTiled: {
+      if (const NarrowEntry* e = find_narrow(c.elem, c.tiled.form)) return e->kernel;
+      if (c.tiled.form == kTileSkew) {
+        const SkewEntry* e = find_skew(c);
+        return e ? e->kernel : nullptr;
+      }
       const TiledEntry* e = find_tiled(c);
       return e ? e->kernel : nullptr;
     }
@@ -434,6 +561,11 @@ static const void* kernel_of(const Candidate& c) {
     default:
       return nullptr;
   }
+}
+
+// Kernels whose LDS is sized at launch.
+static bool dynamic_lds(const Candidate& c) {
+  return c.method == kPacked || c.method == kPackedSplit || (c.method == kTiled && c.tiled.form >= kTileNarrow);
 }
 
 hipError_t launch_candidate(const Candidate& c, const void* in, void* out, hipStream_t stream) {
@@ -458,8 +590,7 @@ hipError_t launch_candidate(const Candidate& c, const void* in, void* out, hipSt
   }
   args[1] = &in;
   args[2] = &out;
-  return hipLaunchKernel(k, grid, block, args, (size_t)((c.method == kPacked || c.method == kPackedSplit) ? c.lds_bytes : 0),
-                         stream);
+  return hipLaunchKernel(k, grid, block, args, (size_t)(dynamic_lds(c) ? c.lds_bytes : 0), stream);
 }
 
 bool replay_candidate(const Candidate& c, const void* in, void* out) {
@@ -468,6 +599,16 @@ bool replay_candidate(const Candidate& c, const void* in, void* out) {
       std::memcpy(out, in, (size_t)(c.bytes / 2));
       return true;
     case kTiled: {
+      if (const NarrowEntry* e = find_narrow(c.elem, c.tiled.form)) {
+        e->replay(c, in, out);
+        return true;
+      }
+      if (c.tiled.form == kTileSkew) {
+        const SkewEntry* e = find_skew(c);
+        if (!e) return false;
+        e->replay(c, in, out);
+        return true;
+      }
       const TiledEntry* e = find_tiled(c);
       if (!e) return false;
       e->replay(c, in, out);
@@ -548,7 +689,7 @@ static std::map<OccKey, int> g_occ;
 int query_occupancy(const Candidate& c) {
   const void* k = kernel_of(c);
   if (!k) return 0;
-  const bool dyn = c.method == kPacked || c.method == kPackedSplit;
+  const bool dyn = dynamic_lds(c);
   const int lds = dyn ? c.lds_bytes : 0;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
@@ -573,7 +714,7 @@ int query_occupancy(const Candidate& c) {
 }
 
 int prepare_kernel(const Candidate& c) {
-  if (c.method != kPacked && c.method != kPackedSplit) return 0;
+  if (!dynamic_lds(c)) return 0;
   const void* k = kernel_of(c);
   if (!k) return -1;
   return ensure_lds_limit(k, c.lds_bytes) ? 0 : -1;

@@ -18,27 +18,19 @@ namespace lrt {
 
 namespace {
 
-// Blocks per CU that Tiled / TiledCopy grids are capped at (each block loops
-// over the remaining tiles). LIBRETT_GRID_PER_CU overrides it.
-int grid_per_cu() {
-  static int v = [] {
-    const char* e = std::getenv("LIBRETT_GRID_PER_CU");
-    int x = e ? std::atoi(e) : 0;
-    return x > 0 ? x : 64;
-  }();
-  return v;
-}
-
-// Tile-row group of the Tiled order (16 measured best for 256 MiB f32 and
-// f64 2-D transposes on MI355X: +20-25% over row-major tile order in a
-// steady stream of transposes); LIBRETT_TILE_GROUP overrides it.
-int tile_group() {
+// Tile-row group of the Tiled order for tiles of `ty` rows of elem bytes: as
+// many tile rows as write 4 KiB of each output column. For 256 MiB 2-D
+// transposes on MI355X the best group covers 4 KiB whatever the tile: f32
+// 64x32 32 rows (97 us; 16: 109, 64: 107), 64x64 16 (102; 8: 117, 32: 109),
+// 128x128 8 (90; 4: 94, 16: 94); f64 32x32 16 (91; 8: 115, 32: 97), 64x64 8
+// (92; 4: 105, 16: 94). Skewed tiles do as well with 8 KiB, which covers more
+// columns' phases. LIBRETT_TILE_GROUP overrides it.
+int tile_group(int ty, int elem, bool skew) {
   static int v = [] {
     const char* e = std::getenv("LIBRETT_TILE_GROUP");
-    int x = e ? std::atoi(e) : 0;
-    return x > 0 ? x : 16;
+    return e ? std::atoi(e) : 0;
   }();
-  return v;
+  return v > 0 ? v : std::max(1, (skew ? 8192 : 4096) / (ty * elem));
 }
 
 
@@ -68,12 +60,34 @@ void output_strides(const Problem& p, long long* s) {
 }
 
 // Rows of at least this many bytes that stay rows (perm[0] == 0) are copied by
-// TiledCopy, not by a Packed plan (which librettPlanMeasure still times). On
-// MI355X, best TiledCopy against best Packed plan of ~200 MiB f32 / f64 / c128 problems: rows of 16 B
-// 148 / 146 / - against 142 / 142 / - us; of 32 B 103 / 103 / 89 against
-// 109 / 107 / 98; of 64 B 79 / 79 / 78 against 88 / 90 / 86; of 1040 B
-// 73 / 74 / 72 against 105 / 100 / 89.
-constexpr int kCopyOnlyRow = 32;
+// TiledCopy, not by a Packed plan (which librettPlanMeasure still times). Best
+// TiledCopy over best other plan of random 16-500 MB problems on MI355X:
+// median 0.78 for rows of 64 to 1024 bytes, but at 16 to 48 bytes 0.75-1.08
+// with a wide spread, where the inputs' lines are split between many rows
+// ([4,58,684,2,30] f32 43.6 us against 22.9; [2,3,4392,2,2,35] c128 34 against
+// 19.5), so there the choice is left to the selector. More than 3% worse: 22%
+// of the problems with 32-byte rows, 14% at 64 bytes, 6% at 128, 2% at 256.
+constexpr int kCopyOnlyRow = 128;
+
+// Output columns (the contiguous side of a tile's plane) of at least this many
+// bytes get skewed tiles where they start off their lines: four lines, so
+// that most of what a column writes is whole ones.
+constexpr int kSkewColumn = 512;
+
+// Widest plane that narrow tiles take (and longest short column): with more
+// columns, skewed tiles of 32 fill their lanes well enough. 200 MiB on MI355X,
+// narrow against the best other plan: f32 X = 7 72 against 106 us, 9 89
+// against 88, 12 79 against 75; f64 8 72 against 102, 12 73 against 80, 14 74
+// against 76; c128 8 74 against 76, 12 75 against 72.
+constexpr int kNarrowX = 12;
+
+// Non-temporal loads for an input of `bytes` bytes that a kernel reads in
+// whole lines, once, or nearly so: copies between rotating buffers on MI355X gain from
+// 96 MiB on (33.8 -> 32.2 us at 96 MiB, 85.5 -> 83.1 us at 256 MiB), where
+// input and output no longer fit the 256 MiB Infinity Cache together; below,
+// the input may still be there from whoever wrote it, and streaming it costs
+// (19.9 -> 22.0 us at 64 MiB).
+int stream_input(long long bytes) { return bytes >= (96LL << 20) ? 1 : 0; }
 
 // Outer map over the input dims for which `skip[d]` is false, in input order.
 void build_outer(const Problem& p, const bool* skip, const long long* cin, const long long* cout,
@@ -332,14 +346,15 @@ std::string Candidate::describe() const {
   char buf[256];
   static const char* names[] = {"Unknown", "Trivial", "Packed", "PackedSplit", "Tiled", "TiledCopy"};
   const char* n = (method >= 0 && method < kNumMethods) ? names[method] : "?";
+  static const char* kForms[] = {"", " skew", " narrow", " short"};
   switch (method) {
     case kTiled:
       if (xgroup > 1 || ygroup > 1)
-        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d groups %d/%d grid %d%s", n, tile_x, tile_y, vec_x,
-                 vec_y, xgroup, ygroup, grid_x, tile_order(*this) ? " xcd" : "");
+        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s groups %d/%d grid %d%s", n, tile_x, tile_y, vec_x,
+                 vec_y, kForms[tiled.form], xgroup, ygroup, grid_x, tile_order(*this) ? " xcd" : "");
       else
-        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d grid %d%s", n, tile_x, tile_y, vec_x, vec_y, grid_x,
-                 tile_order(*this) ? " xcd" : "");
+        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s grid %d%s", n, tile_x, tile_y, vec_x, vec_y,
+                 kForms[tiled.form], grid_x, tile_order(*this) ? " xcd" : "");
       break;
     case kTiledCopy:
       snprintf(buf, sizeof(buf), "%s word %dB rows %d grid %d%s", n, word, copy.X, grid_x,
@@ -383,6 +398,12 @@ void make_group(const Problem& r, const int* dims, int n, const long long* strid
   for (int k = 0; k < kMaxGroup - 1; k++) g.div[k] = make_fastdiv(k < n ? (uint32_t)r.dim[dims[k]] : 1u);
 }
 
+// One workgroup per tile, in rows of at most 2^20 workgroups (2^29 threads).
+void set_tile_grid(Candidate& c) {
+  c.grid_x = std::max(1, std::min(c.tiled.items, 1 << 20));
+  c.grid_y = (c.tiled.items + c.grid_x - 1) / c.grid_x;
+}
+
 // Tiled candidates of the reduced problem whose plane is x = input dims
 // [0, a) and y = output dims [0, b) (the reference's Tiled is a = b = 1).
 void add_tiled_plane(const Problem& r, const DeviceInfo& dev, int a_dims, int b_dims, std::vector<Candidate>& out) {
@@ -421,15 +442,132 @@ void add_tiled_plane(const Problem& r, const DeviceInfo& dev, int a_dims, int b_
   make_group(r, xdims, a_dims, cout, xg);
   make_group(r, ydims, b_dims, cin, yg);
   const bool general = a_dims > 1 || b_dims > 1;
-  for (int s = 0; s < nshapes; s++) {
-    Candidate c;
+  // Whether every output column (input row) of a tile starts on a line.
+  bool out_lines = true, in_lines = true;
+  const int le = 128 / B;
+  for (int d = 0; d < r.rank; d++) {
+    bool in_y = false, in_x = d < a_dims;
+    for (int k = 0; k < b_dims; k++) in_y = in_y || ydims[k] == d;
+    if (!in_y) out_lines = out_lines && cout[d] % le == 0;
+    if (!in_x) in_lines = in_lines && cin[d] % le == 0;
+  }
+  TiledArgs base;
+  base.X = (int)X;
+  base.Y = (int)Y;
+  base.in_ys = (int)cin[ydims[0]];
+  base.out_xs = (int)cout[0];
+  base.xg = xg;
+  base.yg = yg;
+  base.xcds = 1;
+  base.form = kTileRect;
+  base.x_div = make_fastdiv((uint32_t)X);
+  base.word_shift = 0;
+  base.stream_in = !dev.batch_mode && in_lines ? stream_input(r.vol * B) : 0;
+  base.outer = outer;
+  // Tile `c` of the shape given, `rows` of the plane high including what the
+  // skew needs.
+  auto push = [&](Candidate& c, long long rows) {
+    TiledArgs& a = c.tiled;
+    a.ntx = (int)((X + c.tile_x - 1) / c.tile_x);
+    const int nty = (int)((rows + c.tile_y - 1) / c.tile_y);
+    a.ntiles = a.ntx * nty;
+    a.ntx_div = make_fastdiv((uint32_t)a.ntx);
+    a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
+    a.items = (int)std::min<long long>((long long)a.ntiles * vol_outer, 0x7fffffffLL);
+    set_tile_group(a, nty, tile_group(c.tile_y, B, a.form != kTileRect));
     c.method = kTiled;
     c.elem = B;
     c.source = "reduced";
-    c.tile_x = shapes[s][0];
-    c.tile_y = shapes[s][1];
     c.xgroup = a_dims;
     c.ygroup = b_dims;
+    set_tile_grid(c);
+    c.bytes = 2 * r.vol * B;
+    c.split.sizeMm = a_dims;
+    c.split.sizeMk = b_dims;
+    c.split.volMm = (int)X;
+    c.split.volMk = (int)Y;
+    c.split.volMbar = vol_outer;
+    c.split.volMmk = (int)(X * Y);
+    out.push_back(c);
+  };
+  // Skewed tiles where columns start off their lines and are long enough to
+  // hold whole ones.
+  const bool skew = !out_lines && Y * B >= kSkewColumn;
+  if (skew) {
+    static const int skew4[4][3] = {{64, 128, 512}, {64, 64, 256}, {32, 128, 256}, {32, 64, 256}};
+    static const int skew8[4][3] = {{64, 64, 512}, {32, 64, 256}, {32, 128, 512}, {32, 32, 256}};
+    static const int skew16[4][3] = {{32, 32, 256}, {32, 64, 512}, {16, 32, 256}, {32, 16, 256}};
+    for (const auto& sh : B == 16 ? skew16 : B == 8 ? skew8 : skew4) {
+      if (dev.batch_mode && !batch_skew_available(B, sh[0], sh[1])) continue;
+      Candidate c;
+      c.tiled = base;
+      c.tiled.form = kTileSkew;
+      c.tiled.stream_in = 0;
+      c.tile_x = sh[0];
+      c.tile_y = sh[1];
+      c.block = sh[2];
+      c.vec_x = 1;
+      c.vec_y = 16 / B;
+      c.word = 16;
+      const int rows = c.tile_y + le;
+      c.lds_bytes = rows * (c.tile_x + 1) * B + (general ? ((rows + c.tile_x) * 4 + B - 1) / B * B : 0);
+      push(c, Y + le - 1);
+    }
+  }
+  // Narrow planes, whose rows lie back to back in the input: tiles of all X
+  // columns, as many rows as the kernel's registers hold.
+  const int pe = 16 / B;
+  if (X <= kNarrowX && b_dims == 1 && cin[ydims[0]] == X && Y * B >= kSkewColumn) {
+    Candidate c;
+    c.tiled = base;
+    c.tiled.form = kTileNarrow;
+    c.tiled.stream_in = 0;
+    int most;
+    narrow_shape(B, kTileNarrow, c.block, most);
+    int shift = 0;
+    while ((pe << shift) < Y && X * ((pe << (shift + 1)) + le) <= most) shift++;
+    c.tiled.word_shift = shift;
+    c.tile_x = (int)X;
+    c.tile_y = pe << shift;
+    c.vec_x = 1;
+    c.vec_y = pe;
+    c.word = 16;
+    c.lds_bytes = (c.tile_y + le) * ((int)X | 1) * B + (int)X * 4;
+    push(c, Y + le - 1);
+  }
+  // Short columns that lie back to back in the output: tiles are stretches of
+  // it (push counts them as the plane's columns).
+  if (Y <= kNarrowX && a_dims == 1 && cout[0] == Y && X * B >= kSkewColumn) {
+    Candidate c;
+    c.tiled = base;
+    c.tiled.form = kTileShort;
+    c.tiled.stream_in = 0;
+    int ch;
+    narrow_shape(B, kTileShort, c.block, ch);
+    const int nx = (ch + (int)Y - 2) / (int)Y + 1;
+    c.tiled.x_div = make_fastdiv((uint32_t)Y);
+    c.tiled.nx_div = make_fastdiv((uint32_t)nx);
+    c.tile_x = ch;
+    c.tile_y = (int)Y;
+    c.vec_x = 1;
+    c.vec_y = pe;
+    c.word = 16;
+    c.lds_bytes = (int)Y * (nx | 1) * B + (int)Y * 4;
+    push(c, Y);
+    // Tiles of the plane's X * Y elements, and a line's for the phase.
+    TiledArgs& a = out.back().tiled;
+    a.ntx = a.ntiles = (int)((X * Y + le - 1 + ch - 1) / ch);
+    a.ntx_div = a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
+    a.items = (int)std::min<long long>((long long)a.ntiles * vol_outer, 0x7fffffffLL);
+    set_tile_grid(out.back());
+  }
+  for (int s = 0; s < nshapes; s++) {
+    // Long rows of tiles pay where whole lines move.
+    if (skew && (shapes[s][0] > 64 || shapes[s][1] > 64)) continue;
+    Candidate c;
+    c.tiled = base;
+    c.tile_x = shapes[s][0];
+    c.tile_y = shapes[s][1];
     // Widest lanes (vx elements per input access, vy per output access)
     // that divide the plane's extents and have a kernel instantiated;
     // ties go to the larger sum. Every input offset outside the x group is
@@ -450,34 +588,10 @@ void add_tiled_plane(const Problem& r, const DeviceInfo& dev, int a_dims, int b_
     if (vx == 0) continue;
     c.vec_x = vx;
     c.vec_y = vy;
-    TiledArgs& a = c.tiled;
-    a.X = (int)X;
-    a.Y = (int)Y;
-    a.in_ys = (int)cin[ydims[0]];
-    a.out_xs = (int)cout[0];
-    a.xg = xg;
-    a.yg = yg;
-    a.ntx = (int)((X + c.tile_x - 1) / c.tile_x);
-    const int nty = (int)((Y + c.tile_y - 1) / c.tile_y);
-    a.ntiles = a.ntx * nty;
-    a.ntx_div = make_fastdiv((uint32_t)a.ntx);
-    a.ntiles_div = make_fastdiv((uint32_t)a.ntiles);
-    a.items = (int)std::min<long long>((long long)a.ntiles * vol_outer, 0x7fffffffLL);
-    set_tile_group(a, nty, tile_group());
-    a.xcds = 1;
-    a.outer = outer;
-    c.block = 256;
+    c.block = tiled_threads(c.tile_x, c.tile_y);
     // Group planes keep the tile's row and column offsets after the tile.
     c.lds_bytes = c.tile_y * (c.tile_x + 1) * B + (general ? ((c.tile_x + c.tile_y) * 4 + B - 1) / B * B : 0);
-    c.grid_x = std::max(1, std::min(a.items, dev.cu_count * grid_per_cu()));
-    c.bytes = 2 * r.vol * B;
-    c.split.sizeMm = a_dims;
-    c.split.sizeMk = b_dims;
-    c.split.volMm = (int)X;
-    c.split.volMk = (int)Y;
-    c.split.volMbar = vol_outer;
-    c.split.volMmk = (int)(X * Y);
-    out.push_back(c);
+    push(c, Y);
   }
 }
 
@@ -526,14 +640,6 @@ void add_tiled(const Problem& r, const DeviceInfo& dev, std::vector<Candidate>& 
     if (!dup) add_tiled_plane(r, dev, ab[0], ab[1], out);
   }
 }
-
-// Non-temporal loads for an input of `bytes` bytes that a kernel reads in
-// whole lines, once, or nearly so: copies between rotating buffers on MI355X gain from
-// 96 MiB on (33.8 -> 32.2 us at 96 MiB, 85.5 -> 83.1 us at 256 MiB), where
-// input and output no longer fit the 256 MiB Infinity Cache together; below,
-// the input may still be there from whoever wrote it, and streaming it costs
-// (19.9 -> 22.0 us at 64 MiB).
-int stream_input(long long bytes) { return bytes >= (96LL << 20) ? 1 : 0; }
 
 // Words of 16 bytes over the output in order; one plan (and its twin in the
 // other work order).
@@ -934,7 +1040,9 @@ void model_tiled(Candidate& c) {
   const TiledArgs& a = c.tiled;
   const int B = c.elem;
   double R = 0, W = 0, P = 0, TR = 0, TW = 0;
-  std::vector<long long> ws = sample_indices(a.items, 24);
+  // All items when there are at most 24, else a sample (fewer of the skewed
+  // tiles, whose split rows take longer to count).
+  std::vector<long long> ws = sample_indices(a.items, a.form != kTileRect && a.items > 24 ? 8 : 24);
   std::vector<Run> rin, rout;
   for (long long w : ws) {
     uint32_t mb = (uint32_t)(w / a.ntiles);
@@ -945,10 +1053,33 @@ void model_tiled(Candidate& c) {
     int tx = std::min(c.tile_x, a.X - x0), ty = std::min(c.tile_y, a.Y - y0);
     rin.clear();
     rout.clear();
+    if (a.form == kTileShort) {
+      // Runs of each input row, one run of the output.
+      int e0, e1;
+      short_tile(a, oo, tile, c.tile_x, 128 / B, e0, e1);
+      if (e0 < e1) rout.push_back({(oo + (long long)e0) * B, (long long)(e1 - e0) * B});
+      for (int y = 0; y < a.Y; y++) {
+        int xa, xb;
+        short_row(a, y, e0, e1, xa, xb);
+        if (xa < xb) rin.push_back({(oi + xa + (long long)tiled_in_y(a, (uint32_t)y)) * B, (long long)(xb - xa) * B});
+      }
+    } else if (a.form != kTileRect) {
+      const SkewTile k = skew_tile(a, oo, x0, tx, 128 / B);
+      for (int y = std::max(0, y0 - k.hi); y < std::min(a.Y, y0 + c.tile_y); y++) {
+        const long long row = oi + x0 + (long long)tiled_in_y(a, (uint32_t)y);
+        skew_row_runs(k, y, y0, c.tile_y,
+                      [&](int i, int n) { rin.push_back({(row + i) * B, (long long)n * B}); });
+      }
+      for (int i = 0; i < tx; i++) {
+        const int ya = std::max(0, y0 - k.s[i]), yb = std::min(a.Y, y0 - k.s[i] + c.tile_y);
+        if (ya < yb) rout.push_back({(oo + ya + (long long)tiled_out_x(a, (uint32_t)(x0 + i))) * B, (long long)(yb - ya) * B});
+      }
+    } else {
     for (int y = 0; y < ty; y++)
       rin.push_back({(oi + x0 + (long long)tiled_in_y(a, (uint32_t)(y0 + y))) * B, (long long)tx * B});
     for (int x = 0; x < tx; x++)
       rout.push_back({(oo + y0 + (long long)tiled_out_x(a, (uint32_t)(x0 + x))) * B, (long long)ty * B});
+    }
     for (const Run& r : rin) TR += tran(r.s, r.n);
     for (const Run& r : rout) TW += tran(r.s, r.n);
     double l, p;
@@ -965,7 +1096,7 @@ void model_tiled(Candidate& c) {
   c.model.read_tran = TR * scale;
   c.model.write_tran = TW * scale;
   c.model.items = a.items;
-  c.model.steps_per_block = (double)a.items / c.grid_x;
+  c.model.steps_per_block = 1;
 }
 
 void model_copy(Candidate& c) {
@@ -1007,7 +1138,7 @@ void model_copy(Candidate& c) {
   c.model.read_tran = TR * scale;
   c.model.write_tran = TW * scale;
   c.model.items = a.items;
-  c.model.steps_per_block = (double)a.items / c.grid_x;
+  c.model.steps_per_block = 1;
 }
 
 }  // namespace
@@ -1247,7 +1378,7 @@ bool order_twins(const Candidate& a, const Candidate& b) {
   if (a.method == kTiled || a.method == kTiledCopy)
     return b.method == a.method && tile_order(a) != tile_order(b) && a.tile_x == b.tile_x &&
            a.tile_y == b.tile_y && a.vec_x == b.vec_x && a.vec_y == b.vec_y && a.word == b.word &&
-           a.copy_tx == b.copy_tx && a.xgroup == b.xgroup && a.ygroup == b.ygroup;
+           a.copy_tx == b.copy_tx && a.block == b.block && a.tiled.form == b.tiled.form && a.xgroup == b.xgroup && a.ygroup == b.ygroup;
   return (a.method == kPacked || a.method == kPackedSplit) && same_packed(a, b) && a.grid_x == b.grid_x &&
          a.grid_y == b.grid_y && a.packed.outer_per_block == b.packed.outer_per_block &&
          a.source == b.source && a.packed.order != b.packed.order;
@@ -1277,6 +1408,12 @@ void add_order_twins(const DeviceInfo& dev, std::vector<Candidate>& out) {
       x.tiled.xcds = xcds;
     else
       x.copy.xcds = xcds;
+    // Narrow and short tiles have no order across XCDs: it measured slower for
+    // every width (f64, 200 MiB: 70-74 us against 80-99).
+    if (tile_order(x) && c.method == kTiled && c.tiled.form >= kTileNarrow) {
+      res.push_back(c);
+      continue;
+    }
     if (c.method == kTiled) {
       res.push_back(x);
       res.push_back(c);
@@ -1423,7 +1560,7 @@ int choose_by_model(const std::vector<Candidate>& cands) {
 
 Candidate scalar_fallback(const Candidate& c) {
   Candidate f = c;
-  if (c.method == kTiled) {
+  if (c.method == kTiled && c.tiled.form == kTileRect) {
     f.vec_x = 1;
     f.vec_y = 1;
   }
@@ -1433,7 +1570,8 @@ Candidate scalar_fallback(const Candidate& c) {
 int needed_alignment(const Candidate& c) {
   switch (c.method) {
     case kTiled:
-      return c.elem * std::max(c.vec_x, c.vec_y);
+      // Skewed tiles place their words by the output's address.
+      return c.tiled.form != kTileRect ? c.elem : c.elem * std::max(c.vec_x, c.vec_y);
     default:
       return c.elem;
   }

@@ -141,15 +141,29 @@ def problems(n, seed, family="random", **kw):
 # Collection (GPU)
 # ---------------------------------------------------------------------------
 
-def collect(probs, stream, in_ptr, out_ptr, log=None):
-    """Features and measured times of every candidate of every problem."""
-    from . import measure_candidates, selector_features
+# Buffer pairs that a steady stream of launches uses in turn.
+STEADY_SETS = 3
+
+
+def _stride(dim, elem):
+    """Bytes from one buffer of a problem to the next, in a steady timing."""
+    return -(-int(np.prod(dim, dtype=np.int64)) * elem // 4096) * 4096
+
+
+def collect(probs, stream, in_ptr, out_ptr, log=None, steady=False):
+    """Features and measured times of every candidate of every problem:
+    librettPlanMeasure's loop, or with `steady` a stream of launches over
+    STEADY_SETS buffer pairs (the buffers then hold that many problems)."""
+    from . import measure_candidates, measure_steady, selector_features
     recs = []
     t0 = time.time()
     last = t0
     for k, (d, p, e) in enumerate(probs):
         feats, mc = selector_features(d, p, e)
-        times = measure_candidates(d, p, e, stream, in_ptr, out_ptr)
+        if steady:
+            times = measure_steady(d, p, e, stream, in_ptr, out_ptr, _stride(d, e), STEADY_SETS)
+        else:
+            times = measure_candidates(d, p, e, stream, in_ptr, out_ptr)
         n = min(len(feats), len(times))
         recs.append({"dims": list(d), "perm": list(p), "elem": int(e), "feats": feats[:n], "times": times[:n],
                      "model_choice": int(mc)})
@@ -430,6 +444,10 @@ def main(argv=None):
     ap.add_argument("--seed", type=int, default=2)
     ap.add_argument("--family", choices=["random", "pow2"], default="random",
                     help="collect: problem family (random dims, or powers of two)")
+    ap.add_argument("--steady", action="store_true",
+                    help="collect: time a stream of launches over several buffers, not single runs")
+    ap.add_argument("--bytes-lo", type=int, default=1 << 20, help="collect: smallest problem")
+    ap.add_argument("--bytes-hi", type=int, default=512 << 20, help="collect: largest problem")
     ap.add_argument("--out", default="selector_data.npz")
     ap.add_argument("--data", nargs="+", default=None)
     ap.add_argument("--weights", default=DEFAULT_WEIGHTS)
@@ -469,9 +487,10 @@ def main(argv=None):
         if a.out:
             save_records(a.out, ho)
     elif a.cmd == "collect":
-        A, B = _buffers(512 << 20)
-        probs = problems(a.total or a.problems, a.seed, a.family)[a.offset:a.offset + a.problems]
-        recs = collect(probs, stream, A.ptr, B.ptr, log)
+        probs = problems(a.total or a.problems, a.seed, a.family, bytes_lo=a.bytes_lo,
+                         bytes_hi=a.bytes_hi)[a.offset:a.offset + a.problems]
+        A, B = _buffers((STEADY_SETS if a.steady else 1) * max(_stride(d, e) for d, _, e in probs))
+        recs = collect(probs, stream, A.ptr, B.ptr, log, a.steady)
         save_records(a.out, recs, with_features=False)
     elif a.cmd == "train":
         recs = []

@@ -56,3 +56,35 @@ def check(stream, dim, perm, elem, offsets, methods=None, only=None):
 ])
 def test_copy_rows(gpu_stream, dim, perm, elem):
     assert check(gpu_stream, dim, perm, elem, [0, 1, 5, 128 // elem - 1], methods=(L.TILED_COPY,)) >= 4
+
+
+# Skewed tiles: columns of just enough whole lines, cut tiles on both sides,
+# planes over dim groups and outer dims that move the phase, and every place
+# in a line that the output can start at.
+SKEWED = [([65, 129], [1, 0], 4), ([70, 131, 3], [1, 0, 2], 4), ([33, 259, 5], [1, 2, 0], 4),
+          ([5, 29, 7, 67], [3, 1, 0, 2], 8), ([65, 129], [1, 0], 8), ([3, 97, 21], [1, 2, 0], 8),
+          ([17, 33], [1, 0], 16), ([7, 67, 5], [1, 0, 2], 16), ([9, 11, 35], [2, 1, 0], 16)]
+
+
+@pytest.mark.parametrize("dim,perm,elem", SKEWED)
+def test_skewed_tiles(gpu_stream, dim, perm, elem):
+    line = 128 // elem
+    assert check(gpu_stream, dim, perm, elem, [0, 1, line // 2, line - 1], only=" skew") >= 8
+
+
+# Narrow planes, 1 to 12 columns, and the same the other way round (short
+# columns): one tile and several, cut by the plane's end, with outer dims that
+# move the phase.
+NARROW = [([7, 1483], [1, 0], 4), ([2, 4099], [1, 0], 4), ([12, 257, 3], [1, 0, 2], 4), ([11, 130, 3], [1, 2, 0], 4),
+          ([5, 1100], [1, 0], 8), ([8, 67, 5], [1, 0, 2], 8), ([12, 64, 3], [1, 0, 2], 8),
+          ([3, 2051], [1, 0], 16), ([12, 33, 4], [1, 0, 2], 16)]
+SHORT = [([1483, 7], [1, 0], 4), ([512, 4, 3], [1, 0, 2], 4), ([4096, 2], [1, 0], 8), ([4099, 2], [1, 0], 4), ([257, 3, 12], [2, 0, 1], 4), ([130, 2, 5, 3], [2, 1, 0, 3], 4),
+         ([1100, 5], [1, 0], 8), ([67, 8, 5], [1, 0, 2], 8), ([515, 2, 3], [2, 1, 0], 8),
+         ([2051, 3], [1, 0], 16), ([33, 4, 12], [2, 0, 1], 16)]
+
+
+@pytest.mark.parametrize("dim,perm,elem", NARROW + SHORT)
+def test_narrow_planes(gpu_stream, dim, perm, elem):
+    line = 128 // elem
+    form = " narrow" if (dim, perm, elem) in NARROW else " short"
+    assert check(gpu_stream, dim, perm, elem, [0, 1, line - 1], only=form) >= 3
