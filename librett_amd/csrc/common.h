@@ -68,14 +68,24 @@ __host__ __device__ inline uint32_t fdiv(uint32_t n, const FastDiv& f) {
 // (k % d0, (k / d0) % d1, ...); digit r moves the input by ct_in[r] and the
 // output by ct_out[r] elements (the reference keeps the same information as
 // TensorConvInOut entries, src/plan.cpp:935-947).
-struct OuterMap {
+template <int DIGITS>
+struct OuterMapOf {
   int n;
-  FastDiv div[kMaxRank];
-  int ct_in[kMaxRank];
-  int ct_out[kMaxRank];
+  FastDiv div[DIGITS];
+  int ct_in[DIGITS];
+  int ct_out[DIGITS];
 };
+using OuterMap = OuterMapOf<kMaxRank>;
 
-__host__ __device__ inline void outer_offsets(const OuterMap& m, uint32_t k,
+// Most plans have few outer dims, and a launch costs more the larger its
+// arguments are: back to back on MI355X 2.8 us at 64 bytes, 3.5 at 256, 3.8 at
+// 512, 4.0 at 960. So the Tiled and TiledCopy kernels also come with arguments
+// for up to this many outer dims (136 to 412 bytes instead of 700 to 970); the
+// others take the kernels with room for kMaxRank.
+constexpr int kFewDigits = 4;
+
+template <int DIGITS>
+__host__ __device__ inline void outer_offsets(const OuterMapOf<DIGITS>& m, uint32_t k,
                                               int& off_in, int& off_out) {
   int oi = 0, oo = 0;
   for (int r = 0; r < m.n; r++) {
@@ -111,6 +121,12 @@ __host__ __device__ inline int group_offset(const GroupMap& g, uint32_t v) {
   return off + (int)v * g.stride[kMaxGroup - 1];
 }
 
+// Stands for a group of one dim in kernels compiled for those alone.
+struct NoGroup {
+  static constexpr int n = 1;
+};
+__host__ __device__ inline int group_offset(const NoGroup&, uint32_t) { return 0; }
+
 enum TileForm : int { kTileRect = 0, kTileSkew = 1, kTileNarrow = 2, kTileShort = 3 };
 
 // Tiled: 2-D tile plane of (x = input dim 0, y = the input dim that becomes
@@ -121,12 +137,10 @@ enum TileForm : int { kTileRect = 0, kTileSkew = 1, kTileNarrow = 2, kTileShort 
 // dims are short still get tiles with long runs on both sides; the output
 // offset of x (the input offset of y) is then group_offset(xg, x)
 // (group_offset(yg, y)) instead of x * out_xs (y * in_ys).
-struct TiledArgs {
+struct TiledPlane {
   int X, Y;          // plane extents in elements
   int in_ys;         // input stride of y (yg.n == 1)
   int out_xs;        // output stride of x (xg.n == 1)
-  GroupMap xg;       // x digits -> output offset
-  GroupMap yg;       // y digits -> input offset
   int ntx;           // tiles along x
   int ntiles;        // tiles per plane
   FastDiv ntx_div;
@@ -155,14 +169,23 @@ struct TiledArgs {
   // walks one contiguous range of tiles (tiles that share 128-byte lines
   // then meet in one XCD's L2); 1: workgroup b starts at tile b.
   int xcds;
-  OuterMap outer;
 };
 
+template <int DIGITS, class GROUP>
+struct TiledArgsOf : TiledPlane {
+  GROUP xg;  // x digits -> output offset
+  GROUP yg;  // y digits -> input offset
+  OuterMapOf<DIGITS> outer;
+};
+using TiledArgs = TiledArgsOf<kMaxRank, GroupMap>;
+
 // Output offset of tile-plane column x and input offset of row y.
-__host__ __device__ inline int tiled_out_x(const TiledArgs& a, uint32_t x) {
+template <class A>
+__host__ __device__ inline int tiled_out_x(const A& a, uint32_t x) {
   return a.xg.n > 1 ? group_offset(a.xg, x) : (int)x * a.out_xs;
 }
-__host__ __device__ inline int tiled_in_y(const TiledArgs& a, uint32_t y) {
+template <class A>
+__host__ __device__ inline int tiled_in_y(const A& a, uint32_t y) {
   return a.yg.n > 1 ? group_offset(a.yg, y) : (int)y * a.in_ys;
 }
 
@@ -174,7 +197,8 @@ struct SkewTile {
   unsigned char s[kMaxSkewTile];
 };
 
-__host__ __device__ inline SkewTile skew_tile(const TiledArgs& a, int off_out, int x0, int tx, int le) {
+template <class A>
+__host__ __device__ inline SkewTile skew_tile(const A& a, int off_out, int x0, int tx, int le) {
   SkewTile k;
   k.tx = tx;
   k.lo = le;
@@ -212,13 +236,15 @@ __host__ __device__ inline void skew_row_runs(const SkewTile& k, int y, int y0, 
 // Output elements [e0, e1) of tile `tile` of a plane of short columns, tiles of
 // ch elements, for an output that starts on a line; and the columns [xa, xb) of
 // plane row y among them.
-__host__ __device__ inline void short_tile(const TiledArgs& a, int off_out, int tile, int ch, int le, int& e0,
+template <class A>
+__host__ __device__ inline void short_tile(const A& a, int off_out, int tile, int ch, int le, int& e0,
                                            int& e1) {
   const int s = tile * ch - (off_out & (le - 1)), n = a.X * a.Y;
   e0 = s < 0 ? 0 : s;
   e1 = n - s < ch ? n : s + ch;
 }
-__host__ __device__ inline void short_row(const TiledArgs& a, int y, int e0, int e1, int& xa, int& xb) {
+template <class A>
+__host__ __device__ inline void short_row(const A& a, int y, int e0, int e1, int& xa, int& xb) {
   xa = (e0 - y + a.Y - 1) / a.Y;
   xb = (e1 - y + a.Y - 1) / a.Y;
 }
@@ -227,7 +253,8 @@ __host__ __device__ inline void short_row(const TiledArgs& a, int y, int e0, int
 // The output is written front to back, so its element index is (row, c) with
 // row = e / X; the row's digits in output order give its input offset.
 // Reference counterpart: transposeTiledCopy, src/kernel.cpp:453-545.
-struct CopyArgs {
+template <int DIGITS>
+struct CopyArgsOf {
   int n;             // elements
   int X;             // elements per row
   FastDiv row_div;   // X
@@ -237,10 +264,12 @@ struct CopyArgs {
   int stream_in;     // non-temporal loads: the input cannot stay in the Infinity Cache
   // Row index digits, fastest first: ct_in[r] elements of input each. The
   // last digit needs no division.
-  OuterMap rows;
+  OuterMapOf<DIGITS> rows;
 };
+using CopyArgs = CopyArgsOf<kMaxRank>;
 
-__host__ __device__ inline int copy_row_offset(const OuterMap& m, uint32_t row) {
+template <int DIGITS>
+__host__ __device__ inline int copy_row_offset(const OuterMapOf<DIGITS>& m, uint32_t row) {
   int off = 0;
   for (int r = 0; r + 1 < m.n; r++) {
     const uint32_t q = fdiv(row, m.div[r]);

@@ -120,7 +120,8 @@ struct TileCtx {
 };
 
 // Tile w of a Tiled plan with tiles of tx_size x ty_size elements.
-__host__ __device__ inline TileCtx tile_item(const TiledArgs& a, uint32_t w, int tx_size, int ty_size) {
+template <class A>
+__host__ __device__ inline TileCtx tile_item(const A& a, uint32_t w, int tx_size, int ty_size) {
   TileCtx c;
   const uint32_t mb = fdiv(w, a.ntiles_div);
   const uint32_t tile = w - mb * (uint32_t)a.ntiles;
@@ -193,7 +194,8 @@ struct TiledOps {
   // magic-number division each), so the load and store loops read them from
   // LDS instead of each thread dividing for every row it moves. A barrier
   // must separate prepare() from load().
-  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx& c, int t, E* lds) {
+  template <class A>
+  __host__ __device__ static void prepare(const A& a, const TileCtx& c, int t, E* lds) {
     if constexpr (G) {
       int* o = offsets(lds);
       if (t < TY) {
@@ -206,11 +208,12 @@ struct TiledOps {
     }
   }
 
-  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) { return tile_item(a, w, TX, TY); }
+  template <class A>
+  __host__ __device__ static TileCtx item(const A& a, uint32_t w) { return tile_item(a, w, TX, TY); }
 
   // LARGE: whole tiles are loaded non-temporally where the plan asks for it.
-  template <bool LARGE = false>
-  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t,
+  template <bool LARGE = false, class A>
+  __host__ __device__ static void load(const A& a, const TileCtx& c, int t,
                                        const E* __restrict__ in, E* lds) {
     VI r[NPR];
     const int lx = (t % LR) * VX;
@@ -258,7 +261,8 @@ struct TiledOps {
     }
   }
 
-  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t,
+  template <class A>
+  __host__ __device__ static void store(const A& a, const TileCtx& c, int t,
                                         E* __restrict__ out, const E* lds) {
     const int ly = (t % LW) * VY;
     const int lx = t / LW;
@@ -328,13 +332,16 @@ struct SkewOps {
     return reinterpret_cast<const int*>(lds + R * PITCH);
   }
 
-  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) { return tile_item(a, w, TX, TY); }
+  template <class A>
+  __host__ __device__ static TileCtx item(const A& a, uint32_t w) { return tile_item(a, w, TX, TY); }
 
   // G only, as in TiledOps: prepare() with a barrier before load() where the y
   // group has several dims; else only the columns' output offsets are needed,
   // by store().
-  __host__ __device__ static bool early(const TiledArgs& a) { return G && a.yg.n > 1; }
-  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx& c, int t, E* lds) {
+  template <class A>
+  __host__ __device__ static bool early(const A& a) { return G && a.yg.n > 1; }
+  template <class A>
+  __host__ __device__ static void prepare(const A& a, const TileCtx& c, int t, E* lds) {
     int* o = offsets(lds);
     if (t < R) {
       const int y = c.y0 - LE + t;
@@ -346,19 +353,22 @@ struct SkewOps {
   }
 
   // Output offset of tile column i, and its skew.
-  __host__ __device__ static int column(const TiledArgs& a, const TileCtx& c, int i, const E* lds) {
+  template <class A>
+  __host__ __device__ static int column(const A& a, const TileCtx& c, int i, const E* lds) {
     return c.off_out + (G ? offsets(lds)[R + i] : (c.x0 + i) * a.out_xs);
   }
   __host__ __device__ static int skew(int base, int phase) { return (base + phase) & (LE - 1); }
 
   // Tile rows [lo, hi) that a column with skew s covers.
-  __host__ __device__ static void rows(const TiledArgs& a, const TileCtx& c, int s, int& lo, int& hi) {
+  template <class A>
+  __host__ __device__ static void rows(const A& a, const TileCtx& c, int s, int& lo, int& hi) {
     const int first = LE - c.y0, end = a.Y - c.y0 + LE;  // rows of y = 0 and y = Y
     lo = LE - s > first ? LE - s : first;
     hi = LE - s + TY < end ? LE - s + TY : end;
   }
 
-  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
+  template <class A>
+  __host__ __device__ static void load(const A& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
                                        int phase) {
     const int lx = t % TX;
     const int ly = t / TX;
@@ -384,7 +394,8 @@ struct SkewOps {
     }
   }
 
-  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t, E* __restrict__ out,
+  template <class A>
+  __host__ __device__ static void store(const A& a, const TileCtx& c, int t, E* __restrict__ out,
                                         const E* lds, int phase) {
     const int ly = (t % LW) * PE;
     const int lx = t / LW;
@@ -433,26 +444,34 @@ struct NarrowOps {
   static constexpr int NW = (NL + PE - 1) / PE;  // store passes
 
   // LDS: rows of odd pitch, then X output offsets of the columns.
-  __host__ __device__ static int pitch(const TiledArgs& a) { return a.X | 1; }
-  __host__ __device__ static int rows(const TiledArgs& a) { return (PE << a.word_shift) + LE; }
-  __host__ __device__ static int* offsets(const TiledArgs& a, E* lds) {
+  template <class A>
+  __host__ __device__ static int pitch(const A& a) { return a.X | 1; }
+  template <class A>
+  __host__ __device__ static int rows(const A& a) { return (PE << a.word_shift) + LE; }
+  template <class A>
+  __host__ __device__ static int* offsets(const A& a, E* lds) {
     return reinterpret_cast<int*>(lds + rows(a) * pitch(a));
   }
-  __host__ __device__ static const int* offsets(const TiledArgs& a, const E* lds) {
+  template <class A>
+  __host__ __device__ static const int* offsets(const A& a, const E* lds) {
     return reinterpret_cast<const int*>(lds + rows(a) * pitch(a));
   }
 
-  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) {
+  template <class A>
+  __host__ __device__ static TileCtx item(const A& a, uint32_t w) {
     return tile_item(a, w, a.X, PE << a.word_shift);
   }
 
   // Before load(), with a barrier between.
-  __host__ __device__ static constexpr bool early(const TiledArgs&) { return true; }
-  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx& c, int t, E* lds) {
+  template <class A>
+  __host__ __device__ static constexpr bool early(const A&) { return true; }
+  template <class A>
+  __host__ __device__ static void prepare(const A& a, const TileCtx& c, int t, E* lds) {
     if (t < a.X) offsets(a, lds)[t] = c.off_out + tiled_out_x(a, (uint32_t)t);
   }
 
-  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
+  template <class A>
+  __host__ __device__ static void load(const A& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
                                        int phase) {
     const int ty = PE << a.word_shift;
     const int n = (ty + LE) * a.X;
@@ -492,7 +511,8 @@ struct NarrowOps {
     }
   }
 
-  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t, E* __restrict__ out,
+  template <class A>
+  __host__ __device__ static void store(const A& a, const TileCtx& c, int t, E* __restrict__ out,
                                         const E* lds, int phase) {
     const int* off = offsets(a, lds);
     const int P = pitch(a);
@@ -544,8 +564,10 @@ struct ShortOps {
   __host__ __device__ static int columns(int Y) { return (CH + Y - 2) / Y + 1; }
   static constexpr int NLD = NL + 1;  // columns(Y) * Y <= CH + 2 * Y <= (NL + 1) * NT
 
-  __host__ __device__ static int pitch(const TiledArgs& a) { return (int)a.nx_div.d | 1; }
-  __host__ __device__ static TileCtx item(const TiledArgs& a, uint32_t w) {
+  template <class A>
+  __host__ __device__ static int pitch(const A& a) { return (int)a.nx_div.d | 1; }
+  template <class A>
+  __host__ __device__ static TileCtx item(const A& a, uint32_t w) {
     TileCtx c;
     const uint32_t mb = fdiv(w, a.ntiles_div);
     c.x0 = (int)(w - mb * (uint32_t)a.ntiles);  // tile of the plane
@@ -559,16 +581,20 @@ struct ShortOps {
     return c.x0 * CH - ((c.off_out + phase) & (LE - 1));
   }
   // Before load(), with a barrier between.
-  __host__ __device__ static constexpr bool early(const TiledArgs&) { return true; }
+  template <class A>
+  __host__ __device__ static constexpr bool early(const A&) { return true; }
   // After the tile's Y rows, their input offsets (ints).
-  __host__ __device__ static const int* offsets(const TiledArgs& a, const E* lds) {
+  template <class A>
+  __host__ __device__ static const int* offsets(const A& a, const E* lds) {
     return reinterpret_cast<const int*>(lds + a.Y * pitch(a));
   }
-  __host__ __device__ static void prepare(const TiledArgs& a, const TileCtx&, int t, E* lds) {
+  template <class A>
+  __host__ __device__ static void prepare(const A& a, const TileCtx&, int t, E* lds) {
     if (t < a.Y) const_cast<int*>(offsets(a, lds))[t] = tiled_in_y(a, (uint32_t)t);
   }
 
-  __host__ __device__ static void load(const TiledArgs& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
+  template <class A>
+  __host__ __device__ static void load(const A& a, const TileCtx& c, int t, const E* __restrict__ in, E* lds,
                                        int phase) {
     const int e0 = first(c, phase), n = a.X * a.Y;
     const uint32_t lo = e0 < 0 ? 0 : (uint32_t)e0;
@@ -594,7 +620,8 @@ struct ShortOps {
     }
   }
 
-  __host__ __device__ static void store(const TiledArgs& a, const TileCtx& c, int t, E* __restrict__ out,
+  template <class A>
+  __host__ __device__ static void store(const A& a, const TileCtx& c, int t, E* __restrict__ out,
                                         const E* lds, int phase) {
     const int e0 = first(c, phase);
     const uint32_t n = (uint32_t)(a.X * a.Y);
@@ -655,7 +682,8 @@ struct CopyOps {
 
   // Words of item w start at element w * PER - phase: word boundaries are
   // 16-byte boundaries of the output's addresses, and items start on lines.
-  __host__ __device__ static void run(const CopyArgs& a, uint32_t w, int t, const E* __restrict__ in,
+  template <class A>
+  __host__ __device__ static void run(const A& a, uint32_t w, int t, const E* __restrict__ in,
                                       E* __restrict__ out) {
     if (a.stream_in) {
       keep_branch();
@@ -666,8 +694,8 @@ struct CopyOps {
     }
   }
 
-  template <bool STREAM>
-  __host__ __device__ static void move(const CopyArgs& a, uint32_t w, int t, const E* __restrict__ in,
+  template <bool STREAM, class A>
+  __host__ __device__ static void move(const A& a, uint32_t w, int t, const E* __restrict__ in,
                                        E* __restrict__ out) {
     const uint32_t e = first(w, t, line_phase(out));
     if (whole(a, e)) {
@@ -693,11 +721,13 @@ struct CopyOps {
   __host__ __device__ static uint32_t first(uint32_t w, int t, int phase) {
     return w * (uint32_t)PER + (uint32_t)(t * PE) - (uint32_t)phase;
   }
-  __host__ __device__ static bool whole(const CopyArgs& a, uint32_t e) {
+  template <class A>
+  __host__ __device__ static bool whole(const A& a, uint32_t e) {
     return e < (uint32_t)a.n && (uint32_t)a.n - e >= (uint32_t)PE;
   }
   // Input offset of output element e.
-  __host__ __device__ static int source(const CopyArgs& a, uint32_t e) {
+  template <class A>
+  __host__ __device__ static int source(const A& a, uint32_t e) {
     const uint32_t row = fdiv(e, a.row_div);
     return copy_row_offset(a.rows, row) + (int)(e - row * (uint32_t)a.X);
   }

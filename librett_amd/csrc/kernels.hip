@@ -9,6 +9,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -48,14 +49,21 @@ namespace lrt {
 // occupancy.)
 // The tile of this workgroup, -1 past the last one. The grid has two dims only
 // because one dim holds at most 2^32 threads.
-__device__ __forceinline__ int tile_of(const TiledArgs& a) {
+__device__ __forceinline__ int tile_of(const TiledPlane& a) {
   const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
   if (b >= (uint32_t)a.items) return -1;
   return a.xcds > 1 ? xcd_logical((int)b, a.items, a.xcds) : (int)b;
 }
 
-template <int B, int TX, int TY, int VX, int VY, bool G>
-__global__ __launch_bounds__((TiledOps<B, TX, TY, VX, VY, G>::NT)) void k_tiled(TiledArgs a,
+// FEW: at most kFewDigits outer dims.
+template <bool G, bool FEW>
+using TiledParam =
+    std::conditional_t<FEW, TiledArgsOf<kFewDigits, std::conditional_t<G, GroupMap, NoGroup>>, TiledArgs>;
+template <bool FEW>
+using CopyParam = std::conditional_t<FEW, CopyArgsOf<kFewDigits>, CopyArgs>;
+
+template <int B, int TX, int TY, int VX, int VY, bool G, bool FEW>
+__global__ __launch_bounds__((TiledOps<B, TX, TY, VX, VY, G>::NT)) void k_tiled(TiledParam<G, FEW> a,
                                                                                  const void* __restrict__ in,
                                                                                  void* __restrict__ out) {
   using Ops = TiledOps<B, TX, TY, VX, VY, G>;
@@ -75,8 +83,9 @@ __global__ __launch_bounds__((TiledOps<B, TX, TY, VX, VY, G>::NT)) void k_tiled(
   Ops::store(a, c, threadIdx.x, dst, lds);
 }
 
-template <int B, int TX, int TY, int NT, bool G>
-__global__ __launch_bounds__(NT) void k_skew(TiledArgs a, const void* __restrict__ in, void* __restrict__ out) {
+template <int B, int TX, int TY, int NT, bool G, bool FEW>
+__global__ __launch_bounds__(NT) void k_skew(TiledParam<G, FEW> a, const void* __restrict__ in,
+                                             void* __restrict__ out) {
   using Ops = SkewOps<B, TX, TY, NT, G>;
   using E = typename Ops::E;
   __shared__ E lds[Ops::LDS_ELEMS];
@@ -96,8 +105,9 @@ __global__ __launch_bounds__(NT) void k_skew(TiledArgs a, const void* __restrict
 }
 
 // Ops: NarrowOps or ShortOps.
-template <class Ops>
-__global__ __launch_bounds__(Ops::NT) void k_narrow(TiledArgs a, const void* __restrict__ in, void* __restrict__ out) {
+template <class Ops, bool FEW>
+__global__ __launch_bounds__(Ops::NT) void k_narrow(TiledParam<true, FEW> a, const void* __restrict__ in,
+                                                    void* __restrict__ out) {
   using E = typename Ops::E;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   E* lds = reinterpret_cast<E*>(smem);
@@ -115,8 +125,8 @@ __global__ __launch_bounds__(Ops::NT) void k_narrow(TiledArgs a, const void* __r
 }
 
 // One item per workgroup.
-template <int B>
-__global__ __launch_bounds__(256) void k_copy(CopyArgs a, const void* __restrict__ in,
+template <int B, bool FEW>
+__global__ __launch_bounds__(256) void k_copy(CopyParam<FEW> a, const void* __restrict__ in,
                                               void* __restrict__ out) {
   using Ops = CopyOps<B>;
   using E = typename Ops::E;
@@ -386,15 +396,23 @@ static void replay_packed(const Candidate& c, const void* in, void* out) {
 // Instantiation tables
 // ---------------------------------------------------------------------------
 
+// Kernels of a shape: for any number of outer dims, and for kFewDigits.
+struct KernelPair {
+  const void* any;
+  const void* few;
+};
+#define LRT_KERNELS(K, ...) \
+  {reinterpret_cast<const void*>(&K<__VA_ARGS__, false>), reinterpret_cast<const void*>(&K<__VA_ARGS__, true>)}
+
 struct TiledEntry {
   int b, tx, ty, vx, vy;
   bool general;  // handles x / y groups of several dims
-  const void* kernel;
+  KernelPair kernel;
   void (*replay)(const Candidate&, const void*, void*);
 };
 struct CopyEntry {
   int b;
-  const void* kernel;
+  KernelPair kernel;
   void (*replay)(const Candidate&, const void*, void*);
 };
 struct PackedEntry {
@@ -404,7 +422,7 @@ struct PackedEntry {
 };
 
 #define LRT_TILED_G(B, TX, TY, VX, VY, G)                                                    \
-  {B, TX, TY, VX, VY, G, reinterpret_cast<const void*>(&k_tiled<B, TX, TY, VX, VY, G>), \
+  {B, TX, TY, VX, VY, G, LRT_KERNELS(k_tiled, B, TX, TY, VX, VY, G), \
    &replay_tiled<B, TX, TY, VX, VY, G>},
 #define LRT_TILED(B, TX, TY, VX, VY) LRT_TILED_G(B, TX, TY, VX, VY, false)
 #define LRT_TILED_V(B, TX, TY, V) \
@@ -439,12 +457,12 @@ static const TiledEntry kTiledTable[] = {
 struct SkewEntry {
   int b, tx, ty, nt;
   bool general;
-  const void* kernel;
+  KernelPair kernel;
   void (*replay)(const Candidate&, const void*, void*);
 };
 
 #define LRT_SKEW_G(B, TX, TY, NT, G) \
-  {B, TX, TY, NT, G, reinterpret_cast<const void*>(&k_skew<B, TX, TY, NT, G>), &replay_skew<SkewOps<B, TX, TY, NT, G>>},
+  {B, TX, TY, NT, G, LRT_KERNELS(k_skew, B, TX, TY, NT, G), &replay_skew<SkewOps<B, TX, TY, NT, G>>},
 #define LRT_SKEW(B, TX, TY, NT) LRT_SKEW_G(B, TX, TY, NT, false) LRT_SKEW_G(B, TX, TY, NT, true)
 
 static const SkewEntry kSkewTable[] = {
@@ -458,19 +476,19 @@ struct NarrowEntry {
   int b;
   TileForm form;
   int nt, elements;
-  const void* kernel;
+  KernelPair kernel;
   void (*replay)(const Candidate&, const void*, void*);
 };
 #define LRT_NARROW(B, NT, NL)                                                                                \
-  {B, kTileNarrow, NT, NarrowOps<B, NT, NL>::MAX, reinterpret_cast<const void*>(&k_narrow<NarrowOps<B, NT, NL>>), \
+  {B, kTileNarrow, NT, NarrowOps<B, NT, NL>::MAX, LRT_KERNELS(k_narrow, NarrowOps<B, NT, NL>), \
    &replay_skew<NarrowOps<B, NT, NL>>},
 #define LRT_SHORT(B, NT, NL)                                                                             \
-  {B, kTileShort, NT, ShortOps<B, NT, NL>::CH, reinterpret_cast<const void*>(&k_narrow<ShortOps<B, NT, NL>>), \
+  {B, kTileShort, NT, ShortOps<B, NT, NL>::CH, LRT_KERNELS(k_narrow, ShortOps<B, NT, NL>), \
    &replay_skew<ShortOps<B, NT, NL>>},
 static const NarrowEntry kNarrowTable[] = {LRT_NARROW(4, 256, 8) LRT_NARROW(8, 256, 6) LRT_NARROW(16, 256, 4)
                                            LRT_SHORT(4, 256, 8) LRT_SHORT(8, 256, 6) LRT_SHORT(16, 256, 4)};
 
-#define LRT_COPY(B) {B, reinterpret_cast<const void*>(&k_copy<B>), &replay_copy<B>},
+#define LRT_COPY(B) {B, LRT_KERNELS(k_copy, B), &replay_copy<B>},
 
 static const CopyEntry kCopyTable[] = {LRT_COPY(4) LRT_COPY(8) LRT_COPY(16)};
 
@@ -538,20 +556,27 @@ bool packed_nreg_available(int elem, int nreg) {
   return false;
 }
 
+// Plans with few outer dims are launched with short arguments.
+static bool few_digits(const Candidate& c) {
+  return c.method == kTiled ? c.tiled.outer.n <= kFewDigits : c.method == kTiledCopy && c.copy.rows.n <= kFewDigits;
+}
+
 static const void* kernel_of(const Candidate& c) {
+  const KernelPair* k = nullptr;
   switch (c.method) {
     case kTiled: {
-      if (const NarrowEntry* e = find_narrow(c.elem, c.tiled.form)) return e->kernel;
-      if (c.tiled.form == kTileSkew) {
-        const SkewEntry* e = find_skew(c);
-        return e ? e->kernel : nullptr;
+      if (const NarrowEntry* e = find_narrow(c.elem, c.tiled.form))
+        k = &e->kernel;
+      else if (c.tiled.form == kTileSkew) {
+        if (const SkewEntry* s = find_skew(c)) k = &s->kernel;
+      } else if (const TiledEntry* t = find_tiled(c)) {
+        k = &t->kernel;
       }
-      const TiledEntry* e = find_tiled(c);
-      return e ? e->kernel : nullptr;
+      break;
     }
     case kTiledCopy: {
-      const CopyEntry* e = find_copy(c);
-      return e ? e->kernel : nullptr;
+      if (const CopyEntry* e = find_copy(c)) k = &e->kernel;
+      break;
     }
     case kPacked:
     case kPackedSplit: {
@@ -559,8 +584,17 @@ static const void* kernel_of(const Candidate& c) {
       return e ? e->kernel : nullptr;
     }
     default:
-      return nullptr;
+      break;
   }
+  if (!k) return nullptr;
+  return few_digits(c) ? k->few : k->any;
+}
+
+static void few_outer(const OuterMap& m, OuterMapOf<kFewDigits>& f) {
+  f.n = m.n;
+  std::copy(m.div, m.div + kFewDigits, f.div);
+  std::copy(m.ct_in, m.ct_in + kFewDigits, f.ct_in);
+  std::copy(m.ct_out, m.ct_out + kFewDigits, f.ct_out);
 }
 
 // Kernels whose LDS is sized at launch.
@@ -577,12 +611,40 @@ hipError_t launch_candidate(const Candidate& c, const void* in, void* out, hipSt
   dim3 grid(c.method == kTiledCopy ? copy_items(c, out) : c.grid_x, c.grid_y, 1);
   dim3 block(c.block, 1, 1);
   void* args[3];
+  TiledParam<true, true> group;
+  TiledParam<false, true> plane;
+  CopyParam<true> copy;
+  const bool few = few_digits(c);
   switch (c.method) {
     case kTiled:
-      args[0] = const_cast<TiledArgs*>(&c.tiled);
+      if (few && (c.tiled.form >= kTileNarrow || c.xgroup > 1 || c.ygroup > 1)) {
+        static_cast<TiledPlane&>(group) = c.tiled;
+        group.xg = c.tiled.xg;
+        group.yg = c.tiled.yg;
+        few_outer(c.tiled.outer, group.outer);
+        args[0] = &group;
+      } else if (few) {
+        static_cast<TiledPlane&>(plane) = c.tiled;
+        few_outer(c.tiled.outer, plane.outer);
+        args[0] = &plane;
+      } else {
+        args[0] = const_cast<TiledArgs*>(&c.tiled);
+      }
       break;
     case kTiledCopy:
-      args[0] = const_cast<CopyArgs*>(&c.copy);
+      if (few) {
+        copy.n = c.copy.n;
+        copy.X = c.copy.X;
+        copy.row_div = c.copy.row_div;
+        copy.per = c.copy.per;
+        copy.items = c.copy.items;
+        copy.xcds = c.copy.xcds;
+        copy.stream_in = c.copy.stream_in;
+        few_outer(c.copy.rows, copy.rows);
+        args[0] = &copy;
+      } else {
+        args[0] = const_cast<CopyArgs*>(&c.copy);
+      }
       break;
     default:
       args[0] = const_cast<PackedArgs*>(&c.packed);

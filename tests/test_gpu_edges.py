@@ -88,3 +88,15 @@ def test_narrow_planes(gpu_stream, dim, perm, elem):
     line = 128 // elem
     form = " narrow" if (dim, perm, elem) in NARROW else " short"
     assert check(gpu_stream, dim, perm, elem, [0, 1, line - 1], only=form) >= 3
+
+
+@pytest.mark.parametrize("dim, perm", [
+    ([33, 2, 3, 2, 3, 35], [5, 4, 3, 2, 1, 0]),
+    ([33, 2, 3, 2, 3, 2, 35], [6, 5, 4, 3, 2, 1, 0]),
+    ([9, 2, 3, 2, 3], [0, 4, 3, 2, 1]),
+    ([9, 2, 3, 2, 3, 2], [0, 5, 4, 3, 2, 1]),
+    ([3, 5, 3, 2, 3, 2, 3, 70], [7, 6, 5, 4, 3, 2, 1, 0]),
+], ids=["plane, 4 outer dims", "plane, 5", "rows, 4", "rows, 5", "groups, 4 to 6"])
+@pytest.mark.parametrize("elem", [4, 8, 16])
+def test_outer_dims_around_the_short_arguments(gpu_stream, dim, perm, elem):
+    check(gpu_stream, dim, perm, elem, [0, 1], methods=(4, 5))
