@@ -154,8 +154,8 @@ __host__ __device__ inline TileCtx tile_item(const A& a, uint32_t w, int tx_size
 // Bound by HBM. One workgroup moves one tile and ends: a loop over tiles kept
 // 106 SGPRs and up to 20 more VGPRs alive (34 SGPRs without it), and the
 // dispatcher's order keeps neighbouring tiles closer in time than a stride
-// over the grid does ([2, 8, 16, 32, 64, 128] f32 95 -> 85 us with the loads
-// non-temporal too; a copy of the bytes takes 85 us).
+// over the grid does ([2, 8, 16, 32, 64, 128] f32 95 -> 88 us as 64 x 128 tiles,
+// with the loads non-temporal too; a copy of the bytes takes 85 us).
 // Reference counterpart: transposeTiled, src/kernel.cpp:48-170.
 // ---------------------------------------------------------------------------
 // G = false compiles only the one-dim-group path (the kernel then needs no
@@ -167,7 +167,7 @@ struct TiledOps {
   using VO = typename Word<B * VY>::type;
   // 128 x 128 tiles take 512 threads: with 256, two workgroups of 66 KiB of LDS
   // leave a CU 8 waves (8192 x 8192 f32 on MI355X: 104 us; with 512, 95 us, and
-  // 85 us with one tile per workgroup and non-temporal loads as well).
+  // 88 us with one tile per workgroup and non-temporal loads as well).
   static constexpr int NT = TX * TY >= 128 * 128 ? 512 : 256;
   static constexpr int LR = TX / VX;   // lanes per input row
   static constexpr int RP = NT / LR;   // input rows per pass
