@@ -273,7 +273,7 @@ static void replay_tiled(const Candidate& c, const void* in, void* out) {
     for (int t = 0; t < Ops::NT; t++) Ops::prepare(a, ctx, t, lds.data());
     for (int t = 0; t < Ops::NT; t++) {
       replay_at(w, t);
-      Ops::load(a, ctx, t, src, lds.data());
+      Ops::template load<true>(a, ctx, t, src, lds.data());
     }
     for (int t = 0; t < Ops::NT; t++) {
       replay_at(w, t);

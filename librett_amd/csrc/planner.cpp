@@ -86,8 +86,14 @@ constexpr int kNarrowX = 12;
 // 96 MiB on (33.8 -> 32.2 us at 96 MiB, 85.5 -> 83.1 us at 256 MiB), where
 // input and output no longer fit the 256 MiB Infinity Cache together; below,
 // the input may still be there from whoever wrote it, and streaming it costs
-// (19.9 -> 22.0 us at 64 MiB).
-int stream_input(long long bytes) { return bytes >= (96LL << 20) ? 1 : 0; }
+// (19.9 -> 22.0 us at 64 MiB). LIBRETT_STREAM_MB overrides the size.
+int stream_input(long long bytes) {
+  static const long long from = [] {
+    const char* e = std::getenv("LIBRETT_STREAM_MB");
+    return e && *e ? std::atoll(e) : 96;
+  }();
+  return bytes >= from << 20 ? 1 : 0;
+}
 
 // Outer map over the input dims for which `skip[d]` is false, in input order.
 void build_outer(const Problem& p, const bool* skip, const long long* cin, const long long* cout,
@@ -347,18 +353,19 @@ std::string Candidate::describe() const {
   static const char* names[] = {"Unknown", "Trivial", "Packed", "PackedSplit", "Tiled", "TiledCopy"};
   const char* n = (method >= 0 && method < kNumMethods) ? names[method] : "?";
   static const char* kForms[] = {"", " skew", " narrow", " short"};
+  const char* order = tile_order(*this) ? " xcd" : "";
   switch (method) {
     case kTiled:
       if (xgroup > 1 || ygroup > 1)
-        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s groups %d/%d grid %d%s", n, tile_x, tile_y, vec_x,
-                 vec_y, kForms[tiled.form], xgroup, ygroup, grid_x, tile_order(*this) ? " xcd" : "");
+        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s groups %d/%d grid %d%s%s", n, tile_x, tile_y, vec_x,
+                 vec_y, kForms[tiled.form], xgroup, ygroup, grid_x, order, tiled.stream_in ? " stream" : "");
       else
-        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s grid %d%s", n, tile_x, tile_y, vec_x, vec_y,
-                 kForms[tiled.form], grid_x, tile_order(*this) ? " xcd" : "");
+        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s grid %d%s%s", n, tile_x, tile_y, vec_x, vec_y,
+                 kForms[tiled.form], grid_x, order, tiled.stream_in ? " stream" : "");
       break;
     case kTiledCopy:
-      snprintf(buf, sizeof(buf), "%s word %dB rows %d grid %d%s", n, word, copy.X, grid_x,
-               tile_order(*this) ? " xcd" : "");
+      snprintf(buf, sizeof(buf), "%s word %dB rows %d grid %d%s%s", n, word, copy.X, grid_x, order,
+               copy.stream_in ? " stream" : "");
       break;
     case kPacked:
     case kPackedSplit:

@@ -100,3 +100,15 @@ def test_narrow_planes(gpu_stream, dim, perm, elem):
 @pytest.mark.parametrize("elem", [4, 8, 16])
 def test_outer_dims_around_the_short_arguments(gpu_stream, dim, perm, elem):
     check(gpu_stream, dim, perm, elem, [0, 1], methods=(4, 5))
+
+
+# Inputs of 96 MiB and more that are read in whole lines: non-temporal loads,
+# over planes of one dim and of dim groups (whole tiles and cut ones), and rows.
+@pytest.mark.parametrize("dim,perm,elem", [
+    ([64, 6, 344, 200], [2, 1, 0, 3], 4), ([32, 12, 344, 100], [2, 1, 0, 3], 8), ([16, 100, 16, 260], [3, 2, 1, 0], 16),
+    ([1024, 160, 161], [0, 2, 1], 4),
+])
+def test_streamed_loads(gpu_stream, dim, perm, elem):
+    want = [c["desc"] for c in L.candidates(dim, perm, elem) if c["desc"].endswith(" stream")]
+    assert len(want) >= 2 and (perm[0] == 0 or any("groups" in d for d in want))
+    assert check(gpu_stream, dim, perm, elem, [0], only=" stream") == len(want)
