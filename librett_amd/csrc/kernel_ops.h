@@ -664,7 +664,7 @@ struct ShortOps {
 // itself and loads the word from wherever the row starts (any element
 // boundary). A word that crosses a row's end is loaded element by element.
 // Bound by HBM. On MI355X a copy of [2307, 115, 126] f64 rows (18456 B, no
-// row on a line boundary) takes 86 us against 129 us for row tiles of 8-byte
+// row on a line boundary) takes 89 us against 128 us for row tiles of 8-byte
 // words, whose lines are written in two parts by different workgroups, and
 // [1024, 256, 256] f32 takes 86 us against 94 us; a plain copy of the bytes
 // takes 85 us. One word per thread runs faster than two or four (85.8, 87.8,

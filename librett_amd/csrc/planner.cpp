@@ -686,11 +686,16 @@ void add_tiled_copy(const Problem& r, const DeviceInfo& dev, std::vector<Candida
   const long long span = r.vol + (dev.batch_mode ? 128 / B - 1 : 0);
   a.items = (int)((span + a.per - 1) / a.per);
   a.xcds = 1;
-  // Rows that end inside lines are read partly by two items; streaming pays
-  // from rows of 2 KiB on (f64, 200 MiB: 72.8 -> 69.9 us with 4104-byte rows,
-  // 73.1 -> 72.8 with 2056, but 73.5 -> 78.7 with 1032 and 79 -> 82 with 520).
-  const long long row = (long long)r.dim[0] * B;
-  a.stream_in = !dev.batch_mode && (row % 128 == 0 || row >= 2048) ? stream_input(r.vol * B) : 0;
+  // Rows that end inside lines: a line at a cut is read by two items, and the
+  // second finds a streamed one gone, from L2 and, if its writer has just left
+  // it there, from the Infinity Cache. So they stream only where the input is
+  // far larger than that cache. 18 KB rows of f64 streamed and not, right after
+  // a kernel that filled the input, and among passes over three buffer pairs:
+  // 112 MiB 49.5 and 38.2 us, 40.2 and 40.6; 256 MiB 106 and 82, 88.2 and 89.7;
+  // 384 MiB 146 and 150, 132 and 134; 500 MiB 193 and 213, 173 and 175. Shorter
+  // rows never gain (1 KB, 500 MiB: 230 and 226, 188 and 185).
+  const long long row = (long long)r.dim[0] * B, bytes = r.vol * B;
+  a.stream_in = !dev.batch_mode && (row % 128 == 0 ? stream_input(bytes) : row >= 2048 && stream_input(bytes / 4));
   c.block = 256;
   c.lds_bytes = 0;
   c.grid_x = a.items;

@@ -53,3 +53,15 @@ def test_streamed_plans(dim, perm):
 
 def test_small_inputs_are_not_streamed():
     assert not any("stream" in d for _, _, d in plans(96, SHAPES))
+
+
+@pytest.mark.parametrize("dim,elem,streamed", [
+    ([1024, 256, 256], 4, True), ([1024, 96, 250], 4, False), ([2307, 115, 126], 8, False),
+    ([2307, 50, 112], 8, False), ([2307, 150, 145], 8, False), ([2307, 150, 146], 8, True), ([129, 700, 700], 8, False),
+])
+def test_rows_cut_by_lines_stream_only_far_beyond_the_cache(dim, elem, streamed):
+    # 256 MiB of whole lines, and 94; cut rows of 18 KB from 384 MiB on (the
+    # two sizes around it), cut rows of 1 KB never.
+    import librett_amd as L
+    copies = [c["desc"] for c in L.host_candidates(dim, [0, 2, 1], elem) if c["method"] == L.TILED_COPY]
+    assert copies and all(d.endswith(" stream") == streamed for d in copies)
