@@ -35,7 +35,7 @@ constexpr int kCountThreads = 256;
 constexpr int kCountMaxGrid = 2048;
 
 // Row pieces of a TiledCopy item: at most 1024 elements (of 4 bytes) in rows
-// of at least 2, the first of which may be cut.
+// of at least 2 (or 2048 in rows of at least 16), the first of which may be cut.
 constexpr int kCopyPieces = 514;
 // Rows of a skewed tile: at most 128 and a line of 4-byte elements.
 constexpr int kSkewRows = 160;
@@ -135,7 +135,7 @@ __host__ __device__ inline int job_passes(const CountJob& j, int store) {
       // A lane's word, or the elements of a word that crosses a row's end
       // (loads) or the tensor's end: its k-th access is counted with the other
       // lanes' k-th.
-      return 16 / j.B;
+      return j.a.copy.per / j.nt;
     default:
       return j.nreg;
   }
@@ -255,20 +255,24 @@ __host__ __device__ inline bool lane_access(const CountJob& j, const ItemCtx& c,
     return true;
   }
   if (j.method == kTiledCopy) {
-    // Addresses for an output that starts on a line.
+    // Addresses for an output that starts on a line. This is the p-th access
+    // that the lane's words take, one word in each 16 * nt bytes of the item.
     const CopyArgs& a = j.a.copy;
     const int pe = 16 / j.B;
-    const long long e = c.out0 + (long long)t * pe;
-    if (e >= a.n) return false;
-    const long long row = e / a.X, k = e - row * a.X;
-    const bool word = a.n - e >= pe && (store || a.X - k >= pe);
-    if (word && p > 0) return false;
-    if (word) bytes = 16;
-    const long long q = e + p;
-    if (q >= a.n) return false;
-    const long long qrow = q / a.X;
-    off = (store ? q : copy_row_offset(a.rows, (uint32_t)qrow) + (q - qrow * a.X)) * j.B;
-    return true;
+    int q = p;
+    for (long long e = c.out0 + (long long)t * pe; e < c.out0 + a.per && e < a.n; e += (long long)j.nt * pe) {
+      const long long row = e / a.X, k = e - row * a.X;
+      const bool word = a.n - e >= pe && (store || a.X - k >= pe);
+      const int n = word ? 1 : (int)(a.n - e < pe ? a.n - e : pe);
+      if (q < n) {
+        if (word) bytes = 16;
+        const long long x = e + q, xrow = x / a.X;
+        off = (store ? x : copy_row_offset(a.rows, (uint32_t)xrow) + (x - xrow * a.X)) * j.B;
+        return true;
+      }
+      q -= n;
+    }
+    return false;
   }
   const StagedShape& s = j.a.packed.shape[c.plus];
   uint32_t k = (uint32_t)(t + p * j.nt);
@@ -541,7 +545,7 @@ bool make_job(const Candidate& c, CountJob& j, std::vector<int>& runs) {
     case kTiledCopy:
       j.B = c.elem;
       j.nt = c.block;
-      if (c.copy.per != kCountThreads * (16 / j.B) || c.copy.X < 2) return false;
+      if (c.copy.per % (kCountThreads * (16 / j.B)) || c.copy.per / c.copy.X + 2 > kCopyPieces) return false;
       j.a.copy = c.copy;
       j.items = c.copy.items;
       return true;

@@ -667,18 +667,20 @@ struct ShortOps {
 // row on a line boundary) takes 89 us against 128 us for row tiles of 8-byte
 // words, whose lines are written in two parts by different workgroups, and
 // [1024, 256, 256] f32 takes 86 us against 94 us; a plain copy of the bytes
-// takes 85 us. One word per thread runs faster than two or four (85.8, 87.8,
-// 90.3 us; in the batched engine 3.34 ms against 3.46 ms for four): more,
-// shorter workgroups keep the open DRAM pages close together.
+// takes 85 us. Out of HBM one word per thread runs faster than two or four
+// (85.8, 87.8, 90.3 us; in the batched engine 3.34 ms against 3.46 ms for
+// four): more, shorter workgroups keep the open DRAM pages close together. Out
+// of the Infinity Cache a workgroup's own time counts for more, and two words
+// per thread are in flight at once (NP = 2; copy_words() in the planner).
 // Reference counterpart: transposeTiledCopy, src/kernel.cpp:453-545.
 // ---------------------------------------------------------------------------
-template <int B>
+template <int B, int NP = 1>
 struct CopyOps {
   using E = typename Word<B>::type;
   using V = typename Word<16>::type;
   static constexpr int NT = 256;
-  static constexpr int PE = 16 / B;    // elements per word
-  static constexpr int PER = NT * PE;  // elements per item
+  static constexpr int PE = 16 / B;         // elements per word
+  static constexpr int PER = NP * NT * PE;  // elements per item
 
   // Words of item w start at element w * PER - phase: word boundaries are
   // 16-byte boundaries of the output's addresses, and items start on lines.
@@ -697,26 +699,35 @@ struct CopyOps {
   template <bool STREAM, class A>
   __host__ __device__ static void move(const A& a, uint32_t w, int t, const E* __restrict__ in,
                                        E* __restrict__ out) {
-    const uint32_t e = first(w, t, line_phase(out));
-    if (whole(a, e)) {
-      V r;
+    const uint32_t first_e = first(w, t, line_phase(out));
+    V r[NP];
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+      const uint32_t e = first_e + (uint32_t)(j * NT * PE);
+      if (!whole(a, e)) continue;
       const uint32_t row = fdiv(e, a.row_div);
       const int c = (int)(e - row * (uint32_t)a.X);
       if (PE == 1 || a.X - c >= PE) {
-        r = ld_unaligned<V, B, STREAM>(in + (copy_row_offset(a.rows, row) + c));
+        r[j] = ld_unaligned<V, B, STREAM>(in + (copy_row_offset(a.rows, row) + c));
       } else {
 #pragma unroll
-        for (int k = 0; k < PE; k++) vset<E>(r, k, ld(in + source(a, e + k)));
+        for (int k = 0; k < PE; k++) vset<E>(r[j], k, ld(in + source(a, e + k)));
       }
-      st(reinterpret_cast<V*>(out + e), r);
-    } else {
+    }
 #pragma unroll
-      for (int k = 0; k < PE; k++)
-        if (e + k < (uint32_t)a.n) st(out + (e + k), ld(in + source(a, e + k)));
+    for (int j = 0; j < NP; j++) {
+      const uint32_t e = first_e + (uint32_t)(j * NT * PE);
+      if (whole(a, e)) {
+        st(reinterpret_cast<V*>(out + e), r[j]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < PE; k++)
+          if (e + k < (uint32_t)a.n) st(out + (e + k), ld(in + source(a, e + k)));
+      }
     }
   }
 
-  // First element of thread t in item w. Unsigned: elements before the
+  // First element of thread t's first word in item w. Unsigned: elements before the
   // tensor wrap to values above any volume, as do words past 2^31.
   __host__ __device__ static uint32_t first(uint32_t w, int t, int phase) {
     return w * (uint32_t)PER + (uint32_t)(t * PE) - (uint32_t)phase;

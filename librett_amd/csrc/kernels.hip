@@ -125,10 +125,10 @@ __global__ __launch_bounds__(Ops::NT) void k_narrow(TiledParam<true, FEW> a, con
 }
 
 // One item per workgroup.
-template <int B, bool FEW>
+template <int B, int NP, bool FEW>
 __global__ __launch_bounds__(256) void k_copy(CopyParam<FEW> a, const void* __restrict__ in,
                                               void* __restrict__ out) {
-  using Ops = CopyOps<B>;
+  using Ops = CopyOps<B, NP>;
   using E = typename Ops::E;
   const uint32_t w = a.xcds > 1 ? (uint32_t)xcd_logical((int)blockIdx.x, (int)gridDim.x, a.xcds) : blockIdx.x;
   Ops::run(a, w, threadIdx.x, static_cast<const E*>(in), static_cast<E*>(out));
@@ -305,9 +305,9 @@ static void replay_skew(const Candidate& c, const void* in, void* out) {
   }
 }
 
-template <int B>
+template <int B, int NP>
 static void replay_copy(const Candidate& c, const void* in, void* out) {
-  using Ops = CopyOps<B>;
+  using Ops = CopyOps<B, NP>;
   using E = typename Ops::E;
   const int items = copy_items(c, out);
   for (int w = 0; w < items; w++)
@@ -411,7 +411,7 @@ struct TiledEntry {
   void (*replay)(const Candidate&, const void*, void*);
 };
 struct CopyEntry {
-  int b;
+  int b, per;
   KernelPair kernel;
   void (*replay)(const Candidate&, const void*, void*);
 };
@@ -488,7 +488,8 @@ struct NarrowEntry {
 static const NarrowEntry kNarrowTable[] = {LRT_NARROW(4, 256, 8) LRT_NARROW(8, 256, 6) LRT_NARROW(16, 256, 4)
                                            LRT_SHORT(4, 256, 8) LRT_SHORT(8, 256, 6) LRT_SHORT(16, 256, 4)};
 
-#define LRT_COPY(B) {B, LRT_KERNELS(k_copy, B), &replay_copy<B>},
+#define LRT_COPY_NP(B, NP) {B, CopyOps<B, NP>::PER, LRT_KERNELS(k_copy, B, NP), &replay_copy<B, NP>},
+#define LRT_COPY(B) LRT_COPY_NP(B, 1) LRT_COPY_NP(B, 2)
 
 static const CopyEntry kCopyTable[] = {LRT_COPY(4) LRT_COPY(8) LRT_COPY(16)};
 
@@ -524,7 +525,7 @@ static const NarrowEntry* find_narrow(int elem, int form) {
 }
 static const CopyEntry* find_copy(const Candidate& c) {
   for (const auto& e : kCopyTable)
-    if (e.b == c.elem) return &e;
+    if (e.b == c.elem && e.per == c.copy.per) return &e;
   return nullptr;
 }
 static const PackedEntry* find_packed(const Candidate& c) {

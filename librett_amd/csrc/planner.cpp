@@ -95,6 +95,18 @@ int stream_input(long long bytes) {
   return bytes >= from << 20 ? 1 : 0;
 }
 
+// Words per thread of a TiledCopy plan whose rows of `row` bytes make `bytes`
+// bytes. Two where the input may come from the Infinity Cache, enough
+// workgroups are left and rows are not small pieces of lines. One word and two
+// on MI355X: rows of 64 B 16 MiB 6.3 and 6.2 us, 48 MiB 17.2 and 15.6, 72 MiB
+// 25.4 and 22.9; of 18 KB 72 MiB 24.1 and 22.0; but rows of 16 B 24 MiB 11.0
+// and 11.5, of 32 B 16 MiB 6.5 and 6.8; rows of 1 KB 96 MiB 33.3 and 34.7,
+// 256 MiB 85.2 and 88.8. (Row tiles with four words per thread, the kernel
+// before, took 16.4, 23.8 and 24.7 us for the 48 and 72 MiB cases.)
+int copy_words(long long bytes, long long row) {
+  return bytes >= (16LL << 20) && bytes < (96LL << 20) && row >= 64 ? 2 : 1;
+}
+
 // Outer map over the input dims for which `skip[d]` is false, in input order.
 void build_outer(const Problem& p, const bool* skip, const long long* cin, const long long* cout,
                  int word_scale_num, int word_scale_den, OuterMap& m, int& vol_outer) {
@@ -680,7 +692,8 @@ void add_tiled_copy(const Problem& r, const DeviceInfo& dev, std::vector<Candida
     a.rows.ct_in[k] = d >= 0 ? (int)cin[d] : 0;
     a.rows.ct_out[k] = d >= 0 ? (int)cout[d] : 0;
   }
-  a.per = 256 * (16 / B);
+  const long long row = (long long)r.dim[0] * B, bytes = r.vol * B;
+  a.per = 256 * (16 / B) * (dev.batch_mode ? 1 : copy_words(bytes, row));
   // The batched engine learns its buffers after planning: its items cover
   // the most that an output off its line can need.
   const long long span = r.vol + (dev.batch_mode ? 128 / B - 1 : 0);
@@ -694,7 +707,6 @@ void add_tiled_copy(const Problem& r, const DeviceInfo& dev, std::vector<Candida
   // 112 MiB 49.5 and 38.2 us, 40.2 and 40.6; 256 MiB 106 and 82, 88.2 and 89.7;
   // 384 MiB 146 and 150, 132 and 134; 500 MiB 193 and 213, 173 and 175. Shorter
   // rows never gain (1 KB, 500 MiB: 230 and 226, 188 and 185).
-  const long long row = (long long)r.dim[0] * B, bytes = r.vol * B;
   a.stream_in = !dev.batch_mode && (row % 128 == 0 ? stream_input(bytes) : row >= 2048 && stream_input(bytes / 4));
   c.block = 256;
   c.lds_bytes = 0;

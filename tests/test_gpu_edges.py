@@ -112,3 +112,9 @@ def test_streamed_loads(gpu_stream, dim, perm, elem):
     want = [c["desc"] for c in L.candidates(dim, perm, elem) if c["desc"].endswith(" stream")]
     assert len(want) >= 2 and (perm[0] == 0 or any("groups" in d for d in want))
     assert check(gpu_stream, dim, perm, elem, [0], only=" stream") == len(want)
+
+
+# 16 to 96 MiB: two words per thread.
+@pytest.mark.parametrize("dim,elem", [([33, 367, 349], 4), ([2053, 32, 33], 8), ([5, 461, 459], 16), ([16, 968, 969], 4)])
+def test_copy_rows_two_words(gpu_stream, dim, elem):
+    assert check(gpu_stream, dim, [0, 2, 1], elem, [0, 1, 128 // elem - 1], methods=(L.TILED_COPY,)) == 6
