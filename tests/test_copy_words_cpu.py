@@ -64,3 +64,14 @@ def test_two_words_per_thread_counted(dim, elem):
         assert np.array_equal(kern[order[0]][:, [0, 1, 3, 4, 5]], mine[order[1]][:, [0, 1, 3, 4, 5]]), c["desc"]
         for k, v in OC.counts(kern).items():
             assert got[k] == v, (c["desc"], k, got[k], v)
+
+
+@pytest.mark.parametrize("dim,perm,elem", [([2, 61, 67], [0, 2, 1], 4), ([3, 7, 9, 40], [0, 3, 1, 2], 4), ([2, 90, 45], [0, 2, 1], 8)])
+def test_lines_of_many_row_pieces(dim, perm, elem):
+    # Up to 512 pieces of rows in one item, scattered over the input: the
+    # counters sort them, and count what the model counts where it walks every item.
+    for i, c in copies(dim, perm, elem):
+        assert 1 < c["feat"][2] <= 24
+        got = L.host_candidate_counters(dim, perm, elem, i)
+        assert (got["read_lines"], got["write_lines"], got["partial_lines"]) == (
+            c["read_lines"], c["write_lines"], c["partial_lines"]), c["desc"]
