@@ -209,16 +209,16 @@ int librett_c_batch_execute(unsigned int handle, int use_graph);
 int librett_c_batch_destroy(unsigned int handle);
 int librett_c_batch_info_get(unsigned int handle, librett_c_batch_info* info);
 
-/* Host replay of the batch's persistent kernel for a described device (no
- * GPU): host buffers, `grid` workgroups (<= 0: the planned grid). */
+/* Host replay of the batch's kernels for a described device (no GPU): host
+ * buffers, `grid` workgroups in a row of the launch grid (<= 0: as launched). */
 int librett_c_batch_host_replay(int count, const int* ranks, const int* dims, const int* perms, const size_t* elems,
                                 const librett_c_device* dev, const void* const* idata, void* const* odata, int grid);
 
 /* Host replay of batch-mode candidate `index` of one problem (the order of
- * the batch planner's ranking), through the persistent kernel's per-thread
- * code between guard bands. `fallback` selects the descriptor for buffers
- * not aligned to the vector width; `unit_bytes` the work-unit size (0:
- * default); `grid` the workgroups replayed (0: 4 per CU). With idata and
+ * the batch planner's ranking), through its kernel's per-thread code between
+ * guard bands. `fallback` selects the descriptor for buffers not aligned to
+ * the vector width; `unit_bytes` the work-unit size (0: default); `grid` the
+ * workgroups in a row of the launch grid (0: as launched). With idata and
  * odata both NULL it only stores the number of candidates in *count.
  * Returns LIBRETT_UNDEFINED_ERROR if a store leaves the output or a unit
  * writes past the kernel's LDS. No reference counterpart: test support for

@@ -103,11 +103,16 @@ int batch_alignment(const Problem& p, const Candidate& c);
 // Batch-mode candidates of a problem, best modelled streaming cost first.
 std::vector<Candidate> batch_candidates(const Problem& p, const DeviceInfo& dev);
 
-// Host replay of the kernel (descriptors hold host pointers).
-// Returns false if a unit wrote past the kernel's LDS.
-bool replay_batch(const BatchDesc* descs, const int* start, int nprob, int total, int grid);
+// Workgroups in a row of the launch grid: a grid dim holds fewer than 2^32
+// threads.
+constexpr int kBatchGridRow = 1 << 20;
+
+// Host replay of the kernel (descriptors hold host pointers): the workgroups
+// of a grid with rows of `row` (<= 0: kBatchGridRow), each with its search for
+// its problem. Returns false if a unit wrote past the kernel's LDS.
+bool replay_batch(const BatchDesc* descs, const int* start, int nprob, int total, int row);
 
 // Host replay of every family of a layout, `grid` workgroups each.
-bool replay_batch_all(const BatchDesc* descs, const BatchLayout& layout, int grid);
+bool replay_batch_all(const BatchDesc* descs, const BatchLayout& layout, int row);
 
 }  // namespace lrt

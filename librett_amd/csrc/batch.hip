@@ -55,22 +55,32 @@ struct BatchShape {
 const BatchShape kBatchShapes[] = {LRT_BATCH_TABLE(LRT_BATCH_ROW)};
 #undef LRT_BATCH_ROW
 
-// The problem owning unit u: the p with start[p] <= u < start[p + 1]. Each
-// step the wave's lanes test 64 evenly spaced problems with one load and a
-// ballot, so 4096 problems take two dependent loads (a binary search takes 12).
-__device__ __forceinline__ int batch_find(const int* __restrict__ start, int nprob, int u) {
-  const int lane = (int)(threadIdx.x & 63);
+// The problem owning unit u of nprob problems: the p with start[p] <= u <
+// start[p + 1]. Each step the wave's lanes test 64 evenly spaced problems with
+// one load and a ballot, so 4096 problems take two dependent loads (a binary
+// search takes 12). hits(lo, n, step): how many of the lanes' problems lo,
+// lo + step, ... below lo + n start at u or before (the first ones, as starts
+// ascend, and start[lo] among them).
+template <class HITS>
+__host__ __device__ __forceinline__ int batch_find(int nprob, HITS&& hits) {
   int lo = 0, n = nprob;  // p is in [lo, lo + n)
   while (n > 1) {
     const int step = (n + 63) >> 6;
-    const int i = lane * step;
-    // start[lo] <= u: the lanes that hit are the first ones, lane 0 among them.
-    const bool hit = i < n && start[lo + i] <= u;
-    const int last = __popcll(__ballot(hit)) - 1;
+    const int last = hits(lo, n, step) - 1;
     lo += last * step;
-    n = min(step, n - last * step);
+    n = step < n - last * step ? step : n - last * step;
   }
   return lo;
+}
+__host__ __device__ __forceinline__ bool starts_by(const int* start, int u, int lo, int n, int step, int lane) {
+  const int i = lane * step;
+  return i < n && start[lo + i] <= u;
+}
+
+// The unit of workgroup (bx, by) of a grid gx wide, -1 past the last one.
+__host__ __device__ __forceinline__ int unit_at(uint32_t bx, uint32_t by, uint32_t gx, int total) {
+  const uint32_t u = by * gx + bx;
+  return u < (uint32_t)total ? (int)u : -1;
 }
 
 template <int B, int TX, int TY, int VX, int VY, bool G = false>
@@ -224,10 +234,13 @@ template <int FAM>
 __global__ __launch_bounds__(256) void k_batch(
     const BatchDesc* __restrict__ descs, const int* __restrict__ start, int nprob, int total) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[kBatchLds];
-  const uint32_t u = blockIdx.y * gridDim.x + blockIdx.x;
-  if (u >= (uint32_t)total) return;
-  const int p = batch_find(start, nprob, (int)u);
-  dev_unit<FAM>(descs[p], (int)u - start[p], lds);
+  const int u = unit_at(blockIdx.x, blockIdx.y, gridDim.x, total);
+  if (u < 0) return;
+  const int lane = (int)(threadIdx.x & 63);
+  const int p = batch_find(nprob, [&](int lo, int n, int step) {
+    return __popcll(__ballot(starts_by(start, u, lo, n, step, lane)));
+  });
+  dev_unit<FAM>(descs[p], u - start[p], lds);
 }
 
 const void* batch_kernel(int fam) {
@@ -466,7 +479,7 @@ int batch_family(int variant) {
 hipError_t launch_batch(int fam, const BatchDesc* d_descs, const int* d_start, int nprob, int total,
                         hipStream_t stream) {
   if (total <= 0 || nprob <= 0) return hipSuccess;
-  const int gx = std::min(total, 1 << 20);  // a grid dim holds fewer than 2^32 threads
+  const int gx = std::min(total, kBatchGridRow);
   void* args[4] = {&d_descs, &d_start, &nprob, &total};
   return hipLaunchKernel(batch_kernel(fam), dim3(gx, (total - 1) / gx + 1), dim3(256), args, 0, stream);
 }
@@ -522,29 +535,31 @@ hipError_t launch_batch_all(const BatchDesc* d_descs, const int* d_start, const 
   return hipSuccess;
 }
 
-bool replay_batch_all(const BatchDesc* descs, const BatchLayout& L, int grid) {
+bool replay_batch_all(const BatchDesc* descs, const BatchLayout& L, int row) {
   for (int f = 0; f < kBatchFamilies; f++) {
     if (L.n[f] == 0) continue;
-    if (!replay_batch(descs + L.first[f], L.start.data() + L.start_off[f], L.n[f], (int)L.total[f], grid))
+    if (!replay_batch(descs + L.first[f], L.start.data() + L.start_off[f], L.n[f], (int)L.total[f], row))
       return false;
   }
   return true;
 }
 
-bool replay_batch(const BatchDesc* descs, const int* start, int nprob, int total, int grid) {
+bool replay_batch(const BatchDesc* descs, const int* start, int nprob, int total, int row) {
   // The workgroup's LDS, followed by a guard band that no unit may touch.
   const size_t guard = 64 << 10;
   std::vector<unsigned char> lds(kBatchLds + guard, 0xC3);
-  for (int g = 0; g < grid; g++) {
-    int u = g;
-    if (u >= total) continue;
-    int p = 0;
-    while (p < nprob && start[p + 1] <= u) p++;
-    for (; u < total; u += grid) {
-      while (start[p + 1] <= u) p++;
+  const int gx = std::min(total, row > 0 ? row : kBatchGridRow);
+  for (int by = 0; gx > 0 && by < (total - 1) / gx + 1; by++)
+    for (int bx = 0; bx < gx; bx++) {
+      const int u = unit_at((uint32_t)bx, (uint32_t)by, (uint32_t)gx, total);
+      if (u < 0) continue;
+      const int p = batch_find(nprob, [&](int lo, int n, int step) {
+        int hits = 0;
+        for (int lane = 0; lane < 64; lane++) hits += starts_by(start, u, lo, n, step, lane);
+        return hits;
+      });
       host_unit(descs[p], u - start[p], lds.data());
     }
-  }
   for (size_t i = kBatchLds; i < lds.size(); i++)
     if (lds[i] != 0xC3) return false;
   return true;

@@ -590,7 +590,7 @@ int librett_c_batch_host_replay(int count, const int* ranks, const int* dims, co
       ds[k].in = gin[i].data() + g + B.byte_offset[k];
       ds[k].out = gout[i].data() + g + B.byte_offset[k];
     }
-    if (!replay_batch_all(ds.data(), B.layout, grid > 0 ? grid : B.grid_max)) return LIBRETT_C_UNDEFINED_ERROR;
+    if (!replay_batch_all(ds.data(), B.layout, grid)) return LIBRETT_C_UNDEFINED_ERROR;
     for (int i = 0; i < count; i++) {
       const size_t n = (size_t)B.probs[i].vol * B.probs[i].elem;
       for (size_t j = 0; j < g; j++)
@@ -642,8 +642,7 @@ int librett_c_batch_host_candidate(int rank, const int* dim, const int* permutat
       ds[k].out = gout.data() + offs[k];
       start[k + 1] = start[k] + ds[k].units;
     }
-    const int gr = grid > 0 ? grid : dev.cu_count * 4;
-    if (!replay_batch(ds.data(), start.data(), (int)ds.size(), start.back(), gr)) return LIBRETT_C_UNDEFINED_ERROR;
+    if (!replay_batch(ds.data(), start.data(), (int)ds.size(), start.back(), grid)) return LIBRETT_C_UNDEFINED_ERROR;
     if (!gout.intact()) return LIBRETT_C_UNDEFINED_ERROR;
     std::memcpy(odata, gout.data(), n);
     return LIBRETT_C_SUCCESS;

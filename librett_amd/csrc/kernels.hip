@@ -47,12 +47,17 @@ namespace lrt {
 // k_packed does for its large rounds, measured slower on MI355X: 2-3% on the
 // 8192 x 8192 planes and far slower on tiles whose registers then cut
 // occupancy.)
-// The tile of this workgroup, -1 past the last one. The grid has two dims only
-// because one dim holds at most 2^32 threads.
-__device__ __forceinline__ int tile_of(const TiledPlane& a) {
-  const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+// The tile of workgroup (bx, by) of a grid gx wide, -1 past the last one. The
+// grid has two dims only because one dim holds at most 2^32 threads.
+__host__ __device__ __forceinline__ int tile_at(const TiledPlane& a, uint32_t bx, uint32_t by, uint32_t gx) {
+  const uint32_t b = by * gx + bx;
   if (b >= (uint32_t)a.items) return -1;
   return a.xcds > 1 ? xcd_logical((int)b, a.items, a.xcds) : (int)b;
+}
+__device__ __forceinline__ int tile_of(const TiledPlane& a) { return tile_at(a, blockIdx.x, blockIdx.y, gridDim.x); }
+// The item of workgroup b of a TiledCopy launch over `items` of them.
+__host__ __device__ __forceinline__ uint32_t copy_item(int xcds, uint32_t b, uint32_t items) {
+  return xcds > 1 ? (uint32_t)xcd_logical((int)b, (int)items, xcds) : b;
 }
 
 // FEW: at most kFewDigits outer dims.
@@ -130,7 +135,7 @@ __global__ __launch_bounds__(256) void k_copy(CopyParam<FEW> a, const void* __re
                                               void* __restrict__ out) {
   using Ops = CopyOps<B, NP>;
   using E = typename Ops::E;
-  const uint32_t w = a.xcds > 1 ? (uint32_t)xcd_logical((int)blockIdx.x, (int)gridDim.x, a.xcds) : blockIdx.x;
+  const uint32_t w = copy_item(a.xcds, blockIdx.x, gridDim.x);
   Ops::run(a, w, threadIdx.x, static_cast<const E*>(in), static_cast<E*>(out));
 }
 
@@ -260,6 +265,16 @@ static inline void replay_at(long long item, int t) {
   if (g_replay_observer) g_replay_observer->at(item, t);
 }
 
+// f(tile) for the workgroups of a Tiled launch, in their order.
+template <class F>
+static void for_each_tile(const Candidate& c, F&& f) {
+  for (int by = 0; by < c.grid_y; by++)
+    for (int bx = 0; bx < c.grid_x; bx++) {
+      const int w = tile_at(c.tiled, (uint32_t)bx, (uint32_t)by, (uint32_t)c.grid_x);
+      if (w >= 0) f((uint32_t)w);
+    }
+}
+
 template <int B, int TX, int TY, int VX, int VY, bool G>
 static void replay_tiled(const Candidate& c, const void* in, void* out) {
   using Ops = TiledOps<B, TX, TY, VX, VY, G>;
@@ -268,7 +283,7 @@ static void replay_tiled(const Candidate& c, const void* in, void* out) {
   const TiledArgs& a = c.tiled;
   const E* src = static_cast<const E*>(in);
   E* dst = static_cast<E*>(out);
-  for (uint32_t w = 0; w < (uint32_t)a.items; w++) {
+  for_each_tile(c, [&](uint32_t w) {
     const TileCtx ctx = Ops::item(a, w);
     for (int t = 0; t < Ops::NT; t++) Ops::prepare(a, ctx, t, lds.data());
     for (int t = 0; t < Ops::NT; t++) {
@@ -279,7 +294,7 @@ static void replay_tiled(const Candidate& c, const void* in, void* out) {
       replay_at(w, t);
       Ops::store(a, ctx, t, dst, lds.data());
     }
-  }
+  });
 }
 
 template <class Ops>
@@ -290,7 +305,7 @@ static void replay_skew(const Candidate& c, const void* in, void* out) {
   const E* src = static_cast<const E*>(in);
   E* dst = static_cast<E*>(out);
   const int phase = line_phase(dst);
-  for (uint32_t w = 0; w < (uint32_t)a.items; w++) {
+  for_each_tile(c, [&](uint32_t w) {
     const TileCtx ctx = Ops::item(a, w);
     if (Ops::early(a))
       for (int t = 0; t < Ops::NT; t++) Ops::prepare(a, ctx, t, lds.data());
@@ -302,7 +317,7 @@ static void replay_skew(const Candidate& c, const void* in, void* out) {
       replay_at(w, t);
       Ops::store(a, ctx, t, dst, lds.data(), phase);
     }
-  }
+  });
 }
 
 template <int B, int NP>
@@ -310,11 +325,13 @@ static void replay_copy(const Candidate& c, const void* in, void* out) {
   using Ops = CopyOps<B, NP>;
   using E = typename Ops::E;
   const int items = copy_items(c, out);
-  for (int w = 0; w < items; w++)
+  for (int b = 0; b < items; b++) {
+    const uint32_t w = copy_item(c.copy.xcds, (uint32_t)b, (uint32_t)items);
     for (int t = 0; t < Ops::NT; t++) {
       replay_at(w, t);
-      Ops::run(c.copy, (uint32_t)w, t, static_cast<const E*>(in), static_cast<E*>(out));
+      Ops::run(c.copy, w, t, static_cast<const E*>(in), static_cast<E*>(out));
     }
+  }
 }
 
 template <int B, int NREG>

@@ -366,17 +366,19 @@ std::string Candidate::describe() const {
   const char* n = (method >= 0 && method < kNumMethods) ? names[method] : "?";
   static const char* kForms[] = {"", " skew", " narrow", " short"};
   const char* order = tile_order(*this) ? " xcd" : "";
+  char grid[32];
+  snprintf(grid, sizeof(grid), grid_y > 1 ? "%dx%d" : "%d", grid_x, grid_y);
   switch (method) {
     case kTiled:
       if (xgroup > 1 || ygroup > 1)
-        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s groups %d/%d grid %d%s%s", n, tile_x, tile_y, vec_x,
-                 vec_y, kForms[tiled.form], xgroup, ygroup, grid_x, order, tiled.stream_in ? " stream" : "");
+        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s groups %d/%d grid %s%s%s", n, tile_x, tile_y, vec_x,
+                 vec_y, kForms[tiled.form], xgroup, ygroup, grid, order, tiled.stream_in ? " stream" : "");
       else
-        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s grid %d%s%s", n, tile_x, tile_y, vec_x, vec_y,
-                 kForms[tiled.form], grid_x, order, tiled.stream_in ? " stream" : "");
+        snprintf(buf, sizeof(buf), "%s tile %dx%d vec %d/%d%s grid %s%s%s", n, tile_x, tile_y, vec_x, vec_y,
+                 kForms[tiled.form], grid, order, tiled.stream_in ? " stream" : "");
       break;
     case kTiledCopy:
-      snprintf(buf, sizeof(buf), "%s word %dB rows %d grid %d%s%s", n, word, copy.X, grid_x, order,
+      snprintf(buf, sizeof(buf), "%s word %dB rows %d grid %s%s%s", n, word, copy.X, grid, order,
                copy.stream_in ? " stream" : "");
       break;
     case kPacked:

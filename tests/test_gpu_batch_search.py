@@ -26,3 +26,25 @@ def test_unit_finds_its_problem(gpu_stream, count):
     finally:
         b.destroy()
         slab.free()
+
+
+def test_units_of_several_grid_rows(gpu_stream):
+    # One 17 GB problem of 1 048 832 units, 256 more than a row of workgroups
+    # holds: filled and checked on the device.
+    dim, perm, elem = [64, 4097, 4096], [0, 2, 1], 16
+    n = int(np.prod(dim, dtype=np.int64)) * elem
+    print("case:", dim, perm, elem, flush=True)
+    a, c = hip.DeviceBuffer(n), hip.DeviceBuffer(n)
+    b = L.Batch([(dim, perm, elem)], gpu_stream, tune=0)
+    try:
+        assert b.info()["total_units"] > 1 << 20
+        L.check_fill(a.ptr, n, gpu_stream)
+        hip.memset(c.ptr, 0, n)
+        b.set_buffers([a.ptr], [c.ptr])
+        assert b.execute(use_graph=False) == L.LIBRETT_SUCCESS
+        hip.stream_sync(gpu_stream)
+        assert L.check_transpose(c.ptr, dim, perm, elem, gpu_stream) == (0, -1)
+    finally:
+        b.destroy()
+        a.free()
+        c.free()

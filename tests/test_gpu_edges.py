@@ -118,3 +118,27 @@ def test_streamed_loads(gpu_stream, dim, perm, elem):
 @pytest.mark.parametrize("dim,elem", [([33, 367, 349], 4), ([2053, 32, 33], 8), ([5, 461, 459], 16), ([16, 968, 969], 4)])
 def test_copy_rows_two_words(gpu_stream, dim, elem):
     assert check(gpu_stream, dim, [0, 2, 1], elem, [0, 1, 128 // elem - 1], methods=(L.TILED_COPY,)) == 6
+
+
+# More tiles than a row of workgroups holds, in both tile orders, every plan.
+@pytest.mark.parametrize("elem", [4, 8, 16])
+def test_tiles_of_several_grid_rows(gpu_stream, elem):
+    dim, perm = [2, 1100000, 2], [2, 1, 0]
+    many = [c["desc"] for c in L.candidates(dim, perm, elem) if c["grid_y"] > 1 and c["method"] == L.TILED]
+    assert many and any(d.endswith(" xcd") for d in many) and any(not d.endswith(" xcd") for d in many)
+    assert check(gpu_stream, dim, perm, elem, [0], only=" grid 1048576x2") == len(many)
+
+
+# On both sides of the short kernel arguments' four outer dims: plans of either
+# kernel, which test_outer_dims_around_the_short_arguments runs, are there.
+@pytest.mark.parametrize("dim,perm,outer,kind", [
+    ([33, 2, 3, 2, 3, 35], [5, 4, 3, 2, 1, 0], 4, "Tiled"), ([33, 2, 3, 2, 3, 2, 35], [6, 5, 4, 3, 2, 1, 0], 5, "Tiled"),
+    ([9, 2, 3, 2, 3], [0, 4, 3, 2, 1], 4, "TiledCopy"), ([9, 2, 3, 2, 3, 2], [0, 5, 4, 3, 2, 1], 5, "TiledCopy"),
+])
+@pytest.mark.parametrize("elem", [4, 8, 16])
+def test_both_sides_of_the_short_arguments_run(gpu_stream, dim, perm, outer, kind, elem):
+    # Planes of one dim each leave all but two of the dims outside; rows all but one.
+    assert len(dim) - (2 if kind == "Tiled" else 1) == outer
+    ran = check(gpu_stream, dim, perm, elem, [0, 1], methods=(L.TILED if kind == "Tiled" else L.TILED_COPY,))
+    plain = [c for c in L.candidates(dim, perm, elem) if c["desc"].startswith(kind + " ") and "groups" not in c["desc"]]
+    assert len(plain) >= 2 and ran >= 2 * len(plain)
