@@ -472,7 +472,7 @@ void add_tiled_plane(const Problem& r, const DeviceInfo& dev, int a_dims, int b_
     if (!in_y) out_lines = out_lines && cout[d] % le == 0;
     if (!in_x) in_lines = in_lines && cin[d] % le == 0;
   }
-  TiledArgs base;
+  TiledArgs base{};
   base.X = (int)X;
   base.Y = (int)Y;
   base.in_ys = (int)cin[ydims[0]];
@@ -1412,7 +1412,8 @@ bool order_twins(const Candidate& a, const Candidate& b) {
   if (a.method == kTiled || a.method == kTiledCopy)
     return b.method == a.method && tile_order(a) != tile_order(b) && a.tile_x == b.tile_x &&
            a.tile_y == b.tile_y && a.vec_x == b.vec_x && a.vec_y == b.vec_y && a.word == b.word &&
-           a.copy_tx == b.copy_tx && a.block == b.block && a.tiled.form == b.tiled.form && a.xgroup == b.xgroup && a.ygroup == b.ygroup;
+           a.copy_tx == b.copy_tx && a.block == b.block && a.xgroup == b.xgroup && a.ygroup == b.ygroup &&
+           (a.method != kTiled || a.tiled.form == b.tiled.form);
   return (a.method == kPacked || a.method == kPackedSplit) && same_packed(a, b) && a.grid_x == b.grid_x &&
          a.grid_y == b.grid_y && a.packed.outer_per_block == b.packed.outer_per_block &&
          a.source == b.source && a.packed.order != b.packed.order;
@@ -1578,7 +1579,7 @@ std::vector<Candidate> make_candidates(const Problem& full, const DeviceInfo& de
 }
 
 bool copy_beats(const std::vector<Candidate>& cands, const Candidate& c) {
-  return c.method != kTiledCopy && cands[0].method == kTiledCopy &&
+  return (c.method == kPacked || c.method == kPackedSplit) && cands[0].method == kTiledCopy &&
          (long long)cands[0].copy.X * cands[0].elem >= kCopyOnlyRow;
 }
 
