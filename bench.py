@@ -18,7 +18,7 @@ stream) and a CPU baseline (the OpenMP host permutation on a bounded sample).
 
 Unless --quick is given, the same line then carries the other workloads,
 each with its outputs checked on the device: "batched" (4096 uneven
-problems in one persistent graph launch vs a per-call librettExecute loop),
+problems in one graph launch vs a per-call librettExecute loop),
 "serving" (Poisson arrivals through the continuous-batching engine: warm and
 cold plan caches, p50/p99 over a load sweep, per-call baselines),
 "large_random" (48 seeded ~256 MiB cases, librettPlan vs librettPlanMeasure)
@@ -505,7 +505,7 @@ def batched_problems(n, seed=20261202):
 
 
 def bench_batched(args, stream):
-    """Batched workload: the whole batch in one persistent graph launch vs a
+    """Batched workload: the whole batch in one graph launch vs a
     loop of per-problem librettExecute calls on the same buffers. Inputs hold
     the index pattern, and every output of the timed batch is checked on the
     device afterwards."""
@@ -597,7 +597,7 @@ def bench_batched(args, stream):
     for h in handles:
         L.librettDestroy(h)
     line = {
-        "metric": "batched transpose GB/s (2*bytes/t), one persistent graph launch per batch",
+        "metric": "batched transpose GB/s (2*bytes/t), one graph launch per batch",
         "value": round(value, 1),
         "unit": "GB/s",
         "n_gpus": 1,

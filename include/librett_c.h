@@ -177,18 +177,19 @@ void librett_c_set_model_constants(const double* values, int count);
 
 /* ---------------------------------------------------------------------
  * Batched engine (extension; the reference has no batched mode). Many
- * independent transposes run in one persistent kernel launch, replayed from
- * a HIP graph. Problems are given flattened: problem i has ranks[i] dims at
- * dims[o_i ...] and its permutation at perms[o_i ...], o_i = sum_{j<i}
- * ranks[j]. tune = 0 picks each problem's plan with the cost model; tune = k
- * > 0 times the model's k best batch plans of each distinct problem inside
- * the persistent kernel and keeps the fastest (remembered across batches).
+ * independent transposes run in one HIP graph launch of at most four kernels,
+ * one per family of plans, with one workgroup per unit of work. Problems are
+ * given flattened: problem i has ranks[i] dims at dims[o_i ...] and its
+ * permutation at perms[o_i ...], o_i = sum_{j<i} ranks[j]. tune = 0 picks each
+ * problem's plan with the cost model; tune = k > 0 times the model's k best
+ * batch plans of each distinct problem inside their families' kernels and
+ * keeps the fastest (remembered across batches).
  * ------------------------------------------------------------------- */
 typedef struct librett_c_batch_info {
   int count;            /* problems */
-  int descriptors;      /* device descriptors (a flat copy may use two) */
-  int total_units;      /* work units of one launch */
-  int grid;             /* persistent workgroups */
+  int descriptors;      /* device descriptors, one per problem */
+  int total_units;      /* work units of one launch, a workgroup each */
+  int grid;             /* workgroups that the device holds at a time (sizes the units) */
   int tuned;            /* problems timed by the autotuner in this batch */
   int method_count[6];  /* problems per method (index = method number) */
   long long bytes;      /* algorithmic bytes, sum of 2 * vol * elem */

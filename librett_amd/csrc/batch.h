@@ -90,14 +90,11 @@ hipError_t launch_batch_all(const BatchDesc* d_descs, const int* d_start, const 
 // Resident workgroups per CU of family `fam`'s kernel (runtime query).
 int batch_occupancy(int fam);
 
-// Descriptors of one problem planned with candidate c: one descriptor, or
-// up to two for a plain copy (Trivial). `fallback` gets the variants for
-// buffers not aligned to the vector width; `offsets` the byte offset of each
-// descriptor's data inside the problem's buffers.
-bool describe_problem(const Problem& p, const Candidate& c, std::vector<BatchDesc>& descs,
-                      std::vector<BatchDesc>& fallback, std::vector<long long>& offsets);
+// Descriptor of one problem planned with candidate c, and the one for buffers
+// not aligned to its vector width (of the same family).
+bool describe_problem(const Problem& p, const Candidate& c, BatchDesc& desc, BatchDesc& fallback);
 
-// Pointer alignment the descriptors of candidate c need.
+// Pointer alignment the descriptor of candidate c needs.
 int batch_alignment(const Problem& p, const Candidate& c);
 
 // Batch-mode candidates of a problem, best modelled streaming cost first.

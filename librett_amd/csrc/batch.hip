@@ -458,7 +458,7 @@ void batch_regroup(BatchDesc& d, long long unit_bytes) {
 
 long long batch_unit_bytes(long long total_bytes, int grid) {
   // LIBRETT_BATCH_UNIT_KB fixes the unit size; LIBRETT_BATCH_UNITS_PER_WG
-  // sets the units each workgroup should get (default 8).
+  // sets the units for each workgroup that the device holds at a time (default 32).
   static const long long fixed = [] {
     const char* e = std::getenv("LIBRETT_BATCH_UNIT_KB");
     return e ? std::max(1LL, std::atoll(e)) << 10 : 0LL;

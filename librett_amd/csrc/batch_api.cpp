@@ -79,10 +79,9 @@ struct BatchObj {
   int nprob = 0;
   std::vector<Problem> probs;
   std::vector<Candidate> chosen;
-  // Descriptors: one or two per problem (a flat copy may need a tail).
+  // Descriptors, one per problem, in family order.
   std::vector<BatchDesc> descs, fallback;
   std::vector<int> owner;               // problem of each descriptor
-  std::vector<long long> byte_offset;   // offset of the descriptor's data in its problem
   BatchLayout layout;                   // descriptors grouped by kernel family
   long long total = 0;                  // units of all families
   int grid_max = 0;  // workgroups resident at a time, of the family that holds most
@@ -246,36 +245,20 @@ int build_batch(BatchObj& B, const DeviceInfo& dev, int tune) {
   // Descriptors and the unit index space.
   B.descs.clear();
   B.fallback.clear();
-  B.owner.clear();
-  B.byte_offset.clear();
   for (int i = 0; i < B.nprob; i++) {
-    std::vector<BatchDesc> ds, fs;
-    std::vector<long long> offs;
-    if (!describe_problem(B.probs[i], B.chosen[i], ds, fs, offs)) return fail("no descriptor for the chosen plan");
-    for (size_t k = 0; k < ds.size(); k++) {
-      batch_regroup(ds[k], B.unit_bytes);
-      batch_regroup(fs[k], B.unit_bytes);
-      B.descs.push_back(ds[k]);
-      B.fallback.push_back(fs[k]);
-      B.owner.push_back(i);
-      B.byte_offset.push_back(offs[k]);
-    }
+    BatchDesc d, f;
+    if (!describe_problem(B.probs[i], B.chosen[i], d, f)) return fail("no descriptor for the chosen plan");
+    batch_regroup(d, B.unit_bytes);
+    batch_regroup(f, B.unit_bytes);
+    B.descs.push_back(d);
+    B.fallback.push_back(f);
   }
-  // Group by kernel family; the fallback descriptors, owners and offsets
-  // follow the same order (a fallback keeps its descriptor's family).
-  std::vector<int> order;
-  batch_layout(B.descs, B.layout, &order);
-  std::vector<BatchDesc> fb(order.size());
-  std::vector<int> own(order.size());
-  std::vector<long long> off(order.size());
-  for (size_t k = 0; k < order.size(); k++) {
-    fb[k] = B.fallback[order[k]];
-    own[k] = B.owner[order[k]];
-    off[k] = B.byte_offset[order[k]];
-  }
+  // Group by kernel family; the fallback descriptors follow the same order (a
+  // fallback keeps its descriptor's family).
+  batch_layout(B.descs, B.layout, &B.owner);
+  std::vector<BatchDesc> fb(B.owner.size());
+  for (size_t k = 0; k < B.owner.size(); k++) fb[k] = B.fallback[B.owner[k]];
   B.fallback.swap(fb);
-  B.owner.swap(own);
-  B.byte_offset.swap(off);
   B.total = 0;
   for (int f = 0; f < kBatchFamilies; f++) {
     if (B.layout.total[f] >= (1LL << 31)) return LIBRETT_C_INVALID_PARAMETER;
@@ -378,24 +361,12 @@ std::vector<Candidate> batch_candidates(const Problem& p, const DeviceInfo& dev)
 }
 
 int batch_alignment(const Problem& p, const Candidate& c) {
-  if (c.method == kTrivial) return p.elem;
-  if (c.method == kTiled && c.tiled.form == kTileRect) return c.elem * std::max(c.vec_x, c.vec_y);
-  return c.elem;
+  return c.method == kTrivial ? p.elem : needed_alignment(c);
 }
 
-bool describe_problem(const Problem& p, const Candidate& c, std::vector<BatchDesc>& descs,
-                      std::vector<BatchDesc>& fallback, std::vector<long long>& offsets) {
-  descs.clear();
-  fallback.clear();
-  offsets.clear();
-  BatchDesc d, f;
-  if (!batch_describe(c.method == kTrivial ? flat_copy(p) : c, d)) return false;
-  Candidate fc = c.method == kTrivial ? flat_copy(p) : c;
-  if (c.method == kTiled && c.tiled.form == kTileRect) fc.vec_x = fc.vec_y = 1;
-  if (!batch_describe(fc, f)) f = d;
-  descs.push_back(d);
-  fallback.push_back(f);
-  offsets.push_back(0);
+bool describe_problem(const Problem& p, const Candidate& c, BatchDesc& desc, BatchDesc& fallback) {
+  if (!batch_describe(c.method == kTrivial ? flat_copy(p) : c, desc)) return false;
+  if (batch_alignment(p, c) == p.elem || !batch_describe(unaligned_fallback(c), fallback)) fallback = desc;
   return true;
 }
 
@@ -450,13 +421,11 @@ int librett_c_batch_set_buffers(unsigned int handle, const void* const* idata, v
   for (size_t k = 0; k < B->descs.size(); k++) {
     const int i = B->owner[k];
     if (!idata[i] || !odata[i] || idata[i] == odata[i]) return LIBRETT_C_INVALID_PARAMETER;
-    const char* in = (const char*)idata[i] + B->byte_offset[k];
-    char* out = (char*)odata[i] + B->byte_offset[k];
     const int align = batch_alignment(B->probs[i], B->chosen[i]);
-    const bool mis = (((uintptr_t)in | (uintptr_t)out) & (uintptr_t)(align - 1)) != 0;
+    const bool mis = (((uintptr_t)idata[i] | (uintptr_t)odata[i]) & (uintptr_t)(align - 1)) != 0;
     up[k] = mis ? B->fallback[k] : B->descs[k];
-    up[k].in = in;
-    up[k].out = out;
+    up[k].in = idata[i];
+    up[k].out = odata[i];
   }
   // A fallback descriptor may have another unit count: rebuild the index
   // space and re-capture the graph when it changes. The descriptors are
@@ -587,8 +556,8 @@ int librett_c_batch_host_replay(int count, const int* ranks, const int* dims, co
     std::vector<BatchDesc> ds = B.descs;
     for (size_t k = 0; k < ds.size(); k++) {
       const int i = B.owner[k];
-      ds[k].in = gin[i].data() + g + B.byte_offset[k];
-      ds[k].out = gout[i].data() + g + B.byte_offset[k];
+      ds[k].in = gin[i].data() + g;
+      ds[k].out = gout[i].data() + g;
     }
     if (!replay_batch_all(ds.data(), B.layout, grid)) return LIBRETT_C_UNDEFINED_ERROR;
     for (int i = 0; i < count; i++) {
@@ -626,23 +595,19 @@ int librett_c_batch_host_candidate(int rank, const int* dim, const int* permutat
     if (count) *count = (int)ranked.size();
     if (!idata && !odata) return LIBRETT_C_SUCCESS;
     if (!idata || !odata || index < 0 || index >= (int)ranked.size()) return LIBRETT_C_INVALID_PARAMETER;
-    std::vector<BatchDesc> ds, fs;
-    std::vector<long long> offs;
-    if (!describe_problem(p, ranked[index], ds, fs, offs)) return LIBRETT_C_INTERNAL_ERROR;
-    if (fallback) ds = fs;
+    BatchDesc d0, f0;
+    if (!describe_problem(p, ranked[index], d0, f0)) return LIBRETT_C_INTERNAL_ERROR;
+    BatchDesc& run = fallback ? f0 : d0;
     const long long ub = unit_bytes > 0 ? unit_bytes : kBatchUnitBytes;
     const size_t n = (size_t)p.vol * p.elem;
     const int align = fallback ? p.elem : batch_alignment(p, ranked[index]);
     GuardedBuffer gin(n, idata, align, 0xA5), gout(n, odata, align, 0x5A);
     std::memcpy(gin.data(), idata, n);
-    std::vector<int> start(ds.size() + 1, 0);
-    for (size_t k = 0; k < ds.size(); k++) {
-      batch_regroup(ds[k], ub);
-      ds[k].in = gin.data() + offs[k];
-      ds[k].out = gout.data() + offs[k];
-      start[k + 1] = start[k] + ds[k].units;
-    }
-    if (!replay_batch(ds.data(), start.data(), (int)ds.size(), start.back(), grid)) return LIBRETT_C_UNDEFINED_ERROR;
+    batch_regroup(run, ub);
+    run.in = gin.data();
+    run.out = gout.data();
+    const int start[2] = {0, run.units};
+    if (!replay_batch(&run, start, 1, run.units, grid)) return LIBRETT_C_UNDEFINED_ERROR;
     if (!gout.intact()) return LIBRETT_C_UNDEFINED_ERROR;
     std::memcpy(odata, gout.data(), n);
     return LIBRETT_C_SUCCESS;

@@ -1593,15 +1593,6 @@ int choose_by_model(const std::vector<Candidate>& cands) {
   return best;
 }
 
-Candidate scalar_fallback(const Candidate& c) {
-  Candidate f = c;
-  if (c.method == kTiled && c.tiled.form == kTileRect) {
-    f.vec_x = 1;
-    f.vec_y = 1;
-  }
-  return f;
-}
-
 int needed_alignment(const Candidate& c) {
   switch (c.method) {
     case kTiled:
@@ -1612,6 +1603,10 @@ int needed_alignment(const Candidate& c) {
   }
 }
 
-Candidate unaligned_fallback(const Candidate& c) { return c.method == kTiled ? scalar_fallback(c) : c; }
+Candidate unaligned_fallback(const Candidate& c) {
+  Candidate f = c;
+  if (c.method == kTiled && c.tiled.form == kTileRect) f.vec_x = f.vec_y = 1;
+  return f;
+}
 
 }  // namespace lrt

@@ -147,10 +147,6 @@ int choose_by_model(const std::vector<Candidate>& cands);
 // group (group 1 = x fastest).
 void set_tile_group(TiledArgs& a, int nty, int group);
 
-// Variant of a Tiled candidate without vector accesses, used when the
-// caller's pointers are not aligned to the vector width.
-Candidate scalar_fallback(const Candidate& c);
-
 // Pointer alignment a candidate's vector accesses need.
 int needed_alignment(const Candidate& c);
 

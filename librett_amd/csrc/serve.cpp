@@ -324,30 +324,24 @@ class Server {
 
     std::vector<std::shared_ptr<Request>> take, failed, back;
     int ndesc = 0;
-    std::vector<BatchDesc> ds, fs;
-    std::vector<long long> offs;
     std::vector<BatchDesc> use;
     for (size_t i = 0; i < cand.size(); i++) {
       const std::shared_ptr<Request>& r = cand[i];
-      if (!describe_problem(r->prob, r->plan, ds, fs, offs)) {
+      BatchDesc d, f;
+      if (!describe_problem(r->prob, r->plan, d, f)) {
         failed.push_back(r);
         continue;
       }
-      if (ndesc + (int)ds.size() > s.cap) {
+      if (ndesc == s.cap) {
         back.assign(cand.begin() + (long)i, cand.end());
         break;
       }
       const int align = batch_alignment(r->prob, r->plan);
-      for (size_t k = 0; k < ds.size(); k++) {
-        const char* in = (const char*)r->in + offs[k];
-        char* out = (char*)r->out + offs[k];
-        const bool mis = (((uintptr_t)in | (uintptr_t)out) & (uintptr_t)(align - 1)) != 0;
-        BatchDesc d = mis ? fs[k] : ds[k];
-        d.in = in;
-        d.out = out;
-        use.push_back(d);
-        ndesc++;
-      }
+      const bool mis = (((uintptr_t)r->in | (uintptr_t)r->out) & (uintptr_t)(align - 1)) != 0;
+      use.push_back(mis ? f : d);
+      use.back().in = r->in;
+      use.back().out = r->out;
+      ndesc++;
       take.push_back(r);
     }
     bool ok = true;
