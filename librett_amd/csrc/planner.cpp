@@ -81,18 +81,23 @@ constexpr int kSkewColumn = 512;
 // against 76; c128 8 74 against 76, 12 75 against 72.
 constexpr int kNarrowX = 12;
 
-// Non-temporal loads for an input of `bytes` bytes that a kernel reads in
-// whole lines, once, or nearly so: copies between rotating buffers on MI355X gain from
-// 96 MiB on (33.8 -> 32.2 us at 96 MiB, 85.5 -> 83.1 us at 256 MiB), where
-// input and output no longer fit the 256 MiB Infinity Cache together; below,
-// the input may still be there from whoever wrote it, and streaming it costs
-// (19.9 -> 22.0 us at 64 MiB). LIBRETT_STREAM_MB overrides the size.
-int stream_input(long long bytes) {
-  static const long long from = [] {
+// Non-temporal loads for an input of `bytes` bytes that a kernel reads in whole
+// lines, once, or nearly so, from `times` 104 MiB on. Below, the Infinity Cache
+// still holds much of the input, from whoever wrote it or from the last pass,
+// and streaming it costs. Not streamed and streamed on MI355X, among passes
+// over three buffer pairs (and right after a kernel that filled the input):
+// transposed f32 matrices of 80 MiB 25.6 and 33.0 us (28 and 37), 96 MiB 36.8
+// and 40.7 (33 and 45), 100 MiB 38.2 and 40.5 (35.0 and 35.2), 104 MiB 40.7 and
+// 41.7 (36.0 and 35.0), 112 MiB 46.7 and 45.8 (38.5 and 38.5), 192 MiB 78.2 and
+// 76.4 (71 and 62); f64 ones alike. Rows of 4 KB gain more: 100 MiB 35.2 and
+// 35.0, 104 MiB 37.7 and 36.5, 128 MiB 48.3 and 44.1, 256 MiB 95.8 and 88.3.
+// LIBRETT_STREAM_MB overrides the size.
+int stream_input(long long bytes, double times = 1) {
+  static const double from = [] {
     const char* e = std::getenv("LIBRETT_STREAM_MB");
-    return e && *e ? std::atoll(e) : 96;
+    return e && *e ? std::atof(e) : 104.0;
   }();
-  return bytes >= from << 20 ? 1 : 0;
+  return (double)bytes >= times * from * (1 << 20) ? 1 : 0;
 }
 
 // Words per thread of a TiledCopy plan whose rows of `row` bytes make `bytes`
@@ -102,9 +107,11 @@ int stream_input(long long bytes) {
 // 25.4 and 22.9; of 18 KB 72 MiB 24.1 and 22.0; but rows of 16 B 24 MiB 11.0
 // and 11.5, of 32 B 16 MiB 6.5 and 6.8; rows of 1 KB 96 MiB 33.3 and 34.7,
 // 256 MiB 85.2 and 88.8. (Row tiles with four words per thread, the kernel
-// before, took 16.4, 23.8 and 24.7 us for the 48 and 72 MiB cases.)
+// before, took 16.4, 23.8 and 24.7 us for the 48 and 72 MiB cases.) The upper
+// end is where rows of whole lines begin to be streamed: of 4 KB, 100 MiB 35.8
+// and 35.2 us, 108 MiB 39.9 and 40.1, streamed 37.7 and 38.1.
 int copy_words(long long bytes, long long row) {
-  return bytes >= (16LL << 20) && bytes < (96LL << 20) && row >= 64 ? 2 : 1;
+  return bytes >= (16LL << 20) && bytes < (104LL << 20) && row >= 64 ? 2 : 1;
 }
 
 // Outer map over the input dims for which `skip[d]` is false, in input order.
@@ -708,8 +715,13 @@ void add_tiled_copy(const Problem& r, const DeviceInfo& dev, std::vector<Candida
   // a kernel that filled the input, and among passes over three buffer pairs:
   // 112 MiB 49.5 and 38.2 us, 40.2 and 40.6; 256 MiB 106 and 82, 88.2 and 89.7;
   // 384 MiB 146 and 150, 132 and 134; 500 MiB 193 and 213, 173 and 175. Shorter
-  // rows never gain (1 KB, 500 MiB: 230 and 226, 188 and 185).
-  a.stream_in = !dev.batch_mode && (row % 128 == 0 ? stream_input(bytes) : row >= 2048 && stream_input(bytes / 4));
+  // rows never gain (1 KB, 500 MiB: 230 and 226, 188 and 185). Rows of whole
+  // half lines cut but every second line, and gain earlier: 256 MiB 94 and 80,
+  // 86.5 and 89.2; 320 MiB 104 and 110, 107 and 111; 368 MiB 122 and 133, 123
+  // and 128 (52 KB 103 and 109, 106 and 109 at 320 MiB; 8 KB 113 and 118, 109
+  // and 113).
+  a.stream_in = !dev.batch_mode && (row % 128 == 0 ? stream_input(bytes)
+                                                   : row >= 2048 && stream_input(bytes, row % 64 == 0 ? 3.1 : 3.7));
   c.block = 256;
   c.lds_bytes = 0;
   c.grid_x = a.items;

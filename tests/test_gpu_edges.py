@@ -102,11 +102,11 @@ def test_outer_dims_around_the_short_arguments(gpu_stream, dim, perm, elem):
     check(gpu_stream, dim, perm, elem, [0, 1], methods=(4, 5))
 
 
-# Inputs of 96 MiB and more that are read in whole lines: non-temporal loads,
+# Inputs of 104 MiB and more that are read in whole lines: non-temporal loads,
 # over planes of one dim and of dim groups (whole tiles and cut ones), and rows.
 @pytest.mark.parametrize("dim,perm,elem", [
-    ([64, 6, 344, 200], [2, 1, 0, 3], 4), ([32, 12, 344, 100], [2, 1, 0, 3], 8), ([16, 100, 16, 260], [3, 2, 1, 0], 16),
-    ([1024, 160, 161], [0, 2, 1], 4),
+    ([64, 6, 344, 212], [2, 1, 0, 3], 4), ([32, 12, 344, 106], [2, 1, 0, 3], 8), ([16, 100, 16, 275], [3, 2, 1, 0], 16),
+    ([1024, 160, 172], [0, 2, 1], 4),
 ])
 def test_streamed_loads(gpu_stream, dim, perm, elem):
     want = [c["desc"] for c in L.candidates(dim, perm, elem) if c["desc"].endswith(" stream")]
@@ -114,7 +114,7 @@ def test_streamed_loads(gpu_stream, dim, perm, elem):
     assert check(gpu_stream, dim, perm, elem, [0], only=" stream") == len(want)
 
 
-# 16 to 96 MiB: two words per thread.
+# 16 to 104 MiB: two words per thread.
 @pytest.mark.parametrize("dim,elem", [([33, 367, 349], 4), ([2053, 32, 33], 8), ([5, 461, 459], 16), ([16, 968, 969], 4)])
 def test_copy_rows_two_words(gpu_stream, dim, elem):
     assert check(gpu_stream, dim, [0, 2, 1], elem, [0, 1, 128 // elem - 1], methods=(L.TILED_COPY,)) == 6

@@ -65,3 +65,16 @@ def test_rows_cut_by_lines_stream_only_far_beyond_the_cache(dim, elem, streamed)
     import librett_amd as L
     copies = [c["desc"] for c in L.host_candidates(dim, [0, 2, 1], elem) if c["method"] == L.TILED_COPY]
     assert copies and all(d.endswith(" stream") == streamed for d in copies)
+
+
+@pytest.mark.parametrize("dim,perm,elem,streamed", [
+    ([4096, 6592], [1, 0], 4, False), ([4096, 6656], [1, 0], 4, True), ([4096, 3296], [1, 0], 8, False),
+    ([4096, 3328], [1, 0], 8, True), ([1024, 103, 256], [0, 2, 1], 4, False), ([1024, 104, 256], [0, 2, 1], 4, True),
+    ([2312, 115, 157], [0, 2, 1], 8, False), ([2312, 115, 159], [0, 2, 1], 8, True),
+])
+def test_inputs_that_the_cache_half_holds_do_not_stream(dim, perm, elem, streamed):
+    # Whole lines at 103 and 104 MiB; rows of whole half lines at 318 and 322.5.
+    import librett_amd as L
+    method = L.TILED_COPY if perm[0] == 0 else L.TILED
+    plans = [c["desc"] for c in L.host_candidates(dim, perm, elem) if c["method"] == method]
+    assert any(d.endswith(" stream") for d in plans) == streamed
