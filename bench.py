@@ -820,6 +820,8 @@ def serving_catalog(kw, n):
     return out
 
 
+# Kernels that run a plan; a bench step dispatches one per named case.
+TRANSPOSE_KERNELS = ("k_tiled<", "k_skew<", "k_narrow<", "k_copy<", "k_packed<")
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_named_large_cases.json")
 
 
@@ -854,7 +856,9 @@ def pmc_summary(fetch_dir, write_dir, run_log, json_path=None):
     if not cal_r:
         raise SystemExit("no copy-kernel dispatches to calibrate against")
     fr_k, fw_k = float(np.median(cal_r)), float(np.median(cal_w))
-    transposes = [i for i, n in enumerate(names) if any(k in n for k in ("k_tiled", "k_copy<", "k_packed"))]
+    transposes = [i for i, n in enumerate(names) if any(k in n for k in TRANSPOSE_KERNELS)]
+    if len(transposes) < len(CASES):
+        raise SystemExit("%d transposes dispatched, %d cases" % (len(transposes), len(CASES)))
     plans = [ln.split(" -> ", 1)[1].rsplit(" (", 1)[0].strip() for ln in open(run_log) if ln.startswith("plan ")]
     out = {"fetch_factor": round(fr_k, 4), "write_factor": round(fw_k, 4), "cases": []}
     lines = ["# HBM traffic of the named large cases (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)", "",
@@ -921,7 +925,7 @@ def pmc_requests(read_dir, write_dir):
         alg = None
         if "k_devcopy" in name:
             alg = grid * 16.0
-        elif any(t in name for t in ("k_tiled", "k_copy<", "k_packed")):
+        elif any(t in name for t in TRANSPOSE_KERNELS):
             if ntr < len(case_bytes):
                 alg = case_bytes[ntr]
                 short = "%s %s" % (short, "x".join(str(x) for x in CASES[ntr][0]))
