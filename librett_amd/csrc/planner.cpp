@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
 #include <functional>
 #include <mutex>
 #include <thread>
@@ -1110,11 +1111,24 @@ void model_tiled(Candidate& c) {
         if (xa < xb) rin.push_back({(oi + xa + (long long)tiled_in_y(a, (uint32_t)y)) * B, (long long)(xb - xa) * B});
       }
     } else if (a.form != kTileRect) {
+      // Row y covers the columns whose skew is at least y0 - y and less than
+      // y0 - y + tile_y: with a bit per column, those of two masks. (A walk over
+      // the columns of every split row took two thirds of a skewed plan's model.)
       const SkewTile k = skew_tile(a, oo, x0, tx, 128 / B);
+      uint64_t least[33] = {};  // columns whose skew is at least v
+      for (int i = 0; i < tx; i++) least[k.s[i]] |= 1ull << i;
+      for (int v = 128 / B; v-- > 0;) least[v] |= least[v + 1];
+      auto from = [&](int v) { return v <= 0 ? least[0] : v >= 128 / B ? 0 : least[v]; };
       for (int y = std::max(0, y0 - k.hi); y < std::min(a.Y, y0 + c.tile_y); y++) {
         const long long row = oi + x0 + (long long)tiled_in_y(a, (uint32_t)y);
-        skew_row_runs(k, y, y0, c.tile_y,
-                      [&](int i, int n) { rin.push_back({(row + i) * B, (long long)n * B}); });
+        uint64_t m = from(y0 - y) & ~from(y0 - y + c.tile_y);
+        while (m) {
+          const int i = __builtin_ctzll(m);
+          const uint64_t past = ~m & (~0ull << i);  // columns after i that are not covered
+          const int n = (past ? __builtin_ctzll(past) : 64) - i;
+          rin.push_back({(row + i) * B, (long long)n * B});
+          m = i + n < 64 ? m & (~0ull << (i + n)) : 0;
+        }
       }
       for (int i = 0; i < tx; i++) {
         const int ya = std::max(0, y0 - k.s[i]), yb = std::min(a.Y, y0 - k.s[i] + c.tile_y);
@@ -1250,7 +1264,6 @@ struct PackedSums {
 // last line touched (relative to the line holding the base) and the merged
 // intervals that touch those two lines.
 struct RoundPattern {
-  bool done = false;
   double lines = 0, partial = 0, tran = 0;
   long long first = 0, last = -1;
   std::vector<Run> head, tail;
@@ -1308,12 +1321,16 @@ PackedSums packed_sums(const Candidate& c) {
     staged_runs(a.shape[v], true, rout[v]);
   }
   // Round patterns of variant v, side (0 in, 1 out) at byte alignment `al`
-  // = (base * B) mod 128.
-  std::vector<RoundPattern> memo(2 * 2 * 128);
+  // = (base * B) mod 128, made when first met (few of the 512 are).
+  short at[2 * 2 * 128];
+  std::fill(std::begin(at), std::end(at), (short)-1);
+  std::deque<RoundPattern> memo;
   std::vector<Run> tmp, merged;
   auto pattern = [&](int v, int side, long long al) -> const RoundPattern& {
-    RoundPattern& r = memo[(v * 2 + side) * 128 + al];
-    if (!r.done) {
+    short& k = at[(v * 2 + side) * 128 + al];
+    if (k < 0) {
+      k = (short)memo.size();
+      RoundPattern& r = memo.emplace_back();
       const auto& runs = side ? rout[v] : rin[v];
       tmp.clear();
       for (const auto& x : runs) tmp.push_back({al + x.first * B, (long long)x.second * B});
@@ -1328,9 +1345,8 @@ PackedSums packed_sums(const Candidate& c) {
           if (((m.s + m.n - 1) >> 7) >= r.last) r.tail.push_back(m);
         }
       }
-      r.done = true;
     }
-    return r;
+    return memo[k];
   };
   const long long nblocks = (long long)c.grid_x * c.grid_y;
   const int window = std::max(1, std::min(4, a.outer_per_block));
@@ -1532,6 +1548,12 @@ void model_times(Candidate& c, const DeviceInfo& dev) {
   m.predicted_s = std::max(m.t_hbm, m.t_latency) + m.t_launch;
 }
 
+// Whether the candidates begin with a copy of rows that no Packed plan beats.
+static bool long_row_copy(const std::vector<Candidate>& cands) {
+  return !cands.empty() && cands[0].method == kTiledCopy &&
+         (long long)cands[0].copy.X * cands[0].elem >= kCopyOnlyRow;
+}
+
 std::vector<Candidate> make_candidates(const Problem& full, const DeviceInfo& dev) {
   std::vector<Candidate> out;
   if (full.rank < 1 || full.rank > kMaxRank) return out;
@@ -1552,8 +1574,12 @@ std::vector<Candidate> make_candidates(const Problem& full, const DeviceInfo& de
   else
     add_tiled(red, dev, out);
   if (!dev.batch_mode) add_order_twins(dev, out);
-  add_packed(full, "full", dev, out);
-  if (red.rank != full.rank) add_packed(red, "reduced", dev, out);
+  // The batched engine never takes a Packed plan where a copy of long rows is
+  // one (batch_candidates), so there they are not planned at all.
+  if (!dev.batch_mode || !long_row_copy(out)) {
+    add_packed(full, "full", dev, out);
+    if (red.rank != full.rank) add_packed(red, "reduced", dev, out);
+  }
   for (auto& c : out)
     if (c.active_blocks_per_cu <= 0) c.active_blocks_per_cu = active_blocks(c, dev);
   // Model every candidate; the XCD-interleaved twin of a Packed plan follows
@@ -1591,8 +1617,7 @@ std::vector<Candidate> make_candidates(const Problem& full, const DeviceInfo& de
 }
 
 bool copy_beats(const std::vector<Candidate>& cands, const Candidate& c) {
-  return (c.method == kPacked || c.method == kPackedSplit) && cands[0].method == kTiledCopy &&
-         (long long)cands[0].copy.X * cands[0].elem >= kCopyOnlyRow;
+  return (c.method == kPacked || c.method == kPackedSplit) && long_row_copy(cands);
 }
 
 int choose_by_model(const std::vector<Candidate>& cands) {
