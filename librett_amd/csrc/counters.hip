@@ -344,8 +344,9 @@ __host__ __device__ inline void sort_small(long long* v, int n) {
 // Lines one item reads and writes: Tiled reads tile rows (y ascending) and
 // writes tile columns (x ascending); TiledCopy reads pieces of rows and
 // writes one run; Packed walks the staged shape's runs, which the host sorted
-// by start. `st` has room for kCopyPieces values.
-__host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, unsigned long long* acc, long long* st) {
+// by start. `st` has room for kCopyPieces values; `masks` is scratch.
+__host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, unsigned long long* acc, long long* st,
+                                           SkewMasks& masks) {
   LineWalk rd, wr;
   const long long B = j.B;
   if (j.method == kTiled && j.a.tiled.form == kTileShort) {
@@ -364,17 +365,18 @@ __host__ __device__ inline void item_lines(const CountJob& j, const ItemCtx& c, 
     // TY + a line's elements of them).
     const TiledArgs& a = j.a.tiled;
     int n = 0;
+    skew_masks(c.skew, 128 / j.B, masks);
     const int ya = c.y0 - c.skew.hi > 0 ? c.y0 - c.skew.hi : 0;
     const int yb = imin(a.Y, c.y0 + j.TY);
     if (a.yg.n > 1) {
       for (int y = ya; y < yb; y++) st[n++] = ((c.in0 + c.x0 + (long long)tiled_in_y(a, (uint32_t)y)) << 8) | (y - ya);
       sort_small(st, n);
       for (int k = 0; k < n; k++)
-        skew_row_runs(c.skew, ya + (int)(st[k] & 255), c.y0, j.TY,
+        skew_row_runs(masks, ya + (int)(st[k] & 255), c.y0, j.TY,
                       [&](int i, int len) { rd.add(((st[k] >> 8) + i) * B, len * B); });
     } else {
       for (int y = ya; y < yb; y++)
-        skew_row_runs(c.skew, y, c.y0, j.TY, [&](int i, int len) {
+        skew_row_runs(masks, y, c.y0, j.TY, [&](int i, int len) {
           rd.add((c.in0 + c.x0 + (long long)tiled_in_y(a, (uint32_t)y) + i) * B, len * B);
         });
     }
@@ -470,6 +472,7 @@ __device__ inline void wave_count(bool act, long long off, int bytes, int lane, 
 __global__ __launch_bounds__(kCountThreads) void k_count(CountJob job, unsigned long long* __restrict__ part) {
   __shared__ unsigned long long red[kCountThreads];
   __shared__ long long starts[kCopyPieces];
+  __shared__ SkewMasks masks;
   unsigned long long acc[kNumCounts];
   for (int i = 0; i < kNumCounts; i++) acc[i] = 0;
   const int lane = threadIdx.x & 63;
@@ -489,7 +492,7 @@ __global__ __launch_bounds__(kCountThreads) void k_count(CountJob job, unsigned 
           wave_count(act, off, bytes, lane, acc[kLdReq + store], acc[kLdTran + store], acc[kLdBytes + store]);
         }
     }
-    if (threadIdx.x == 0) item_lines(job, c, acc, starts);
+    if (threadIdx.x == 0) item_lines(job, c, acc, starts, masks);
   }
   for (int i = 0; i < kNumCounts; i++) {
     red[threadIdx.x] = acc[i];
@@ -587,6 +590,7 @@ void host_walk(const CountJob& j, unsigned long long* acc, F&& f) {
   long long off[64];
   int bytes[64];
   long long starts[kCopyPieces];
+  SkewMasks masks;
   for (long long w = 0; w < j.items; w++) {
     const ItemCtx c = item_ctx(j, (uint32_t)w);
     for (int store = 0; store < 2; store++) {
@@ -603,7 +607,7 @@ void host_walk(const CountJob& j, unsigned long long* acc, F&& f) {
           host_wave_count(act, off, bytes, acc[kLdReq + store], acc[kLdTran + store], acc[kLdBytes + store]);
         }
     }
-    item_lines(j, c, acc, starts);
+    item_lines(j, c, acc, starts, masks);
   }
 }
 

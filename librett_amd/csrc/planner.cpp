@@ -1111,24 +1111,13 @@ void model_tiled(Candidate& c) {
         if (xa < xb) rin.push_back({(oi + xa + (long long)tiled_in_y(a, (uint32_t)y)) * B, (long long)(xb - xa) * B});
       }
     } else if (a.form != kTileRect) {
-      // Row y covers the columns whose skew is at least y0 - y and less than
-      // y0 - y + tile_y: with a bit per column, those of two masks. (A walk over
-      // the columns of every split row took two thirds of a skewed plan's model.)
       const SkewTile k = skew_tile(a, oo, x0, tx, 128 / B);
-      uint64_t least[33] = {};  // columns whose skew is at least v
-      for (int i = 0; i < tx; i++) least[k.s[i]] |= 1ull << i;
-      for (int v = 128 / B; v-- > 0;) least[v] |= least[v + 1];
-      auto from = [&](int v) { return v <= 0 ? least[0] : v >= 128 / B ? 0 : least[v]; };
+      SkewMasks masks;
+      skew_masks(k, 128 / B, masks);
       for (int y = std::max(0, y0 - k.hi); y < std::min(a.Y, y0 + c.tile_y); y++) {
         const long long row = oi + x0 + (long long)tiled_in_y(a, (uint32_t)y);
-        uint64_t m = from(y0 - y) & ~from(y0 - y + c.tile_y);
-        while (m) {
-          const int i = __builtin_ctzll(m);
-          const uint64_t past = ~m & (~0ull << i);  // columns after i that are not covered
-          const int n = (past ? __builtin_ctzll(past) : 64) - i;
-          rin.push_back({(row + i) * B, (long long)n * B});
-          m = i + n < 64 ? m & (~0ull << (i + n)) : 0;
-        }
+        skew_row_runs(masks, y, y0, c.tile_y,
+                      [&](int i, int n) { rin.push_back({(row + i) * B, (long long)n * B}); });
       }
       for (int i = 0; i < tx; i++) {
         const int ya = std::max(0, y0 - k.s[i]), yb = std::min(a.Y, y0 - k.s[i] + c.tile_y);
