@@ -155,7 +155,8 @@ __host__ __device__ inline TileCtx tile_item(const A& a, uint32_t w, int tx_size
 // 106 SGPRs and up to 20 more VGPRs alive (34 SGPRs without it), and the
 // dispatcher's order keeps neighbouring tiles closer in time than a stride
 // over the grid does ([2, 8, 16, 32, 64, 128] f32 95 -> 88 us as 64 x 128 tiles,
-// with the loads non-temporal too; a copy of the bytes takes 85 us).
+// with the loads non-temporal too; a copy of the bytes takes 85 us, and the 64 x
+// 64 tiles that librettPlan takes there 94 us, as before).
 // Reference counterpart: transposeTiled, src/kernel.cpp:48-170.
 // ---------------------------------------------------------------------------
 // G = false compiles only the one-dim-group path (the kernel then needs no
@@ -298,10 +299,16 @@ struct TiledOps {
 // LE (a line's elements) more rows than TY, of which each column uses its TY;
 // each lane loads just the rows of its column, so no element is loaded twice.
 // Bound by HBM. What it removes: lines written in two halves by two
-// workgroups (1.06 x the bytes in DRAM writes, but each partial line costs a
-// read-modify-write there). On MI355X, against unskewed tiles with their best
-// lanes: (8191, 8193) f32 130 -> 94 us, (4097, 8191) f64 122 -> 94 us,
-// (5, 97, 211, 331) f64 131 -> 105 us; a copy of the bytes takes 85 us.
+// workgroups, which cost far more than their share of the bytes. What it costs:
+// the input lines of the rows that a tile splits with its neighbours are read
+// by both, in dispatch order into two L2s. (5, 97, 211, 331) f64 by the request
+// counters: writes 1.063 -> 1.016, reads 1.002 -> 1.75 times the bytes, 129 ->
+// 116 us. On MI355X, against unskewed tiles with their best lanes: (8191, 8193)
+// f32 130 -> 94 us, (4097, 8191) f64 122 -> 94 us, (5, 97, 211, 331) f64 131 ->
+// 107 us with 32 x 128 tiles (116 with the 32 x 64 that librettPlan takes); a
+// copy of the bytes takes 85 us. That is among passes over three buffer pairs;
+// where the input has just been written, (8191, 8193) goes from 97 to 91 us but
+// (5, 97, 211, 331) from 115 to 117, and to 94-98 in the order across XCDs.
 // One-element loads are as fast as 16-byte ones here (93-95 against 93 us,
 // f32), and non-temporal loads slower (106 us), as neighbouring tiles share
 // the lines of the rows they split. Tiles aligned to 64 bytes instead of 128
